@@ -51,7 +51,7 @@ int dev_alloc(cav_ctx* ctx, void** p, size_t bytes, const char* what) {
 static void bvh_free(cav_bvh* h) {
     void* ptrs[] = {h->b.keys[0], h->b.keys[1], h->b.vals[0], h->b.vals[1], h->b.hist, h->b.counts,
                     h->b.scene_ord, h->b.nbox, h->b.topo, h->b.visited, h->b.ref,
-                    h->b.partial, h->b.leaf_ids, h->b.counters, h->rec, h->root, h->mesh,
+                    h->b.partial, h->b.counters, h->rec, h->root, h->mesh,
                     h->b.lvl_list, h->b.lvl_cnt, h->b.lvl_cursor, h->b.lvl_off,
                     h->b.bounds_part, h->b.gate64};
     for (void* p : ptrs)
@@ -81,7 +81,6 @@ static int bvh_alloc(cav_ctx* ctx, cav_bvh* h, int n) {
         {(void**)&h->b.gate64, sizeof(uint64_t) * bottom_up_gate_words(n), "split gates"},
         {(void**)&h->b.ref, sizeof(int32_t) * m, "ref"},
         {(void**)&h->b.partial, sizeof(uint32_t) * (lbvh_partials(m) + 1), "partial"},
-        {(void**)&h->b.leaf_ids, sizeof(uint32_t) * n, "leaf_ids"},
         {(void**)&h->b.counters, 256, "counters"},
         {(void**)&h->rec, sizeof(TRec) * 2 * (size_t)n, "traversal records"},
         {(void**)&h->root, 64, "root"},
@@ -143,7 +142,7 @@ static int bvh_run(cav_ctx* ctx, cav_bvh* h, const float* tris_dev, const float*
     HIPCHK(ctx, hipMemcpyAsync(root_lbvh, h->b.nbox, sizeof(NodeBox), hipMemcpyDeviceToHost, s));
     HIPCHK(ctx, hipMemcpyAsync(&sort_err, h->b.hist + kSortHistWords + 8, 4, hipMemcpyDeviceToHost, s));
     mark(mk, "readback");
-    for (int r = 0; r < opt_rounds; ++r) HIPCHK(ctx, treelet_round_impl(h->b, n, r == 0, s, mk));
+    for (int r = 0; r < opt_rounds; ++r) HIPCHK(ctx, treelet_round_impl(h->b, n, s, mk));
     if (opt_rounds > 0) HIPCHK(ctx, lbvh_refs(h->b, n, s, mk, "flatten_refs"));
     HIPCHK(ctx, lbvh_flatten(h->b, tris_dev, h->mesh, n, opt_rounds == 0, h->rec, h->root, s, mk));
     float root_final[8];

@@ -45,11 +45,10 @@ struct LbvhBuffers {
     uint32_t* bounds_part = nullptr;          // per-workgroup partial bounds (6 each)
     NodeBox* nbox = nullptr;                  // 2n-1
     int4* topo = nullptr;                     // 2n-1
-    uint32_t* visited = nullptr;              // 2n-1 (arrivals << 16 | height)
+    uint32_t* visited = nullptr;              // 2n-1 (2 << 16 | height, inner nodes)
     unsigned long long* gate64 = nullptr;     // bottom_up_gate_words(n): split gates and edge arrivals (gates zero between builds)
     int32_t* ref = nullptr;                   // 2n-1 (restructured trees)
     uint32_t* partial = nullptr;              // scan partials
-    uint32_t* leaf_ids = nullptr;             // n (treelet round start list)
     uint32_t* counters = nullptr;             // small device counters
     uint32_t* lvl_list = nullptr;             // 2n-1 internal node ids grouped by height
     uint32_t* lvl_cnt = nullptr;              // kMaxLevels + 2 (count per height, error flag)
@@ -79,14 +78,13 @@ int64_t bottom_up_gate_words(int n);
 hipError_t lbvh_bottom_up(LbvhBuffers& b, const void* codes, int keybits, const float* tris, int n,
                           hipStream_t s, Marker* mk);
 
-// levels.hip: height climb + bucketing by height (treelet rounds)
-hipError_t levels_from_list(LbvhBuffers& b, int n, hipStream_t s, Marker* mk);
+// levels.hip: bucketing by height (treelet rounds)
 hipError_t levels_bucket(LbvhBuffers& b, int n, hipStream_t s, Marker* mk);
 // deepest leaf (edges from the root) of the current tree into *out (device word)
 hipError_t levels_max_depth(const LbvhBuffers& b, int n, uint32_t* out, hipStream_t s);
 
-// treelet.hip: one restructuring round; `first` = leaves still at ids N-1..2N-2
-hipError_t treelet_round_impl(LbvhBuffers& b, int n, bool first, hipStream_t s, Marker* mk);
+// treelet.hip: one restructuring round
+hipError_t treelet_round_impl(LbvhBuffers& b, int n, hipStream_t s, Marker* mk);
 
 // traverse.hip
 // Traversal over a flattened BVH of ntris triangles. counters[0] (closest) and

@@ -3,14 +3,12 @@
 // The reference orders its treelet rounds by letting each leaf thread climb
 // and the second visitor of a node continue (BVH/Optimization.cu:467-507).
 // A treelet reads and rewrites up to 13 nodes, far more than the box that
-// the build's climb passes between arrivals, so here the climb only computes
-// heights, and every height level is then processed by its own launch;
-// kernel boundaries order the levels and no data fences are needed:
+// the build's climb passes between arrivals, so here every height level is
+// processed by its own launch; kernel boundaries order the levels and no
+// data fences are needed:
 //
-//   1. climb: every leaf walks up; each visitor of a node adds
-//      (1 << 16 | its height + 1) to the node's word with one atomic, so the
-//      second visitor finds the first one's height in the returned value
-//      (the build's climb leaves the same words for the first round);
+//   1. heights: the build's climb leaves each inner node's height in its word,
+//      and a treelet updates the words of the nodes it rewrites;
 //   2. bucket the internal nodes by height (block-aggregated counting sort);
 //   3. level h = 3..H in order: a launch over the nodes of height h, the few
 //      nodes of the top levels in a single workgroup with barriers.
@@ -25,31 +23,6 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kLdsBins = 256;
-
-// Climb from one leaf. Each visitor adds (1 << 16 | its height + 1) to the
-// parent's word; the second visitor reads the first one's height from the
-// returned value, stores the parent's final (2 << 16 | height) and goes on.
-__device__ __forceinline__ void climb_heights(const int4* __restrict__ topo, uint32_t* hw, int leaf,
-                                              int max_steps) {
-    int cur = leaf;
-    uint32_t h = 0;
-    for (int step = 0; cur != 0 && step < max_steps; ++step) {
-        const int p = topo[cur].z;
-        const uint32_t old = atomicAdd(&hw[p], (1u << 16) | (h + 1));
-        if ((old >> 16) != 1u) return;  // first visitor stops here
-        h = max(old & 0xffffu, h + 1);
-        hw[p] = (2u << 16) | h;
-        cur = p;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_heights(const int4* __restrict__ topo,
-                                                    const uint32_t* __restrict__ leaf_ids,
-                                                    int nleaves, uint32_t* hw) {
-    const int k = blockIdx.x * kBlock + threadIdx.x;
-    if (k >= nleaves) return;
-    climb_heights(topo, hw, (int)leaf_ids[k], nleaves);
-}
 
 __global__ void k_fill(uint32_t* p, int64_t n, uint32_t v) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -134,15 +107,6 @@ hipError_t levels_max_depth(const LbvhBuffers& b, int n, uint32_t* out, hipStrea
     hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, s, out, (int64_t)1, 0u);
     hipLaunchKernelGGL(k_max_depth, dim3((unsigned)((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, b.topo, m, n,
                        out);
-    return hipGetLastError();
-}
-
-hipError_t levels_from_list(LbvhBuffers& b, int n, hipStream_t s, Marker* mk) {
-    const int64_t m = 2 * (int64_t)n - 1;
-    hipLaunchKernelGGL(k_fill, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, b.visited, m, 0u);
-    const int nb = (n + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(k_heights, dim3(nb), dim3(kBlock), 0, s, b.topo, b.leaf_ids, n, b.visited);
-    mark(mk, "treelet_heights");
     return hipGetLastError();
 }
 
