@@ -24,6 +24,8 @@ SOURCES = [
     "bottomup.hip",
     "treelet.hip",
     "traverse.hip",
+    "wide.hip",
+    "wide_trace.hip",
     "render.hip",
     "rlpath.hip",
     "queue_sort.hip",

@@ -176,10 +176,10 @@ class BVH:
                 "max_stack_closest": int(out[2]), "max_stack_occluded": int(out[3])}
 
     def trace_fetches(self, reset: bool = False) -> dict:
-        """64-byte records (node visits + triangle tests) fetched by the
-        closest-hit and any-hit launches since the last reset, and the rays
-        of the last any-hit / closest-hit launch finished by the cooperative
-        passes (and of those, traced again on one lane)."""
+        """Records (node visits + triangle tests) fetched by the closest-hit
+        and any-hit launches since the last reset, and the rays of the last
+        any-hit / closest-hit launch finished by whole waves (and of those,
+        traced over the reference's tree on one lane)."""
         out = np.zeros(6, np.uint64)
         check(self.ctx.handle, lib().cav_trace_fetches(self.ctx.handle, self.handle, _ptr(out), 1 if reset else 0))
         return {"closest": int(out[0]), "occluded": int(out[1]), "spilled_rays": int(out[2]),

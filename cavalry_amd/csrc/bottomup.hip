@@ -394,25 +394,30 @@ __global__ __launch_bounds__(kBlock) void k_climb_crossing(int n, int nedges, No
 // per workgroup edge.
 int64_t bottom_up_gate_words(int n) { return (int64_t)n + 2 * ((int64_t)(n + kBlock - 1) / kBlock) + 2; }
 
-hipError_t lbvh_bottom_up(LbvhBuffers& b, const void* codes, int keybits, const float* tris, int n,
+hipError_t bottom_up_tree(const void* codes, int keybits, const float* tris, int n, const BottomUpOut& o,
                           hipStream_t s, Marker* mk) {
     const int nb = (n + kBlock - 1) / kBlock;
     if (keybits > 32)
         hipLaunchKernelGGL(k_bottom_up<uint64_t>, dim3(nb), dim3(kBlock), 0, s,
-                           static_cast<const uint64_t*>(codes), n, keybits, b.order, tris, b.nbox, b.topo,
-                           b.visited, b.gate64);
+                           static_cast<const uint64_t*>(codes), n, keybits, o.order, tris, o.nbox, o.topo,
+                           o.hw, o.gate64);
     else
         hipLaunchKernelGGL(k_bottom_up<uint32_t>, dim3(nb), dim3(kBlock), 0, s,
-                           static_cast<const uint32_t*>(codes), n, keybits, b.order, tris, b.nbox, b.topo,
-                           b.visited, b.gate64);
+                           static_cast<const uint32_t*>(codes), n, keybits, o.order, tris, o.nbox, o.topo,
+                           o.hw, o.gate64);
     mark(mk, "refit_bottom_up");
     const int nedges = nb - 1;
     if (nedges > 0) {
         hipLaunchKernelGGL(k_climb_crossing, dim3((unsigned)((nedges + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
-                           n, nedges, b.nbox, b.topo, b.visited, b.gate64);
+                           n, nedges, o.nbox, o.topo, o.hw, o.gate64);
         mark(mk, "refit_crossing");
     }
     return hipGetLastError();
+}
+
+hipError_t lbvh_bottom_up(LbvhBuffers& b, const void* codes, int keybits, const float* tris, int n,
+                          hipStream_t s, Marker* mk) {
+    return bottom_up_tree(codes, keybits, tris, n, BottomUpOut{b.order, b.nbox, b.topo, b.visited, b.gate64}, s, mk);
 }
 
 }  // namespace cav

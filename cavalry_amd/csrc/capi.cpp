@@ -57,6 +57,7 @@ static void bvh_free(cav_bvh* h) {
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (h->spill) (void)hipFree(h->spill);
+    if (h->wide.base) (void)hipFree(h->wide.base);
     if (h->b.h_lvl) (void)hipHostFree(h->b.h_lvl);
     delete[] h->b.h_off;
     if (h->events)
@@ -97,6 +98,15 @@ static int bvh_alloc(cav_ctx* ctx, cav_bvh* h, int n) {
     // the traversal counters only ever add to (or max into) their words
     HIPCHK(ctx, hipMemsetAsync(h->b.gate64, 0, sizeof(uint64_t) * bottom_up_gate_words(n), ctx->stream));
     HIPCHK(ctx, hipMemsetAsync(h->b.counters, 0, 256, ctx->stream));
+    // the wide tree is left out where memory is short: the traces then walk
+    // the reference's tree
+    void* wide = nullptr;
+    if (hipMalloc(&wide, wide_bytes(n)) == hipSuccess) {
+        wide_carve(h->wide, wide, n);
+        HIPCHK(ctx, hipMemsetAsync(h->wide.gate, 0, sizeof(uint64_t) * bottom_up_gate_words(n), ctx->stream));
+    } else {
+        (void)hipGetLastError();
+    }
     HIPCHK(ctx, hipHostMalloc((void**)&h->b.h_lvl, sizeof(uint32_t) * (kMaxLevels + 2), hipHostMallocDefault));
     h->b.h_off = new uint32_t[kMaxLevels + 2]();
     for (auto& e : h->mk.ev) HIPCHK(ctx, hipEventCreate(&e));
@@ -111,6 +121,13 @@ static void host_to_ord(const float* f6, uint32_t* o6) {
         std::memcpy(&u, &f6[i], 4);
         o6[i] = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
     }
+}
+
+static float ord_to_float(uint32_t o) {
+    const uint32_t u = (o & 0x80000000u) ? (o & 0x7fffffffu) : ~o;
+    float f;
+    std::memcpy(&f, &u, 4);
+    return f;
 }
 
 static float elapsed(hipEvent_t a, hipEvent_t b) {
@@ -144,10 +161,27 @@ static int bvh_run(cav_ctx* ctx, cav_bvh* h, const float* tris_dev, const float*
     mark(mk, "readback");
     for (int r = 0; r < opt_rounds; ++r) HIPCHK(ctx, treelet_round_impl(h->b, n, s, mk));
     if (opt_rounds > 0) HIPCHK(ctx, lbvh_refs(h->b, n, s, mk, "flatten_refs"));
-    HIPCHK(ctx, lbvh_flatten(h->b, tris_dev, h->mesh, n, opt_rounds == 0, h->rec, h->root, s, mk));
+    HIPCHK(ctx, lbvh_flatten(h->b, tris_dev, h->mesh, n, opt_rounds == 0, h->rec, h->root, h->wide.leaf_of, s, mk));
+    const uint32_t* bounds = h->b.scene_ord;
+    if (h->wide.base) {
+        if (scene_bounds) {
+            bounds = h->wide.bounds;
+            HIPCHK(ctx, lbvh_scene_bounds(tris_dev, n, h->wide.bounds, h->b.bounds_part, s, nullptr));
+        }
+        HIPCHK(ctx, wide_build(h->wide, h->b, tris_dev, h->mesh, n, bounds, s, mk));
+    }
     float root_final[8];
+    uint32_t box[6], height = 0, wide_err = 0;
+    HIPCHK(ctx, hipMemcpyAsync(box, bounds, sizeof box, hipMemcpyDeviceToHost, s));
+    HIPCHK(ctx, hipMemcpyAsync(&height, h->b.visited, 4, hipMemcpyDeviceToHost, s));
+    HIPCHK(ctx, hipMemcpyAsync(&wide_err, h->b.hist + kSortHistWords + 8, 4, hipMemcpyDeviceToHost, s));
     HIPCHK(ctx, hipMemcpyAsync(root_final, h->b.nbox, sizeof(NodeBox), hipMemcpyDeviceToHost, s));
     HIPCHK(ctx, hipStreamSynchronize(s));
+    // The wide tree stands in for the reference's when every coordinate is
+    // within 2^40 (its planes' distances then stay finite) and no traversal of
+    // the reference's tree can outgrow its 64-entry stack.
+    h->wide_ok = h->wide.base != nullptr && (height & 0xffffu) <= 64u && wide_err == 0;
+    for (int k = 0; k < 6; ++k) h->wide_ok = h->wide_ok && std::fabs(ord_to_float(box[k])) <= 1099511627776.f;
     if (sort_err) return fail(ctx, CAV_ERR_HIP, "radix sort: a look-back wait exceeded its bound");
     cav_bvh_stats st{};
     st.n = n;
@@ -407,7 +441,7 @@ int cav_trace_closest_async(cav_ctx* ctx, const cav_bvh* h, const float* rays, i
     TraceCoop coop;
     const int rc = ensure_spill(ctx, h, nrays, &coop);
     if (rc != CAV_OK) return rc;
-    HIPCHK(ctx, trace_closest(h->rec, h->n, h->root, rays, nrays, prim, t, nullptr, nullptr,
+    HIPCHK(ctx, trace_closest(bvh_trace(h), rays, nrays, prim, t, nullptr, nullptr,
                               h->b.counters, ctx->launch[CAV_TRACE_STANDALONE], ctx->stream, &coop));
     return CAV_OK;
 }
@@ -418,7 +452,7 @@ int cav_trace_occluded_async(cav_ctx* ctx, const cav_bvh* h, const float* rays,
     TraceCoop coop;
     const int rc = ensure_spill(ctx, h, nrays, &coop);
     if (rc != CAV_OK) return rc;
-    HIPCHK(ctx, trace_occluded(h->rec, h->n, rays, limit, nullptr, nullptr, nrays, visible,
+    HIPCHK(ctx, trace_occluded(bvh_trace(h), rays, limit, nullptr, nullptr, nrays, visible,
                                h->b.counters, ctx->launch[CAV_TRACE_STANDALONE], ctx->stream, &coop));
     return CAV_OK;
 }
@@ -479,7 +513,7 @@ int cav_trace_closest_device(cav_ctx* ctx, const cav_bvh* h, const float* rays, 
     TraceCoop coop;
     const int rc = ensure_spill(ctx, h, nrays, &coop);
     if (rc != CAV_OK) return rc;
-    HIPCHK(ctx, trace_closest(h->rec, h->n, h->root, rays, nrays, prim, t, u, v, h->b.counters,
+    HIPCHK(ctx, trace_closest(bvh_trace(h), rays, nrays, prim, t, u, v, h->b.counters,
                               ctx->launch[CAV_TRACE_STANDALONE], ctx->stream, &coop));
     uint32_t ovf = 0;
     HIPCHK(ctx, hipMemcpyAsync(&ovf, h->b.counters, 4, hipMemcpyDeviceToHost, ctx->stream));
@@ -499,7 +533,7 @@ int cav_trace_occluded_device(cav_ctx* ctx, const cav_bvh* h, const float* rays,
     TraceCoop coop;
     const int rc = ensure_spill(ctx, h, nrays, &coop);
     if (rc != CAV_OK) return rc;
-    HIPCHK(ctx, trace_occluded(h->rec, h->n, rays, limit, src, dst, nrays, visible, h->b.counters,
+    HIPCHK(ctx, trace_occluded(bvh_trace(h), rays, limit, src, dst, nrays, visible, h->b.counters,
                                ctx->launch[CAV_TRACE_STANDALONE], ctx->stream, &coop));
     uint32_t ovf = 0;
     HIPCHK(ctx, hipMemcpyAsync(&ovf, h->b.counters + 1, 4, hipMemcpyDeviceToHost, ctx->stream));

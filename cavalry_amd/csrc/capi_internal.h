@@ -6,6 +6,7 @@
 
 #include "../../include/cavalry.h"
 #include "lbvh.h"
+#include "wide.h"
 
 struct cav_ctx {
     int device = 0;
@@ -28,6 +29,8 @@ struct cav_bvh {
     cav::TRec* rec = nullptr;   // 2n traversal records (sibling-pair layout)
     float* root = nullptr;      // 8 floats
     int32_t* mesh = nullptr;    // n, original order (may be null)
+    cav::WideBuffers wide;      // wide traversal tree (base null: no memory for it)
+    bool wide_ok = false;       // the last build's wide tree can stand in for the reference's
     // long-ray pass buffers (cav::trace_coop_bytes(spill_cap, spill_cap)),
     // grown to the largest batch traced
     mutable void* spill = nullptr;
@@ -44,6 +47,12 @@ namespace cav {
 int fail(cav_ctx* ctx, int code, const std::string& msg);
 int hip_fail(cav_ctx* ctx, hipError_t e, const char* what);
 int dev_alloc(cav_ctx* ctx, void** p, size_t bytes, const char* what);
+// what the traces of a BVH read
+inline TraceBvh bvh_trace(const cav_bvh* h) {
+    TraceBvh t{h->rec, h->n, h->root, WideDev{}};
+    if (h->wide_ok) t.wide = WideDev{h->wide.nodes, h->wide.tris, h->b.nbox, h->b.topo, h->wide.leaf_of};
+    return t;
+}
 // frees context-owned state of other subsystems before the stream goes away
 void ctx_release(cav_ctx* ctx);
 // noalloc.hip: finds the no-alloc staging array on `device` (current), once per device

@@ -68,13 +68,22 @@ hipError_t lbvh_build(LbvhBuffers& b, const float* tris, int n, int morton_bits,
                       Marker* mk);
 hipError_t lbvh_refs(LbvhBuffers& b, int n, hipStream_t s, Marker* mk, const char* label);
 hipError_t lbvh_flatten(LbvhBuffers& b, const float* tris, const int32_t* mesh, int n,
-                        bool identity_refs, TRec* rec, float* root, hipStream_t s,
+                        bool identity_refs, TRec* rec, float* root, int32_t* leaf_of, hipStream_t s,
                         Marker* mk);
 int64_t lbvh_partials(int64_t m);
 
 // bottomup.hip: node ids, children, parents, boxes and heights of the
 // radix tree over the sorted codes, in one climb from the leaves
 int64_t bottom_up_gate_words(int n);
+struct BottomUpOut {
+    const uint32_t* order;       // sorted position -> triangle
+    NodeBox* nbox;               // 2n-1
+    int4* topo;                  // 2n-1
+    uint32_t* hw;                // 2n-1 heights of the inner nodes
+    unsigned long long* gate64;  // bottom_up_gate_words(n), zero before and after
+};
+hipError_t bottom_up_tree(const void* codes, int keybits, const float* tris, int n, const BottomUpOut& o,
+                          hipStream_t s, Marker* mk);
 hipError_t lbvh_bottom_up(LbvhBuffers& b, const void* codes, int keybits, const float* tris, int n,
                           hipStream_t s, Marker* mk);
 
@@ -162,30 +171,48 @@ inline TraceCoop trace_coop_in(void* base, uint32_t spill_cap, uint32_t long_cap
     return c;
 }
 
-// coop: null (every ray traced by one lane) or the cooperative passes' buffers
-hipError_t trace_closest(const TRec* rec, int ntris, const float* root,
-                         const float* rays, int64_t nrays, int32_t* prim, float* t, float* u,
+// What the wide tree's traces read (wide.h). tris: 3 words per triangle in
+// tree order: v0 | original index, v1 | mesh, v2 | 0. nbox, topo and leaf_of
+// (the leaf id of each original triangle) are the reference BVH's, for the
+// rare rays whose answer depends on its visiting order.
+struct WideDev {
+    const uint4* nodes = nullptr;  // null: no wide tree
+    const float4* tris = nullptr;
+    const NodeBox* nbox = nullptr;
+    const int4* topo = nullptr;
+    const int32_t* leaf_of = nullptr;
+};
+// A flattened BVH of ntris triangles with its wide tree, if it has one.
+struct TraceBvh {
+    const TRec* rec = nullptr;
+    int ntris = 0;
+    const float* root = nullptr;
+    WideDev wide;
+};
+
+// coop: null (every ray traced by one lane in the reference's order) or the
+// cooperative passes' buffers
+hipError_t trace_closest(const TraceBvh& bvh, const float* rays, int64_t nrays, int32_t* prim, float* t, float* u,
                          float* v, uint32_t* counters, const TraceLaunch& L, hipStream_t s,
                          const TraceCoop* coop = nullptr);
-hipError_t trace_occluded(const TRec* rec, int ntris, const float* rays,
+hipError_t trace_occluded(const TraceBvh& bvh, const float* rays,
                           const float* limit, const int32_t* src, const int32_t* dst,
                           int64_t nrays, uint8_t* visible, uint32_t* counters, const TraceLaunch& L,
                           hipStream_t s, const TraceCoop* coop = nullptr);
 
-hipError_t trace_closest_queue(const TRec* rec, int ntris, const float* root,
-                               const float* rays, const uint32_t* nrays_dev, int64_t capacity,
+hipError_t trace_closest_queue(const TraceBvh& bvh, const float* rays, const uint32_t* nrays_dev, int64_t capacity,
                                int32_t* prim, float* t, float* u, float* v, uint32_t* counters,
                                const TraceLaunch& L, hipStream_t s, const TraceCoop* coop = nullptr);
-hipError_t trace_occluded_queue(const TRec* rec, int ntris, const float* rays,
+hipError_t trace_occluded_queue(const TraceBvh& bvh, const float* rays,
                                 const uint32_t* nrays_dev, int64_t capacity, const float* limit,
                                 const int32_t* src, const int32_t* dst, uint8_t* visible,
                                 uint32_t* counters, const TraceLaunch& L, hipStream_t s,
                                 const TraceCoop* coop = nullptr);
 // the same, launched through a sink (a stream or a graph under construction)
-void trace_closest_queue(const TRec* rec, int ntris, const float* root, const float* rays,
+void trace_closest_queue(const TraceBvh& bvh, const float* rays,
                          const uint32_t* nrays_dev, int64_t capacity, int32_t* prim, float* t, float* u, float* v,
                          uint32_t* counters, const TraceLaunch& L, LaunchSink& ls, const TraceCoop* coop = nullptr);
-void trace_occluded_queue(const TRec* rec, int ntris, const float* rays, const uint32_t* nrays_dev,
+void trace_occluded_queue(const TraceBvh& bvh, const float* rays, const uint32_t* nrays_dev,
                           int64_t capacity, const float* limit, const int32_t* src, const int32_t* dst,
                           uint8_t* visible, uint32_t* counters, const TraceLaunch& L, LaunchSink& ls,
                           const TraceCoop* coop = nullptr);

@@ -313,7 +313,8 @@ __global__ __launch_bounds__(kBlock) void k_flatten(const NodeBox* __restrict__ 
                                                     const float* __restrict__ tris,
                                                     const int32_t* __restrict__ mesh,
                                                     TRec* __restrict__ rec,
-                                                    float* __restrict__ root) {
+                                                    float* __restrict__ root,
+                                                    int32_t* __restrict__ leaf_of) {
     const int64_t id = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int64_t m = 2 * (int64_t)n - 1;
     if (id >= m) return;
@@ -338,6 +339,7 @@ __global__ __launch_bounds__(kBlock) void k_flatten(const NodeBox* __restrict__ 
         o.q3 = make_float4(__int_as_float(ll ? ~base : base), __int_as_float(rl ? ~(base + 1) : base + 1), 0.f, 0.f);
     } else {
         const int p = tp.w;
+        if (leaf_of) leaf_of[p] = (int32_t)id;
         const v3 v0 = load_v(tris, p, 0), v1 = load_v(tris, p, 1), v2 = load_v(tris, p, 2);
         const v3 e1 = sub3(v1, v0), e2 = sub3(v2, v0);
         o.q0 = make_float4(v0.x, v0.y, v0.z, __int_as_float(p));
@@ -408,12 +410,12 @@ hipError_t lbvh_refs(LbvhBuffers& b, int n, hipStream_t s, Marker* mk, const cha
 }
 
 hipError_t lbvh_flatten(LbvhBuffers& b, const float* tris, const int32_t* mesh, int n,
-                        bool identity_refs, TRec* rec, float* root, hipStream_t s,
+                        bool identity_refs, TRec* rec, float* root, int32_t* leaf_of, hipStream_t s,
                         Marker* mk) {
     const int64_t m = 2 * (int64_t)n - 1;
     const int nb = (int)((m + kBlock - 1) / kBlock);
     hipLaunchKernelGGL(k_flatten, dim3(nb), dim3(kBlock), 0, s, b.nbox, b.topo, n,
-                       identity_refs ? nullptr : b.ref, tris, mesh, rec, root);
+                       identity_refs ? nullptr : b.ref, tris, mesh, rec, root, leaf_of);
     mark(mk, "flatten");
     return hipGetLastError();
 }

@@ -92,7 +92,7 @@ extern "C" int cav_trace_closest_noalloc(cav_ctx* ctx, const cav_bvh* h, const f
     const size_t r = (size_t)nrays;
     NACHK(ctx, hipMemcpyAsync(drays, rays, 24 * r, hipMemcpyHostToDevice, s));
     NACHK(ctx, hipMemsetAsync(counters, 0, kCounterBytes, s));
-    NACHK(ctx, cav::trace_closest(h->rec, h->n, h->root, drays, nrays, dprim, dt, u ? du : nullptr,
+    NACHK(ctx, cav::trace_closest(cav::bvh_trace(h), drays, nrays, dprim, dt, u ? du : nullptr,
                                   v ? dv : nullptr, counters, ctx->launch[CAV_TRACE_STANDALONE], s));
     uint32_t ovf = 0;
     NACHK(ctx, hipMemcpyAsync(&ovf, counters, 4, hipMemcpyDeviceToHost, s));

@@ -51,6 +51,8 @@ struct SceneDev {
     // maximum over the queue, which is 3 as soon as any task picked an area
     // light; this fixes it per scene.
     int light_dims;
+    WideDev wide;  // the wide traversal tree, if the BVH has one
+    TraceBvh trace() const { return TraceBvh{rec, ntris, root, wide}; }
     // hit barycentrics are needed for vertex normals and texture coordinates
     __host__ __device__ bool needs_bary() const { return normals != nullptr || texels != nullptr; }
 };

@@ -266,7 +266,7 @@ hipError_t render_direct(const RenderArgs& a, hipStream_t s) {
     render_raygen(a, s);
     float* hu = a.scene.needs_bary() ? a.hit_u : nullptr;
     float* hv = a.scene.needs_bary() ? a.hit_v : nullptr;
-    if ((e = trace_closest_queue(a.scene.rec, a.scene.ntris, a.scene.root, a.q[0].ray, a.counts, nq,
+    if ((e = trace_closest_queue(a.scene.trace(), a.q[0].ray, a.counts, nq,
                                  a.hit_prim, a.hit_t, hu, hv, a.trace_counters, a.launch, s, &a.coop)) != hipSuccess)
         return e;
     if (a.sort_perm && (e = sort_hits_by_material(a.scene, a.hit_prim, a.counts, nq, a.sort_hist, a.sort_perm, s)) !=
@@ -274,7 +274,7 @@ hipError_t render_direct(const RenderArgs& a, hipStream_t s) {
         return e;
     hipLaunchKernelGGL(k_direct, dim3(nb), dim3(kBlock), 0, s, a.scene, a.halton, a.q[0], a.sh, a.hit_prim, a.hit_t,
                        hu, hv, a.res, a.counts, a.sort_perm);
-    if ((e = trace_occluded_queue(a.scene.rec, a.scene.ntris, a.sh.ray, a.counts + 2, nq, a.sh.limit,
+    if ((e = trace_occluded_queue(a.scene.trace(), a.sh.ray, a.counts + 2, nq, a.sh.limit,
                                   a.sh.src, a.sh.dst, a.vis, a.trace_counters, a.launch, s, &a.coop)) != hipSuccess)
         return e;
     hipLaunchKernelGGL(k_nee, dim3(nb), dim3(kBlock), 0, s, a.sh, a.vis, a.res, a.counts);
@@ -293,7 +293,7 @@ hipError_t render_path(const RenderArgs& a, hipStream_t s) {
     int qin = 0, dim0 = 2;
     for (int depth = 0; depth < a.max_depth; ++depth) {
         const int qout = qin ^ 1;
-        if ((e = trace_closest_queue(a.scene.rec, a.scene.ntris, a.scene.root, a.q[qin].ray,
+        if ((e = trace_closest_queue(a.scene.trace(), a.q[qin].ray,
                                      a.counts + qin, nsamp, a.hit_prim, a.hit_t, hu, hv,
                                      a.trace_counters, a.launch, s, &a.coop)) != hipSuccess)
             return e;
@@ -317,7 +317,7 @@ hipError_t render_path(const RenderArgs& a, hipStream_t s) {
                           a.q[qout], a.sh, a.hit_prim, a.hit_t, hu, hv, a.res, a.counts, qin, qout, a.sort_perm);
             if (ls.err != hipSuccess) return ls.err;
         }
-        if ((e = trace_occluded_queue(a.scene.rec, a.scene.ntris, a.sh.ray, a.counts + 2,
+        if ((e = trace_occluded_queue(a.scene.trace(), a.sh.ray, a.counts + 2,
                                       nsamp, a.sh.limit, a.sh.src, a.sh.dst, a.vis, a.trace_counters, a.launch,
                                       s, &a.coop)) != hipSuccess)
             return e;

@@ -298,7 +298,8 @@ SceneDev scene_dev(const cav_scene* sc) {
     return SceneDev{sc->bvh->rec,  sc->bvh->root, sc->ntris,   sc->soup,
                     sc->tri_mesh,   sc->meshes,   sc->area,      sc->lights,  sc->nmeshes,
                     sc->nlights,    sc->normals,  sc->mesh_normals, sc->uv,   sc->texels,
-                    sc->tex,        sc->env,      sc->env_miss,     sc->light_dims};
+                    sc->tex,        sc->env,      sc->env_miss,     sc->light_dims,
+                    bvh_trace(sc->bvh).wide};
 }
 
 int halton_dev(cav_ctx* ctx, HaltonDev* out) {

@@ -1027,7 +1027,7 @@ hipError_t render_rlpath(const RenderArgs& a, const RlArgs& rl, bool init_tables
     for (int depth = 0; depth < a.max_depth; ++depth) {
         const int qout = qin ^ 1;
         const RenderSrc src{st, depth};
-        if ((e = trace_closest_queue(a.scene.rec, a.scene.ntris, a.scene.root, a.q[qin].ray,
+        if ((e = trace_closest_queue(a.scene.trace(), a.q[qin].ray,
                                      a.counts + qin, nsamp, a.hit_prim, a.hit_t, hu, hv,
                                      a.trace_counters, a.launch, s, &a.coop)) != hipSuccess)
             return e;
@@ -1050,7 +1050,7 @@ hipError_t render_rlpath(const RenderArgs& a, const RlArgs& rl, bool init_tables
         }
         ls.launch("k_lighting", &k_lighting<RenderSrc>, dim3(nb), dim3(kBlock), src, a.scene, a.halton, a.q[qin],
                   rl.slots, a.sh, a.hit_prim, a.hit_t, hu, hv, a.counts, qin, perm);
-        if ((e = trace_occluded_queue(a.scene.rec, a.scene.ntris, a.sh.ray, a.counts + 2, nsamp,
+        if ((e = trace_occluded_queue(a.scene.trace(), a.sh.ray, a.counts + 2, nsamp,
                                       a.sh.limit, a.sh.src, a.sh.dst, a.vis, a.trace_counters, a.launch, s, &a.coop)) != hipSuccess)
             return e;
         const RlRecords rec{rl.rec_keys[0], rl.rec_val, rl.rec_count, rl.rec_idx[0]};

@@ -1,4 +1,7 @@
-// Closest-hit and any-hit BVH traversal.
+// Closest-hit and any-hit traversal of the reference's BVH. Most traces go
+// over the wide tree (wide_trace.hip) instead; these kernels serve launch
+// shapes that ask for the reference's visiting order, trees deeper than its
+// stack, scenes the wide tree does not take, and the no-allocation entry point.
 //
 // Reference: BVH::intersect and BVH::testVisibility (BVH/BVH.h:23-189), the
 // slab test of Core/BoundingBox.h:55-74 and Moller-Trumbore of
@@ -17,6 +20,8 @@
 #include "dev_common.h"
 #include "launch.h"
 #include "lbvh.h"
+#include "trace_common.h"
+#include "wide_trace.h"
 
 namespace cav {
 namespace {
@@ -45,43 +50,6 @@ __device__ __forceinline__ int stack_pop(int (*lds)[B], const volatile int* spil
     --sp;
     if (sp < D) return *(const lds_int*)(&lds[sp][threadIdx.x]);
     return spill[sp - D];
-}
-
-// Core/BoundingBox.h:55-74; returns the entry distance or -1.
-__device__ __forceinline__ float slab(float lx, float ly, float lz, float hx, float hy, float hz,
-                                      v3 o, v3 inv) {
-    const float t0x = (lx - o.x) * inv.x, t0y = (ly - o.y) * inv.y, t0z = (lz - o.z) * inv.z;
-    const float t1x = (hx - o.x) * inv.x, t1y = (hy - o.y) * inv.y, t1z = (hz - o.z) * inv.z;
-    const float maxmin = fmin_fmax(t0x, t1x, fmin_fmax(t0y, t1y, fmn(t0z, t1z)));
-    const float minmax = fmax_fmin(t0x, t1x, fmax_fmin(t0y, t1y, fmx(t0z, t1z)));
-    if (maxmin <= minmax && minmax > 0) return fmx(0.f, maxmin);
-    return -1.f;
-}
-
-// Core/Triangle.h:7-52
-__device__ __forceinline__ bool tri_hit(const TTri& tr, v3 o, v3 d, float& t, float& u, float& v) {
-    const v3 v0 = mk3(tr.a.x, tr.a.y, tr.a.z);
-    const v3 e1 = mk3(tr.b.x, tr.b.y, tr.b.z);
-    const v3 e2 = mk3(tr.c.x, tr.c.y, tr.c.z);
-    const v3 tvec = sub3(o, v0);
-    const v3 pvec = cross3(d, e2);
-    float det = dot3(e1, pvec);
-    if (det == 0) return false;
-    det = 1.f / det;
-    u = dot3(tvec, pvec) * det;
-    if (u < 0.0f || u > 1.0f) return false;
-    const v3 qvec = cross3(tvec, e1);
-    v = dot3(d, qvec) * det;
-    if (v < 0.0f || (u + v) > 1.0f) return false;
-    t = dot3(e2, qvec) * det;
-    return t > 0.f;
-}
-
-__device__ __forceinline__ void load_ray(const float* __restrict__ rays, int64_t i, v3& o, v3& d) {
-    const float2* r = reinterpret_cast<const float2*>(rays + i * 6);
-    const float2 a = r[0], b = r[1], c = r[2];
-    o = mk3(a.x, a.y, b.x);
-    d = mk3(b.y, c.x, c.y);
 }
 
 // Persistent closest-hit traversal: a fixed grid whose lanes each keep one
@@ -1051,12 +1019,6 @@ __global__ __launch_bounds__(64) void k_closest_coop(const TRec* __restrict__ re
     if (lane == 0 && nfetch > 0) atomicAdd(fetched, (unsigned long long)nfetch);
 }
 
-// 64-bit count of records fetched by closest-hit (words 16-17) or any-hit
-// (words 18-19) launches
-__host__ __device__ inline unsigned long long* fetch_word(uint32_t* counters, bool closest) {
-    return reinterpret_cast<unsigned long long*>(counters + (closest ? 16 : 18));
-}
-
 // zeroes n words; a kernel rather than hipMemsetAsync so the launch sequence
 // can be captured into a hipGraph
 __global__ void k_clear_words(uint32_t* p, int n) {
@@ -1066,13 +1028,7 @@ __global__ void k_clear_words(uint32_t* p, int n) {
 // Workgroups of a persistent launch of `threads`-thread workgroups:
 // max_per_cu per CU (0: as many as fit).
 int persistent_blocks(const void* kernel, int threads, int max_per_cu) {
-    // (initialised once, thread-safely: contexts on several threads launch here)
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
+    const int cus = device_cus();
     int per = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess || per <= 0)
         per = 4 * 256 / threads;
@@ -1162,22 +1118,31 @@ constexpr int64_t kPhase3Lanes = 16384;
 
 // Workgroups of a cooperative pass: as many one-wave workgroups as fit.
 int coop_grid(const void* kernel) {
-    int dev = 0, cus = 0, per = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        cus = 256;
+    const int cus = device_cus();
+    int per = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, 64, 0) != hipSuccess || per <= 0) per = 4;
     return cus * per;
 }
 
-// Any-hit in three launches: phase 1 (one lane per ray, long rays spilled),
-// phase 2 (a wave per spilled ray), phase 3 (rays phase 2 could not hold,
-// from their roots, one lane each; normally none). Words 20..25 of the
-// counters: spill count, spill cursor, failure count, phase-3 dispenser.
-void trace_any(const TRec* rec, int ntris, const float* rays, int64_t nrays, const uint32_t* nrays_dev,
+// Any-hit. Over the wide tree (its trace and the finishing pass) unless the
+// launch shape asks for the reference's visiting order or for sibling pairs,
+// or the BVH has no wide tree; else in three launches: phase 1 (one lane per
+// ray, long rays spilled), phase 2 (a wave per spilled ray), phase 3 (rays
+// phase 2 could not hold, from their roots, one lane each; normally none).
+// Words 20..25 of the counters: spill count, spill cursor, failure count,
+// phase-3 dispenser.
+void trace_any(const TraceBvh& bvh, const float* rays, int64_t nrays, const uint32_t* nrays_dev,
                const float* limit, const int32_t* src, const int32_t* dst, uint8_t* visible, uint32_t* counters,
-               const TraceLaunch& L, AnySpill* spill, uint32_t spill_cap, LaunchSink& ls) {
+               const TraceLaunch& L, const TraceCoop* tc, LaunchSink& ls) {
+    AnySpill* spill = tc ? tc->spill : nullptr;
+    const uint32_t spill_cap = tc ? tc->spill_cap : 0u;
     const bool coop = spill && spill_cap > 0 && nrays < (int64_t(1) << 32) && L.handoff < kNoHandoff;
+    if (coop && bvh.wide.nodes && !L.any_full && !any_step_pairs(L)) {
+        wide_occluded(bvh, rays, nrays, nrays_dev, limit, src, dst, visible, counters, L, *tc, ls);
+        return;
+    }
+    const TRec* rec = bvh.rec;
+    const int ntris = bvh.ntris;
     auto* disp = reinterpret_cast<unsigned long long*>(counters + 4);
     launch_any(L, nrays, ls, rec, rays, nrays, nrays_dev, (const uint32_t*)nullptr, limit, src, dst, visible,
                      counters + 1, disp, fetch_word(counters, false), coop ? spill : (AnySpill*)nullptr,
@@ -1198,15 +1163,24 @@ void trace_any(const TRec* rec, int ntris, const float* rays, int64_t nrays, con
                      (AnySpill*)nullptr, counters + 20, 0u, 0, L.any_full ? 0 : 1, 2 * ntris - 1);
 }
 
-// Closest-hit in three launches, like any-hit: phase 1 (one lane per ray,
-// long rays handed over), phase 2 (a wave per long ray, k_closest_coop),
-// phase 3 (the rays phase 2 sent back, one lane each, the reference's
-// order). Words 26..30 of the counters: long rays, their cursor, phase-3
-// dispenser (64-bit, words 28-29), phase-3 rays.
-void trace_near(const TRec* rec, int ntris, const float* root, const float* rays, int64_t nrays,
+// Closest-hit. Over the wide tree unless the launch shape asks for one lane
+// per ray in the reference's order (no hand-off) or the BVH has no wide tree;
+// else in three launches, like any-hit: phase 1 (one lane per ray, long rays
+// handed over), phase 2 (a wave per long ray, k_closest_coop), phase 3 (the
+// rays phase 2 sent back, one lane each, the reference's order). Words 26..30
+// of the counters: long rays, their cursor, phase-3 dispenser (64-bit, words
+// 28-29), phase-3 rays.
+void trace_near(const TraceBvh& bvh, const float* rays, int64_t nrays,
                 const uint32_t* nrays_dev, int32_t* prim, float* t, float* u, float* v, uint32_t* counters,
                 const TraceLaunch& L, const TraceCoop* coop, LaunchSink& ls) {
     const bool on = coop && coop->longs && coop->long_cap > 0 && nrays < (int64_t(1) << 32) && L.handoff < kNoHandoff;
+    if (on && bvh.wide.nodes) {
+        wide_closest(bvh, rays, nrays, nrays_dev, prim, t, u, v, counters, L, *coop, ls);
+        return;
+    }
+    const TRec* rec = bvh.rec;
+    const float* root = bvh.root;
+    const int ntris = bvh.ntris;
     LongRays lr;
     if (on) {
         lr.ids = coop->longs;
@@ -1230,8 +1204,7 @@ void trace_near(const TRec* rec, int ntris, const float* root, const float* rays
 
 }  // namespace
 
-hipError_t trace_closest(const TRec* rec, int ntris, const float* root,
-                         const float* rays, int64_t nrays, int32_t* prim, float* t, float* u,
+hipError_t trace_closest(const TraceBvh& bvh, const float* rays, int64_t nrays, int32_t* prim, float* t, float* u,
                          float* v, uint32_t* counters, const TraceLaunch& L, hipStream_t s,
                          const TraceCoop* coop) {
     if (nrays <= 0) return hipSuccess;
@@ -1239,11 +1212,11 @@ hipError_t trace_closest(const TRec* rec, int ntris, const float* root,
     if (e == hipSuccess) e = hipMemsetAsync(counters + 26, 0, 20, s);
     if (e != hipSuccess) return e;
     LaunchSink ls(s);
-    trace_near(rec, ntris, root, rays, nrays, nullptr, prim, t, u, v, counters, L, coop, ls);
+    trace_near(bvh, rays, nrays, nullptr, prim, t, u, v, counters, L, coop, ls);
     return ls.err;
 }
 
-hipError_t trace_occluded(const TRec* rec, int ntris, const float* rays,
+hipError_t trace_occluded(const TraceBvh& bvh, const float* rays,
                           const float* limit, const int32_t* src, const int32_t* dst,
                           int64_t nrays, uint8_t* visible, uint32_t* counters, const TraceLaunch& L,
                           hipStream_t s, const TraceCoop* coop) {
@@ -1252,8 +1225,7 @@ hipError_t trace_occluded(const TRec* rec, int ntris, const float* rays,
     if (e == hipSuccess) e = hipMemsetAsync(counters + 20, 0, 24, s);
     if (e != hipSuccess) return e;
     LaunchSink ls(s);
-    trace_any(rec, ntris, rays, nrays, nullptr, limit, src, dst, visible, counters, L,
-              coop ? coop->spill : nullptr, coop ? coop->spill_cap : 0u, ls);
+    trace_any(bvh, rays, nrays, nullptr, limit, src, dst, visible, counters, L, coop, ls);
     return ls.err;
 }
 
@@ -1261,41 +1233,39 @@ hipError_t trace_occluded(const TRec* rec, int ntris, const float* rays,
 // the grid is the full persistent size. counters as above. The dispensers
 // and pass counters are cleared by a kernel, so the sequence can be recorded
 // into a graph.
-void trace_closest_queue(const TRec* rec, int ntris, const float* root, const float* rays,
+void trace_closest_queue(const TraceBvh& bvh, const float* rays,
                          const uint32_t* nrays_dev, int64_t capacity, int32_t* prim, float* t, float* u, float* v,
                          uint32_t* counters, const TraceLaunch& L, LaunchSink& ls, const TraceCoop* coop) {
     ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 2, 2);
     if (coop && coop->longs && L.handoff < kNoHandoff)
         ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 26, 5);
-    trace_near(rec, ntris, root, rays, capacity, nrays_dev, prim, t, u, v, counters, L, coop, ls);
+    trace_near(bvh, rays, capacity, nrays_dev, prim, t, u, v, counters, L, coop, ls);
 }
 
-void trace_occluded_queue(const TRec* rec, int ntris, const float* rays, const uint32_t* nrays_dev,
+void trace_occluded_queue(const TraceBvh& bvh, const float* rays, const uint32_t* nrays_dev,
                           int64_t capacity, const float* limit, const int32_t* src, const int32_t* dst,
                           uint8_t* visible, uint32_t* counters, const TraceLaunch& L, LaunchSink& ls,
                           const TraceCoop* coop) {
     ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 4, 2);
     if (coop && coop->spill && L.handoff < kNoHandoff)
         ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 20, 6);
-    trace_any(rec, ntris, rays, capacity, nrays_dev, limit, src, dst, visible, counters, L,
-              coop ? coop->spill : nullptr, coop ? coop->spill_cap : 0u, ls);
+    trace_any(bvh, rays, capacity, nrays_dev, limit, src, dst, visible, counters, L, coop, ls);
 }
 
-hipError_t trace_closest_queue(const TRec* rec, int ntris, const float* root,
-                               const float* rays, const uint32_t* nrays_dev, int64_t capacity,
+hipError_t trace_closest_queue(const TraceBvh& bvh, const float* rays, const uint32_t* nrays_dev, int64_t capacity,
                                int32_t* prim, float* t, float* u, float* v, uint32_t* counters,
                                const TraceLaunch& L, hipStream_t s, const TraceCoop* coop) {
     LaunchSink ls(s);
-    trace_closest_queue(rec, ntris, root, rays, nrays_dev, capacity, prim, t, u, v, counters, L, ls, coop);
+    trace_closest_queue(bvh, rays, nrays_dev, capacity, prim, t, u, v, counters, L, ls, coop);
     return ls.err;
 }
 
-hipError_t trace_occluded_queue(const TRec* rec, int ntris, const float* rays,
+hipError_t trace_occluded_queue(const TraceBvh& bvh, const float* rays,
                                 const uint32_t* nrays_dev, int64_t capacity, const float* limit,
                                 const int32_t* src, const int32_t* dst, uint8_t* visible,
                                 uint32_t* counters, const TraceLaunch& L, hipStream_t s, const TraceCoop* coop) {
     LaunchSink ls(s);
-    trace_occluded_queue(rec, ntris, rays, nrays_dev, capacity, limit, src, dst, visible, counters, L, ls, coop);
+    trace_occluded_queue(bvh, rays, nrays_dev, capacity, limit, src, dst, visible, counters, L, ls, coop);
     return ls.err;
 }
 

@@ -1,0 +1,53 @@
+// The wide traversal tree: an 8-wide tree with 8-bit child boxes over the
+// triangles, built beside the reference's BVH and walked by the closest-hit
+// and any-hit traces in its place; see wide.hip and wide_trace.hip.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "dev_common.h"
+#include "lbvh.h"
+
+namespace cav {
+
+// One node, 128 bytes (one L2 line), eight 16-byte words:
+//   0: box origin xyz | scale exponents x, y, z (biased, one byte each) and
+//      the mask of slots holding an inner child
+//   1: first inner child's node | first triangle | 8 slot bytes (WideSlot)
+//   2, 3, 4: x, y, z: 8 low planes, 8 high planes, in units of 2^exponent
+//      from the origin, rounded outwards
+//   5: build only: {binary node, first leaf, last leaf, 0}
+// Inner children lie one after the other in slot order, and so do the
+// triangles of the leaf slots.
+// A slot's byte: 0 empty; inner 1 << 5 | (24 + slot); leaf of c triangles
+// ((1 << c) - 1) << 5 | offset from the first triangle.
+constexpr int kWideWords = 8;
+constexpr int kWideLeaf = 3;  // triangles per leaf slot at most
+// nodes for n triangles: a node with inner children has all 8 slots filled,
+// one without holds at least 4 triangles (or is the root)
+inline int64_t wide_node_capacity(int64_t n) { return 2 * n / 7 + 16; }
+
+// Scratch and results of one build (library-owned, sized for n triangles).
+struct WideBuffers {
+    void* base = nullptr;  // the one allocation that holds the rest
+    uint32_t* keys[2] = {nullptr, nullptr};
+    uint32_t* vals[2] = {nullptr, nullptr};
+    NodeBox* nbox = nullptr;             // the binary tree over the wide tree's codes
+    int4* topo = nullptr;
+    unsigned long long* gate = nullptr;  // bottom_up_gate_words(n), zero between builds
+    uint32_t* ctr = nullptr;             // kWideCtrWords
+    uint32_t* bounds = nullptr;          // 6 order-preserving ints: the triangles' box
+    uint4* nodes = nullptr;
+    float4* tris = nullptr;
+    int32_t* leaf_of = nullptr;
+};
+constexpr int kWideCtrWords = 96;
+size_t wide_bytes(int n);
+void wide_carve(WideBuffers& w, void* base, int n);
+// Builds the tree. bounds: the triangles' box (b.scene_ord when the caller
+// gave none, else w.bounds). Uses b's sort work space and level list as
+// scratch, on the same stream as b's own build and after it.
+hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, const float* tris, const int32_t* mesh, int n,
+                      const uint32_t* bounds, hipStream_t s, Marker* mk);
+
+}  // namespace cav

@@ -1,0 +1,915 @@
+// Closest-hit and any-hit traces over the wide tree (wide.h), with the
+// reference's answers bit for bit (BVH::intersect and BVH::testVisibility,
+// BVH/BVH.h:23-189).
+//
+// Why another tree gives the same answers. A triangle is a candidate when the
+// reference can reach its leaf: when the ray hits the leaf's own box. The slab
+// test (Core/BoundingBox.h:55-74) is monotone under box inclusion -- the
+// subtraction, the product with the ray's reciprocal direction, min and max
+// all are -- so a ray that hits the leaf's box hits every box above it, and
+// starts in them no later -- unless the ray runs exactly along a plane of the
+// leaf's box (0 * inf = NaN in the slab test, which then can fail further up):
+// such a hit counts only after every box above it has been tested (grazes,
+// leaf_path). The triangle's vertices are in the wide tree's
+// record, so its leaf box is tested here exactly as the reference tests it.
+//
+// Any-hit: the answer is whether any candidate blocks the ray before its
+// limit, which no order changes.
+//
+// Closest-hit: the nearest candidate M is the reference's answer unless it
+// skips M, and it skips a box only at or beyond a hit X found before: every
+// box on M's path starts at or before M's own (e_M), so such an X lies at or
+// before max(t_M, e_M). A ray that met another hit X with t_X <= max(t_M,
+// e_M) -- coincident surfaces, a box standing on a floor -- goes to
+// k_wide_finish, which collects all hits that close and replays the
+// reference's order among them from the reference's tree.
+//
+// The wide boxes only have to contain the exact ones. They are rounded
+// outwards, their planes' distances carry a slack of 2^-20 of their terms
+// (the two roundings are 2^-23 each), and boxes are skipped only beyond
+// kReach = 1 + 2^-5 times the nearest hit (any-hit: times the limit). A
+// triangle beyond that could matter only if Moller-Trumbore put its t more
+// than 2^-6 (relative) short of the start of its own box: the same
+// assumption, with a margin 16 times wider, that the cooperative passes over
+// the reference's tree make (traverse.hip).
+//
+// Per node and lane: five 16-byte loads from one line and about 230 VALU
+// instructions for eight children, against four loads and 90 instructions
+// for the two children of a reference node; a stack entry holds all of a
+// node's remaining children.
+#include <algorithm>
+#include <cfloat>
+
+#include "dev_common.h"
+#include "launch.h"
+#include "lbvh.h"
+#include "trace_common.h"
+#include "wide.h"
+#include "wide_trace.h"
+
+namespace cav {
+namespace {
+
+constexpr float kReach = 1.0f + 1.0f / 32.0f;
+constexpr float kOwnBox = 1.0f + 1.0f / 64.0f;  // a box starting further beyond its hit: the reference decides
+constexpr float kSlack = 1.0f / 1048576.0f;     // 2^-20
+constexpr float kFarthest = 1099511627776.f;    // 2^40: origins beyond go to the reference's traversal
+constexpr int kWideStack = 12;                  // stack entries in LDS
+constexpr int kWideDeep = 68;                   // entries in all: more than a tree over 32-bit codes has levels
+constexpr int kUndecided = -2;                  // hit id of a ray that the finishing pass still has to find by scanning
+
+// The ray as the node tests use it: direction scaled to a largest component
+// in [1, 2) (a power of two, exact), reciprocals bounded by 2^60 so that an
+// axis the ray runs along gives huge distances instead of infinities.
+struct WideRay {
+    v3 o, inv;
+    float scale;  // true t * scale = t in the scaled direction
+    uint32_t oct;
+};
+__device__ __forceinline__ float wide_rcp(float d) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    return __builtin_copysignf(fmn(fabsf(r), 1152921504606846976.f), d);
+}
+enum RayKind {
+    kRayFine,
+    kRayOdd,  // only the reference's traversal takes it: from beyond 2^40, or a direction near float's limits
+    kRayDead  // hits nothing: a zero direction (every determinant is 0) or one that is not finite, or a NaN
+              // origin (Moller-Trumbore's t is 0 or NaN for every finite triangle)
+};
+__device__ __forceinline__ RayKind wide_ray(v3 o, v3 d, WideRay& r) {
+    const float m = fmx(fabsf(d.x), fmx(fabsf(d.y), fabsf(d.z)));
+    const uint32_t e = __float_as_uint(m) >> 23;
+    const bool dead = !(fabsf(d.x) <= FLT_MAX && fabsf(d.y) <= FLT_MAX && fabsf(d.z) <= FLT_MAX) || m == 0.f ||
+                      !(o.x == o.x && o.y == o.y && o.z == o.z);
+    const bool fine = fabsf(o.x) <= kFarthest && fabsf(o.y) <= kFarthest && fabsf(o.z) <= kFarthest && e >= 2u &&
+                      e <= 252u;
+    r.o = o;
+    r.scale = __uint_as_float(e << 23);
+    const float down = __uint_as_float((254u - e) << 23);
+    r.inv = mk3(wide_rcp(d.x * down), wide_rcp(d.y * down), wide_rcp(d.z * down));
+    r.oct = (r.inv.x < 0.f ? 1u : 0u) | (r.inv.y < 0.f ? 2u : 0u) | (r.inv.z < 0.f ? 4u : 0u);
+    return dead ? kRayDead : (fine ? kRayFine : kRayOdd);
+}
+
+// Bits of a node's eight slot bytes, four at a time: the inner ones get the
+// ray's octant xored into their slot, so that ascending bits go front to back.
+__device__ __forceinline__ uint32_t order_slots(uint32_t meta, uint32_t oct4) {
+    const uint32_t inner = (meta & (meta << 1)) & 0x10101010u;  // 24 + slot: bits 3 and 4
+    return meta ^ (oct4 & ((inner >> 4) * 7u));
+}
+
+// One axis of one node: plane distances are q * a + b.
+struct AxisPlanes {
+    float an, af, bn, bf;
+};
+__device__ __forceinline__ AxisPlanes axis_planes(float p, uint32_t e, float o, float inv) {
+    const float a = __uint_as_float(e << 23) * inv, b = (p - o) * inv;
+    AxisPlanes r;
+    r.an = __builtin_fmaf(-kSlack, fabsf(a), a);
+    r.af = __builtin_fmaf(kSlack, fabsf(a), a);
+    r.bn = __builtin_fmaf(-kSlack, fabsf(b), b);
+    r.bf = __builtin_fmaf(kSlack, fabsf(b), b);
+    return r;
+}
+__device__ __forceinline__ float ubyte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 255u); }
+
+// Tests a node's children against the ray up to `cut` (scaled units): bits
+// 0..23 the triangles of hit leaf slots, 24..31 the hit inner children in
+// front-to-back order.
+__device__ __forceinline__ uint32_t test_children(const uint4& w0, const uint4& w1, const uint4& w2, const uint4& w3,
+                                                  const uint4& w4, const WideRay& r, float cut) {
+    const AxisPlanes x = axis_planes(__uint_as_float(w0.x), w0.w & 255u, r.o.x, r.inv.x);
+    const AxisPlanes y = axis_planes(__uint_as_float(w0.y), (w0.w >> 8) & 255u, r.o.y, r.inv.y);
+    const AxisPlanes z = axis_planes(__uint_as_float(w0.z), (w0.w >> 16) & 255u, r.o.z, r.inv.z);
+    const bool nx = r.inv.x < 0.f, ny = r.inv.y < 0.f, nz = r.inv.z < 0.f;
+    const uint32_t oct4 = r.oct * 0x01010101u;
+    uint32_t mask = 0;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const uint32_t lx = half ? w2.y : w2.x, hx = half ? w2.w : w2.z;
+        const uint32_t ly = half ? w3.y : w3.x, hy = half ? w3.w : w3.z;
+        const uint32_t lz = half ? w4.y : w4.x, hz = half ? w4.w : w4.z;
+        const uint32_t xn = nx ? hx : lx, xf = nx ? lx : hx;
+        const uint32_t yn = ny ? hy : ly, yf = ny ? ly : hy;
+        const uint32_t zn = nz ? hz : lz, zf = nz ? lz : hz;
+        const uint32_t meta = order_slots(half ? w1.w : w1.z, oct4);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float tn = fmx(fmx(__builtin_fmaf(ubyte(xn, k), x.an, x.bn), __builtin_fmaf(ubyte(yn, k), y.an, y.bn)),
+                                 fmx(__builtin_fmaf(ubyte(zn, k), z.an, z.bn), 0.f));
+            const float tf = fmn(fmn(__builtin_fmaf(ubyte(xf, k), x.af, x.bf), __builtin_fmaf(ubyte(yf, k), y.af, y.bf)),
+                                 fmn(__builtin_fmaf(ubyte(zf, k), z.af, z.bf), cut));
+            const uint32_t m = meta >> (8 * k);
+            const uint32_t bits = ((m >> 5) & 7u) << (m & 31u);
+            mask |= tn <= tf ? bits : 0u;
+        }
+    }
+    return mask;
+}
+
+// Whether a slab test divides 0 by 0 on an axis: the ray does not move along
+// it and starts on one of the box's two planes.
+__device__ __forceinline__ bool grazes(float inv, float o, float lo, float hi) {
+    return fabsf(inv) == INFINITY && (o == lo || o == hi);
+}
+
+// The triangle's own box as the reference's leaf has it (Core/Triangle.h:242-268)
+// and where the ray enters it (-1: never). touch: the ray runs along a plane of
+// the box (see grazes).
+__device__ __forceinline__ float leaf_entry(const float4& a, const float4& b, const float4& c, v3 o, v3 d, bool& touch) {
+    const v3 inv = div3(mk3(1.f, 1.f, 1.f), d);
+    const v3 lo = mk3(fmn(a.x, fmn(b.x, c.x)), fmn(a.y, fmn(b.y, c.y)), fmn(a.z, fmn(b.z, c.z)));
+    const v3 hi = mk3(fmx(a.x, fmx(b.x, c.x)), fmx(a.y, fmx(b.y, c.y)), fmx(a.z, fmx(b.z, c.z)));
+    touch = grazes(inv.x, o.x, lo.x, hi.x) || grazes(inv.y, o.y, lo.y, hi.y) || grazes(inv.z, o.z, lo.z, hi.z);
+    return slab(lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, o, inv);
+}
+__device__ __forceinline__ bool wide_tri_hit(const float4& a, const float4& b, const float4& c, v3 o, v3 d, float& t,
+                                             float& u, float& v) {
+    TTri tr;
+    tr.a = a;
+    tr.b = make_float4(b.x - a.x, b.y - a.y, b.z - a.z, 0.f);
+    tr.c = make_float4(c.x - a.x, c.y - a.y, c.z - a.z, 0.f);
+    return tri_hit(tr, o, d, t, u, v);
+}
+
+// Rays a wave takes at a time: `chunk` at most, fewer when the batch would
+// not give every wave of the grid its share.
+__device__ __forceinline__ int share_of(int64_t nrays, int chunk) {
+    const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
+    int64_t c = (nrays + waves - 1) / waves;
+    c = (c + 63) / 64 * 64;
+    return (int)(c < chunk ? (c < 64 ? 64 : c) : chunk);
+}
+
+// A wave's next rays for the lanes that need one (wave-uniform control flow):
+// the dispenser is asked once per chunk. Returns the lane's ray number.
+struct Dispenser {
+    int64_t base = 0;
+    int avail = 0;
+    __device__ __forceinline__ int64_t next(uint64_t need, int lane, unsigned long long* counter, int chunk) {
+        const int cnt = __popcll(need), rank = __popcll(need & ((1ull << lane) - 1ull));
+        int64_t mine;
+        if (avail < cnt) {
+            unsigned long long nb = 0;
+            const int first = __ffsll((long long)need) - 1;
+            if (lane == first) nb = atomicAdd(counter, (unsigned long long)chunk);
+            nb = __shfl(nb, first, 64);
+            mine = rank < avail ? base + rank : (int64_t)nb + (rank - avail);
+            base = (int64_t)nb + (cnt - avail);
+            avail = chunk - (cnt - avail);
+        } else {
+            mine = base + rank;
+            base += cnt;
+            avail -= cnt;
+        }
+        return mine;
+    }
+};
+
+// Stack of a lane: entry {first inner child, mask of inner slots << 8 |
+// remaining children's bits}; the first kWideStack in LDS, the rest (skewed
+// trees only) in scratch.
+template <int B>
+struct WideStackLds {
+    uint32_t base[kWideStack][B];
+    uint16_t bits[kWideStack][B];
+};
+
+struct WideList {           // rays left to the finishing pass
+    uint32_t* ids = nullptr;
+    uint32_t* n = nullptr;  // rays listed (past cap: the rest are marked in the hit ids)
+    uint32_t cap = 0;
+    int after = 0;          // steps before a ray still in flight at the batch's end is listed (0: never)
+};
+
+// kAny: any-hit (limit, src, dst, ovis) instead of closest-hit (oprim ...).
+template <bool kAny, int B>
+__global__ __launch_bounds__(B) void k_wide_trace(const uint4* __restrict__ nodes, const float4* __restrict__ tris,
+                                                  const float* __restrict__ rays, int64_t nrays_arg,
+                                                  const uint32_t* __restrict__ nrays_dev,
+                                                  int32_t* __restrict__ oprim, float* __restrict__ ot,
+                                                  float* __restrict__ ou, float* __restrict__ ov,
+                                                  const float* __restrict__ limit, const int32_t* __restrict__ src,
+                                                  const int32_t* __restrict__ dst, uint8_t* __restrict__ ovis,
+                                                  uint32_t* __restrict__ overflow,
+                                                  unsigned long long* __restrict__ next_ray,
+                                                  unsigned long long* __restrict__ fetched, WideList wl, int chunk_arg) {
+    __shared__ WideStackLds<B> lds;
+    const int lane = threadIdx.x & 63;
+    const int64_t nrays = nrays_dev ? (int64_t)*nrays_dev : nrays_arg;
+    const int chunk = share_of(nrays, chunk_arg);
+
+    int64_t ri = -1;  // ray held by this lane; -1 = needs one, -2 = none left
+    WideRay r;
+    r.o = r.inv = mk3(0, 0, 0);
+    r.scale = 1.f;
+    r.oct = 0;
+    v3 d = mk3(0, 0, 0);
+    float best = FLT_MAX, own = 0.f, bu = 0.f, bv = 0.f, cut = 0.f;  // own: where the nearest hit's box starts
+    int bp = -1, sm = -1, dm = -1, steps = 0;
+    bool unsure = false, grazed = false, may_list = false, drained = false;
+    uint32_t cbase = 0, group = 0;  // the current node's inner children: first one, slot mask << 8 | bits to visit
+    uint32_t tbase = 0, tbits = 0;  // triangles to test
+    int sp = 0, maxsp = 0;
+    uint32_t deep[2 * (kWideDeep - kWideStack)];
+    uint64_t nfetch = 0;
+    Dispenser disp;
+
+    while (true) {
+        const uint64_t need = __ballot(ri == -1);
+        if (need) {
+            const int64_t mine = disp.next(need, lane, next_ray, chunk);
+            if (ri == -1) {
+                ri = mine < nrays ? mine : -2;
+                if (ri >= 0) {
+                    v3 o;
+                    load_ray(rays, ri, o, d);
+                    const RayKind kind = wide_ray(o, d, r);
+                    best = FLT_MAX; own = 0.f; bp = -1; bu = 0.f; bv = 0.f;
+                    unsure = kind == kRayOdd;
+                    grazed = false;
+                    may_list = wl.after > 0;
+                    steps = 0; sp = 0; tbits = 0;
+                    cbase = 0;
+                    group = (1u << 8) | (1u << r.oct);  // the root, as slot 0 of a node of one child
+                    cut = FLT_MAX;
+                    if (kAny) {
+                        best = limit[ri];
+                        const bool use = !(best == INFINITY);
+                        if (use) cut = best * kReach * r.scale;
+                        if (use && !(best > 0.f)) group = 0;  // nothing lies before it
+                        sm = src ? src[ri] : -1;
+                        dm = dst ? dst[ri] : -1;
+                    }
+                    if (kind != kRayFine) group = 0;
+                }
+            }
+        }
+        if (!__ballot(ri >= 0)) break;  // every lane is out of rays
+        if (ri < 0) continue;
+
+        bool done = false, listed = false, hit = false;
+        if (may_list && steps >= wl.after) {
+            if (!drained && ((steps - wl.after) & 255) == 0)
+                drained = (int64_t)__hip_atomic_load(next_ray, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= nrays;
+            if (drained) {  // a long ray at the end: a whole wave finishes it
+                const uint32_t slot = atomicAdd(wl.n, 1u);
+                if (slot < wl.cap) {
+                    wl.ids[slot] = (uint32_t)ri;
+                    done = listed = true;
+                }
+                may_list = false;
+            }
+        }
+        ++steps;
+
+        if (!done && tbits == 0) {
+            if ((group & 255u) == 0u) {
+                if (sp == 0) {
+                    done = true;
+                } else {
+                    --sp;
+                    if (sp < kWideStack) {
+                        cbase = lds.base[sp][threadIdx.x];
+                        group = lds.bits[sp][threadIdx.x];
+                    } else {
+                        cbase = deep[2 * (sp - kWideStack)];
+                        group = deep[2 * (sp - kWideStack) + 1];
+                    }
+                }
+            }
+            if (!done) {
+                const int bit = __ffs((int)(group & 255u)) - 1;
+                group &= group - 1u;
+                const uint32_t slot = (uint32_t)bit ^ r.oct;
+                const uint32_t child = cbase + (uint32_t)__popc((group >> 8) & ((1u << slot) - 1u));
+                if (group & 255u) {
+                    if (sp < kWideStack) {
+                        lds.base[sp][threadIdx.x] = cbase;
+                        lds.bits[sp][threadIdx.x] = (uint16_t)group;
+                    } else {
+                        deep[2 * (sp - kWideStack)] = cbase;
+                        deep[2 * (sp - kWideStack) + 1] = group;
+                    }
+                    ++sp;
+                    maxsp = max(maxsp, sp);
+                }
+                const uint4* nd = nodes + (int64_t)child * kWideWords;
+                const uint4 w0 = nd[0], w1 = nd[1], w2 = nd[2], w3 = nd[3], w4 = nd[4];
+                ++nfetch;
+                const uint32_t mask = test_children(w0, w1, w2, w3, w4, r, cut);
+                cbase = w1.x;
+                tbase = w1.y;
+                tbits = mask & 0xffffffu;
+                group = ((w0.w >> 24) << 8) | (mask >> 24);
+            }
+        }
+        if (!done && tbits != 0) {
+            const uint32_t k = (uint32_t)__ffs((int)tbits) - 1u;
+            tbits &= tbits - 1u;
+            const float4* tp = tris + (int64_t)(tbase + k) * 3;
+            const float4 a = tp[0], b = tp[1], c = tp[2];
+            ++nfetch;
+            float t, u, v;
+            if (kAny) {
+                const int mesh = __float_as_int(b.w);
+                if (mesh != sm && mesh != dm && wide_tri_hit(a, b, c, r.o, d, t, u, v) &&
+                    (best == INFINITY || t < best)) {
+                    bool touch;
+                    const bool in = leaf_entry(a, b, c, r.o, d, touch) >= 0.f;
+                    if (in && touch) unsure = true;
+                    else if (in) done = hit = true;
+                }
+            } else if (wide_tri_hit(a, b, c, r.o, d, t, u, v) && t <= fmx(best, own)) {
+                bool touch;
+                const float e = leaf_entry(a, b, c, r.o, d, touch);
+                if (e >= 0.f) {
+                    if (touch) {
+                        grazed = true;
+                    } else if (t < best) {
+                        // the earlier nearest hit is this one's only possible rival so far
+                        unsure = best <= fmx(t, e) || e > t * kOwnBox;
+                        best = t; own = e; bu = u; bv = v; bp = __float_as_int(a.w);
+                        cut = t * kReach * r.scale;
+                    } else {
+                        unsure = true;
+                    }
+                }
+            }
+        }
+        if (done) {
+            if (listed) {
+                // nothing to write
+            } else if (kAny) {
+                ovis[ri] = hit ? 0 : 1;
+                if (unsure && !hit) {
+                    const uint32_t slot = atomicAdd(wl.n, 1u);
+                    if (slot < wl.cap) wl.ids[slot] = (uint32_t)ri;
+                    else ovis[ri] = 255;
+                }
+            } else {
+                oprim[ri] = bp;
+                ot[ri] = bp >= 0 ? best : 0.f;
+                if (ou) ou[ri] = bu;
+                if (ov) ov[ri] = bv;
+                if (unsure || grazed) {
+                    const uint32_t slot = atomicAdd(wl.n, 1u);
+                    if (slot < wl.cap) wl.ids[slot] = (uint32_t)ri;
+                    else oprim[ri] = kUndecided;
+                }
+            }
+            ri = -1;
+        }
+    }
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) {
+        maxsp = max(maxsp, __shfl_xor(maxsp, dd, 64));
+        nfetch += __shfl_xor(nfetch, dd, 64);
+    }
+    if (lane == 0 && maxsp > 0) atomicMax(overflow + 6, (uint32_t)maxsp);
+    if (lane == 0 && nfetch > 0) atomicAdd(fetched, (unsigned long long)nfetch);
+}
+
+// ------------------------------------------------------------- finishing pass
+// One wave per listed ray, from the wide tree's root: pending nodes in LDS,
+// eight at a time, one child per lane. Closest-hit collects every hit within
+// kReach of the nearest (64 at most) and, when several lie close enough for
+// the reference's order to decide, replays that order; any-hit stops at the
+// first blocker. A ray that does not fit goes through the reference's tree on
+// one lane of the wave.
+constexpr int kPend = 1024;
+constexpr int kCands = 64;
+constexpr int kRefStack = 64;  // BVH/BVH.h:41,122
+
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Where a leaf comes in the reference's depth-first traversal of a ray: its
+// path from the root, bit 63 first, 1 where it goes to the child taken second
+// (the farther one, the right one on ties; BVH/BVH.h:83-94). The leaf earlier
+// in that order has the smaller path, and two paths part at their leaves'
+// lowest common ancestor. reach: the ray hits every box on the path below the
+// root's. The tree has at most 64 levels; false: the walk did not end (never
+// for a valid tree).
+__device__ bool leaf_path(const WideDev& w, int leaf, v3 o, v3 inv, uint64_t& path, int& depth, bool& reach) {
+    path = 0;
+    depth = 0;
+    reach = true;
+    for (int x = leaf; x != 0;) {
+        if (depth >= kRefStack) return false;
+        const int p = w.topo[x].z;
+        const int4 t = w.topo[p];
+        const NodeBox l = w.nbox[t.x], r = w.nbox[t.y];
+        const float dl = slab(l.a.x, l.a.y, l.a.z, l.b.x, l.b.y, l.b.z, o, inv);
+        const float dr = slab(r.a.x, r.a.y, r.a.z, r.b.x, r.b.y, r.b.z, o, inv);
+        reach = reach && (t.x == x ? dl : dr) >= 0.f;
+        const bool second = (dl > dr) == (t.x == x);
+        path = (path >> 1) | (second ? 1ull << 63 : 0ull);
+        x = p;
+        ++depth;
+    }
+    return true;
+}
+
+// Whether the ray hits every box above a triangle's leaf (but the root's).
+__device__ bool reached(const WideDev& w, int prim, v3 o, v3 d, bool& bad) {
+    uint64_t path;
+    int depth;
+    bool reach;
+    if (!leaf_path(w, w.leaf_of[prim], o, div3(mk3(1.f, 1.f, 1.f), d), path, depth, reach)) bad = true;
+    return reach;
+}
+
+// The reference's traversal of one ray by one lane (k_trace / k_trace_any).
+__device__ void reference_closest(const TRec* recs, const float* root, v3 o, v3 d, int max_steps, int* stack,
+                                  int& prim, float& t, float& u, float& v, uint32_t& ovf) {
+    const v3 inv = div3(mk3(1.f, 1.f, 1.f), d);
+    float best = FLT_MAX, bu = 0.f, bv = 0.f;
+    bool hit = false;
+    int bp = -1, cur = 0, sp = 0;
+    prim = -1; t = u = v = 0.f;
+    if (slab(root[0], root[1], root[2], root[3], root[4], root[5], o, inv) < 0.f) return;
+    for (int steps = 0;; ++steps) {
+        if (steps >= max_steps) { ++ovf; break; }
+        const float4* rec = reinterpret_cast<const float4*>(recs + (cur >= 0 ? cur : ~cur));
+        const float4 q0 = rec[0], q1 = rec[1], q2 = rec[2];
+        bool next = false;
+        if (cur >= 0) {
+            const int4 refs = reinterpret_cast<const int4*>(rec)[3];
+            const float dl = slab(q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, o, inv);
+            const float dr = slab(q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, o, inv);
+            const bool hl = dl >= 0 && dl < best, hr = dr >= 0 && dr < best;
+            if (hl && hr) {
+                const bool lfar = dl > dr;
+                if (sp < kRefStack) stack[sp++] = lfar ? refs.x : refs.y; else ++ovf;
+                if (sp < kRefStack) { cur = lfar ? refs.y : refs.x; next = true; } else ++ovf;
+            } else if (hl || hr) {
+                if (sp < kRefStack) { cur = hl ? refs.x : refs.y; next = true; } else ++ovf;
+            }
+        } else {
+            float ht, hu, hv;
+            if (tri_hit(TTri{q0, q1, q2}, o, d, ht, hu, hv) && (!hit || ht < best)) {
+                hit = true; best = ht; bu = hu; bv = hv; bp = __float_as_int(q0.w);
+            }
+        }
+        if (!next) {
+            if (sp == 0) break;
+            cur = stack[--sp];
+        }
+    }
+    if (hit) { prim = bp; t = best; u = bu; v = bv; }
+}
+__device__ bool reference_blocked(const TRec* recs, v3 o, v3 d, float lim, int sm, int dm, int max_steps, int* stack,
+                                  uint32_t& ovf) {
+    const v3 inv = div3(mk3(1.f, 1.f, 1.f), d);
+    const bool use = !(lim == INFINITY);
+    int cur = 0, sp = 0;
+    for (int steps = 0;; ++steps) {
+        if (steps >= max_steps) { ++ovf; return false; }
+        const float4* rec = reinterpret_cast<const float4*>(recs + (cur >= 0 ? cur : ~cur));
+        const float4 q0 = rec[0], q1 = rec[1], q2 = rec[2];
+        bool next = false;
+        if (cur >= 0) {
+            const int4 refs = reinterpret_cast<const int4*>(rec)[3];
+            const float dl = slab(q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, o, inv);
+            const float dr = slab(q1.z, q1.w, q2.x, q2.y, q2.z, q2.w, o, inv);
+            const bool hl = dl >= 0, hr = dr >= 0;
+            if (hl && hr) {
+                const bool lfar = dl > dr;
+                if (sp < kRefStack) stack[sp++] = lfar ? refs.x : refs.y; else ++ovf;
+                if (sp < kRefStack) { cur = lfar ? refs.y : refs.x; next = true; } else ++ovf;
+            } else if (hl || hr) {
+                if (sp < kRefStack) { cur = hl ? refs.x : refs.y; next = true; } else ++ovf;
+            }
+        } else {
+            const int mesh = __float_as_int(q1.w);
+            float t, u, v;
+            if (mesh != sm && mesh != dm && tri_hit(TTri{q0, q1, q2}, o, d, t, u, v) && (!use || t < lim)) return true;
+        }
+        if (!next) {
+            if (sp == 0) return false;
+            cur = stack[--sp];
+        }
+    }
+}
+
+struct FinishLds {
+    uint32_t pend[kPend];
+    float t[kCands], u[kCands], v[kCands], e[kCands];
+    int32_t p[kCands];
+    int stack[kRefStack];
+};
+
+// A lane's child of a pending node: its wide box against the ray. Returns the
+// slot byte's meaning: inner child index (inner set) or first triangle and
+// count; count 0 and !inner: nothing hit.
+__device__ __forceinline__ void lane_child(const uint4* nd, int slot, const WideRay& r, float cut, bool& inner,
+                                           uint32_t& at, int& count) {
+    const uint4 w0 = nd[0], w1 = nd[1];
+    const uint8_t* by = reinterpret_cast<const uint8_t*>(nd);
+    const uint32_t m = by[24 + slot];
+    inner = false;
+    at = 0;
+    count = 0;
+    if (m == 0u) return;
+    float tn = 0.f, tf = cut;
+    const float org[3] = {__uint_as_float(w0.x), __uint_as_float(w0.y), __uint_as_float(w0.z)};
+    const float ro[3] = {r.o.x, r.o.y, r.o.z}, ri[3] = {r.inv.x, r.inv.y, r.inv.z};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const AxisPlanes ap = axis_planes(org[k], (w0.w >> (8 * k)) & 255u, ro[k], ri[k]);
+        const float lo = (float)by[32 + 16 * k + slot], hi = (float)by[40 + 16 * k + slot];
+        tn = fmx(tn, __builtin_fmaf(ri[k] < 0.f ? hi : lo, ap.an, ap.bn));
+        tf = fmn(tf, __builtin_fmaf(ri[k] < 0.f ? lo : hi, ap.af, ap.bf));
+    }
+    if (!(tn <= tf)) return;
+    const uint32_t imask = w0.w >> 24;
+    if ((imask >> slot) & 1u) {
+        inner = true;
+        at = w1.x + (uint32_t)__popc(imask & ((1u << slot) - 1u));
+    } else {
+        at = w1.y + (m & 31u);
+        count = __popc(m >> 5);
+    }
+}
+
+struct FinishArgs {
+    WideDev w;
+    const TRec* recs;
+    const float* root;
+    const float* rays;
+    int64_t nrays;
+    const uint32_t* nrays_dev;
+    const uint32_t* ids;
+    const uint32_t* n;
+    uint32_t cap;
+    uint32_t* fails;  // rays that took the reference's traversal
+    uint32_t* overflow;
+    unsigned long long* fetched;
+    int ntris;
+};
+
+__device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, int32_t* oprim, float* ot, float* ou,
+                               float* ov, uint64_t& nfetch) {
+    const int lane = threadIdx.x;
+    v3 o, d;
+    load_ray(A.rays, ri, o, d);
+    WideRay r;
+    const RayKind kind = wide_ray(o, d, r);
+    bool failed = kind == kRayOdd;
+    bool bad = false;  // a walk up the reference's tree did not end
+    const bool root_hit = slab(A.root[0], A.root[1], A.root[2], A.root[3], A.root[4], A.root[5], o,
+                               div3(mk3(1.f, 1.f, 1.f), d)) >= 0.f;
+    float best = FLT_MAX;
+    int count = kind == kRayFine ? 1 : 0, nc = 0;
+    if (lane == 0) L.pend[0] = 0u;
+    wave_fence();
+    while (count > 0) {
+        const int k = count < 8 ? count : 8;
+        const int g = lane >> 3;
+        bool inner = false;
+        uint32_t at = 0;
+        int nt = 0;
+        if (g < k) {
+            const uint32_t node = L.pend[count - 1 - g];
+            const float cut = best == FLT_MAX ? FLT_MAX : best * kReach * r.scale;
+            lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, cut, inner, at, nt);
+            nfetch += (lane & 7) == 0 ? 1u : 0u;
+        }
+        count -= k;
+        wave_fence();
+        for (int j = 0; j < kWideLeaf; ++j) {
+            float t = 0.f, u = 0.f, v = 0.f, e = -1.f;
+            int p = -1;
+            bool hit = false;
+            if (j < nt) {
+                const float4* tp = A.w.tris + (int64_t)(at + (uint32_t)j) * 3;
+                const float4 a = tp[0], b = tp[1], c = tp[2];
+                ++nfetch;
+                if (wide_tri_hit(a, b, c, o, d, t, u, v)) {
+                    bool touch;
+                    e = leaf_entry(a, b, c, o, d, touch);
+                    hit = e >= 0.f && t < FLT_MAX && e < FLT_MAX;
+                    p = __float_as_int(a.w);
+                    if (hit && touch) hit = root_hit && reached(A.w, p, o, d, bad);
+                }
+            }
+            float m = hit ? t : FLT_MAX;
+#pragma unroll
+            for (int dd = 32; dd >= 1; dd >>= 1) m = fmn(m, __shfl_xor(m, dd, 64));
+            best = fmn(best, m);
+            const bool add = hit && t <= best * kReach;
+            const uint64_t am = __ballot(add);
+            if (am == 0ull) continue;
+            const int na = __popcll(am);
+            const uint64_t lt = (1ull << lane) - 1ull;
+            if (nc + na > kCands) {  // keep those still near the nearest
+                const float ct = L.t[lane], cu = L.u[lane], cv = L.v[lane], ce = L.e[lane];
+                const int cp = L.p[lane];
+                const bool keep = lane < nc && ct <= best * kReach;
+                const uint64_t km = __ballot(keep);
+                wave_fence();
+                if (keep) {
+                    const int i = __popcll(km & lt);
+                    L.t[i] = ct; L.u[i] = cu; L.v[i] = cv; L.e[i] = ce; L.p[i] = cp;
+                }
+                nc = __popcll(km);
+                wave_fence();
+            }
+            if (nc + na > kCands) {
+                failed = true;
+            } else {
+                if (add) {
+                    const int i = nc + __popcll(am & lt);
+                    L.t[i] = t; L.u[i] = u; L.v[i] = v; L.e[i] = e; L.p[i] = p;
+                }
+                nc += na;
+            }
+        }
+        const uint64_t im = __ballot(inner);
+        const int ni = __popcll(im);
+        if (count + ni > kPend) failed = true;
+        if (failed) break;
+        if (inner) L.pend[count + __popcll(im & ((1ull << lane) - 1ull))] = at;
+        count += ni;
+        wave_fence();
+    }
+    wave_fence();
+    if (__ballot(bad)) failed = true;
+    int win = -1;
+    if (!failed && nc > 0) {
+        // the hits whose order could matter: at or before the farthest of
+        // their own boxes' starts
+        const float ct = lane < nc ? L.t[lane] : FLT_MAX, ce = lane < nc ? L.e[lane] : 0.f;
+        float bound = best;
+        bool grew = true;
+        while (grew) {
+            float m = ct <= bound ? fmx(ct, ce) : 0.f;
+#pragma unroll
+            for (int dd = 32; dd >= 1; dd >>= 1) m = fmx(m, __shfl_xor(m, dd, 64));
+            grew = m > bound;
+            if (grew) bound = m;
+        }
+        const bool rival = ct <= bound;
+        const uint64_t rm = __ballot(rival);
+        if (bound > best * kOwnBox) {
+            failed = true;
+        } else if (__popcll(rm) == 1) {
+            win = __ffsll((long long)rm) - 1;
+        } else {
+            // Replay the reference's order among them, one lane each. A hit is
+            // skipped when its path, below the box that was pending before an
+            // earlier hit was met, starts at or beyond that hit.
+            const v3 inv = div3(mk3(1.f, 1.f, 1.f), d);
+            uint64_t path = ~0ull;
+            int depth = 0;
+            bool reach;
+            const bool ok = !rival || leaf_path(A.w, A.w.leaf_of[L.p[lane]], o, inv, path, depth, reach);
+            if (__ballot(!ok)) failed = true;
+            float near = FLT_MAX;
+            bool visited = false;
+            for (uint64_t left = rm; left != 0ull && !failed;) {
+                uint64_t first = (left >> lane) & 1ull ? path : ~0ull;
+#pragma unroll
+                for (int dd = 32; dd >= 1; dd >>= 1) {
+                    const uint64_t other = (uint64_t)__shfl_xor((unsigned long long)first, dd, 64);
+                    first = other < first ? other : first;
+                }
+                const uint64_t at = __ballot(((left >> lane) & 1ull) && path == first);
+                const int c = __ffsll((long long)at) - 1;
+                left &= ~(1ull << c);
+                const float ec = __shfl(ce, c, 64), tc = __shfl(ct, c, 64);
+                const int dc = __shfl(depth, c, 64);
+                const bool skips = visited && ec >= ct && dc > __clzll((long long)(path ^ first)) + 1;
+                if (__ballot(skips)) continue;
+                if (lane == c) visited = true;
+                if (tc < near) {
+                    near = tc;
+                    win = c;
+                }
+            }
+        }
+    }
+    if (lane == 0) {
+        int prim = -1;
+        float t = 0.f, u = 0.f, v = 0.f;
+        if (failed) {
+            uint32_t ovf = 0;
+            reference_closest(A.recs, A.root, o, d, 2 * A.ntris - 1, L.stack, prim, t, u, v, ovf);
+            if (ovf) atomicAdd(A.overflow, ovf);
+            atomicAdd(A.fails, 1u);
+        } else if (win >= 0) {
+            prim = L.p[win]; t = L.t[win]; u = L.u[win]; v = L.v[win];
+        }
+        oprim[ri] = prim;
+        ot[ri] = t;
+        if (ou) ou[ri] = u;
+        if (ov) ov[ri] = v;
+    }
+    wave_fence();
+}
+
+__device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const float* limit, const int32_t* src,
+                           const int32_t* dst, uint8_t* ovis, uint64_t& nfetch) {
+    const int lane = threadIdx.x;
+    v3 o, d;
+    load_ray(A.rays, ri, o, d);
+    WideRay r;
+    const RayKind kind = wide_ray(o, d, r);
+    bool failed = kind == kRayOdd;
+    const float lim = limit[ri];
+    const bool use = !(lim == INFINITY);
+    const float cut = use ? lim * kReach * r.scale : FLT_MAX;
+    const int sm = src ? src[ri] : -1, dm = dst ? dst[ri] : -1;
+    int count = kind != kRayFine || (use && !(lim > 0.f)) ? 0 : 1;
+    bool blocked = false, bad = false;
+    if (lane == 0) L.pend[0] = 0u;
+    wave_fence();
+    while (count > 0) {
+        const int k = count < 8 ? count : 8;
+        const int g = lane >> 3;
+        bool inner = false, hit = false;
+        uint32_t at = 0;
+        int nt = 0;
+        if (g < k) {
+            const uint32_t node = L.pend[count - 1 - g];
+            lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, cut, inner, at, nt);
+            nfetch += (lane & 7) == 0 ? 1u : 0u;
+        }
+        count -= k;
+        wave_fence();
+        for (int j = 0; j < nt && !hit; ++j) {
+            const float4* tp = A.w.tris + (int64_t)(at + (uint32_t)j) * 3;
+            const float4 a = tp[0], b = tp[1], c = tp[2];
+            ++nfetch;
+            const int mesh = __float_as_int(b.w);
+            float t, u, v;
+            if (mesh != sm && mesh != dm && wide_tri_hit(a, b, c, o, d, t, u, v) && (!use || t < lim)) {
+                bool touch;
+                hit = leaf_entry(a, b, c, o, d, touch) >= 0.f;
+                if (hit && touch) hit = reached(A.w, __float_as_int(a.w), o, d, bad);
+            }
+        }
+        if (__ballot(hit)) {
+            blocked = true;
+            break;
+        }
+        const uint64_t im = __ballot(inner);
+        const int ni = __popcll(im);
+        if (count + ni > kPend) {
+            failed = true;
+            break;
+        }
+        if (inner) L.pend[count + __popcll(im & ((1ull << lane) - 1ull))] = at;
+        count += ni;
+        wave_fence();
+    }
+    wave_fence();
+    if (!blocked && __ballot(bad)) failed = true;
+    if (lane == 0) {
+        if (failed) {
+            uint32_t ovf = 0;
+            blocked = reference_blocked(A.recs, o, d, lim, sm, dm, 2 * A.ntris - 1, L.stack, ovf);
+            if (ovf) atomicAdd(A.overflow, ovf);
+            atomicAdd(A.fails, 1u);
+        }
+        ovis[ri] = blocked ? 0 : 1;
+    }
+    wave_fence();
+}
+
+template <bool kAny>
+__global__ __launch_bounds__(64) void k_wide_finish(FinishArgs A, int32_t* oprim, float* ot, float* ou, float* ov,
+                                                    const float* limit, const int32_t* src, const int32_t* dst,
+                                                    uint8_t* ovis) {
+    __shared__ FinishLds L;
+    const uint32_t all = *A.n;
+    const uint32_t total = min(all, A.cap);
+    if (blockIdx.x >= total) return;
+    uint64_t nfetch = 0;
+    for (uint32_t i = blockIdx.x; i < total; i += gridDim.x) {
+        if (kAny) finish_any(A, A.ids[i], L, limit, src, dst, ovis, nfetch);
+        else finish_closest(A, A.ids[i], L, oprim, ot, ou, ov, nfetch);
+    }
+    if (all > A.cap) {  // the list ran over: find the marked rays
+        const int64_t nrays = A.nrays_dev ? (int64_t)*A.nrays_dev : A.nrays;
+        for (int64_t b = (int64_t)blockIdx.x * 64; b < nrays; b += (int64_t)gridDim.x * 64) {
+            const int64_t i = b + threadIdx.x;
+            uint64_t m = __ballot(i < nrays && (kAny ? ovis[i] == 255 : oprim[i] == kUndecided));
+            for (; m; m &= m - 1ull) {
+                const int64_t ri = b + __ffsll((long long)m) - 1;
+                if (kAny) finish_any(A, ri, L, limit, src, dst, ovis, nfetch);
+                else finish_closest(A, ri, L, oprim, ot, ou, ov, nfetch);
+            }
+        }
+    }
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) nfetch += __shfl_xor(nfetch, dd, 64);
+    if (threadIdx.x == 0 && nfetch > 0) atomicAdd(A.fetched, (unsigned long long)nfetch);
+}
+
+constexpr int kFinishBlocks = 4096;
+
+template <bool kAny, int B, typename... A>
+void launch_wide(const TraceLaunch& L, int64_t nrays, LaunchSink& ls, A... args) {
+    static const int per_cu = [] {
+        int per = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(&k_wide_trace<kAny, B>), B,
+                                                         0) != hipSuccess || per <= 0)
+            per = 4 * 256 / B;
+        return per;
+    }();
+    // the tree's nodes stay in the caches, so as many waves as fit: the
+    // launch shape's workgroups per CU bound the reference's traversals only
+    const int64_t need = (nrays + B - 1) / B;
+    int64_t blocks = std::min<int64_t>((int64_t)device_cus() * per_cu, need);
+    if (blocks < 1) blocks = 1;
+    ls.launch(kAny ? "k_wide_trace<any>" : "k_wide_trace<closest>", &k_wide_trace<kAny, B>, dim3((unsigned)blocks),
+              dim3(B), args..., L.chunk);
+}
+template <bool kAny, typename... A>
+void launch_wide_block(const TraceLaunch& L, int64_t nrays, LaunchSink& ls, A... args) {
+    if (L.block == 64) launch_wide<kAny, 64>(L, nrays, ls, args...);
+    else if (L.block == 128) launch_wide<kAny, 128>(L, nrays, ls, args...);
+    else launch_wide<kAny, 256>(L, nrays, ls, args...);
+}
+
+}  // namespace
+
+// Words 26 (rays listed) and 30 (rays that took the reference's traversal) of
+// the counters; the list is the cooperative pass's.
+void wide_closest(const TraceBvh& bvh, const float* rays, int64_t nrays, const uint32_t* nrays_dev, int32_t* prim,
+                  float* t, float* u, float* v, uint32_t* counters, const TraceLaunch& L, const TraceCoop& coop,
+                  LaunchSink& ls) {
+    const WideList wl{coop.longs, counters + 26, coop.long_cap, L.handoff};
+    launch_wide_block<false>(L, nrays, ls, bvh.wide.nodes, bvh.wide.tris, rays, nrays, nrays_dev, prim, t, u, v,
+                             (const float*)nullptr, (const int32_t*)nullptr, (const int32_t*)nullptr,
+                             (uint8_t*)nullptr, counters, reinterpret_cast<unsigned long long*>(counters + 2),
+                             fetch_word(counters, true), wl);
+    const FinishArgs A{bvh.wide, bvh.rec, bvh.root, rays, nrays, nrays_dev, coop.longs, counters + 26,
+                       coop.long_cap, counters + 30, counters, fetch_word(counters, true), bvh.ntris};
+    const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks, nrays);
+    ls.launch("k_wide_finish<closest>", &k_wide_finish<false>, dim3(blocks), dim3(64), A, prim, t, u, v,
+              (const float*)nullptr, (const int32_t*)nullptr, (const int32_t*)nullptr, (uint8_t*)nullptr);
+}
+
+// Words 20 and 22 likewise; the list is the failure list behind the spill records.
+void wide_occluded(const TraceBvh& bvh, const float* rays, int64_t nrays, const uint32_t* nrays_dev,
+                   const float* limit, const int32_t* src, const int32_t* dst, uint8_t* visible, uint32_t* counters,
+                   const TraceLaunch& L, const TraceCoop& coop, LaunchSink& ls) {
+    uint32_t* ids = reinterpret_cast<uint32_t*>(coop.spill + coop.spill_cap);
+    const WideList wl{ids, counters + 20, coop.spill_cap, L.handoff};
+    launch_wide_block<true>(L, nrays, ls, bvh.wide.nodes, bvh.wide.tris, rays, nrays, nrays_dev, (int32_t*)nullptr,
+                            (float*)nullptr, (float*)nullptr, (float*)nullptr, limit, src, dst, visible,
+                            counters + 1, reinterpret_cast<unsigned long long*>(counters + 4),
+                            fetch_word(counters, false), wl);
+    const FinishArgs A{bvh.wide, bvh.rec, bvh.root, rays, nrays, nrays_dev, ids, counters + 20,
+                       coop.spill_cap, counters + 22, counters + 1, fetch_word(counters, false), bvh.ntris};
+    const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks, nrays);
+    ls.launch("k_wide_finish<any>", &k_wide_finish<true>, dim3(blocks), dim3(64), A, (int32_t*)nullptr,
+              (float*)nullptr, (float*)nullptr, (float*)nullptr, limit, src, dst, visible);
+}
+
+}  // namespace cav

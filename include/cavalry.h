@@ -138,15 +138,16 @@ int cav_trace_occluded_async(cav_ctx* ctx, const cav_bvh* bvh, const float* rays
  * reference, which writes past its stack. */
 int cav_trace_counters(cav_ctx* ctx, const cav_bvh* bvh, uint32_t* out, int32_t reset);
 /* Work of a BVH's standalone launches (out holds 6 words): out[0] / out[1] =
- * 64-byte traversal records (node visits and triangle tests, one record
- * each) fetched by every closest-hit / any-hit launch since the last reset;
+ * traversal records (node visits and triangle tests, one record each: 80 and
+ * 48 bytes over the wide tree, 64 over the reference's) fetched by every
+ * closest-hit / any-hit launch since the last reset;
  * out[2] = rays of the last any-hit launch finished by a whole wave (long
- * rays still in flight once every ray was handed out), out[3] = those of
- * them the wave could not hold and one lane traced again from the root;
+ * rays still in flight once every ray was handed out, rays along a box plane),
+ * out[3] = those of them that one lane traced over the reference's tree;
  * out[4] = rays of the last closest-hit launch traced again by a whole wave
- * from the root, out[5] = those of them one lane traced once more in the
- * reference's order (two hits within a hair of each other, or a stack that
- * could overflow). reset != 0 clears out[0..1] after reading. No counterpart
+ * from the root (those, and rays with hits too close for their distances to
+ * decide), out[5] = those of them one lane traced once more in the
+ * reference's order. reset != 0 clears out[0..1] after reading. No counterpart
  * in the reference; it measures the algorithmic traffic of BVH::intersect /
  * testVisibility (BVH/BVH.h:23-189). */
 int cav_trace_fetches(cav_ctx* ctx, const cav_bvh* bvh, uint64_t* out, int32_t reset);
@@ -389,8 +390,13 @@ int cav_scene_create_from_pbrt(cav_ctx* ctx, const char* path, const cav_pbrt_ov
 
 /* ---------------------------------------------------------------- launch shapes */
 
-/* Launch shape of the persistent traversal kernels, per context: workgroups
- * per CU (0: as many as fit), rays a wave takes from the dispenser at a time
+/* Launch shape of the persistent traversal kernels, per context. Traces walk
+ * a wide tree built beside the reference's BVH, with the reference's answers;
+ * they walk the reference's own tree in its visiting order when the hand-off
+ * is 1<<30 (closest-hit, any-hit), any_hit_step is CAV_ANY_STEP_PAIR or
+ * any_hit_whole_line is 1 (any-hit), when that tree is more than 64 levels
+ * deep, a coordinate is beyond 2^40, or there was no memory for the wide tree.
+ * Workgroups per CU (0: as many as fit; reference's tree only), rays a wave takes from the dispenser at a time
  * (64..65536), traversal-stack entries kept in LDS (32 or 48; the rest of
  * the reference's 64 in scratch) and threads per traversal workgroup (64,
  * 128 or 256; 0: 256); for WAVEFRONT also the threads per workgroup of the

@@ -1,0 +1,158 @@
+"""Traces over the wide tree vs the CPU oracle, bit for bit, at the sizes where
+its build and its finishing pass can go wrong: trees of one node, of one
+level, across the single-workgroup limit; rays that run along box planes,
+coincident triangles, rays that hit nothing or come from very far, and more
+undecided rays than the finishing pass's list holds."""
+import numpy as np
+import pytest
+
+import oracle
+from cavalry_amd import BVH, scenes, tune
+from helpers import bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(bvh, nd, tris, rays, lim, what):
+    print(f"[wide] {what}: {len(tris)} triangles, {len(rays)} rays", flush=True)
+    ref = oracle.trace_closest(nd, tris, rays)
+    got = bvh.intersect(rays)
+    np.testing.assert_array_equal(got["prim"], ref["prim"])
+    for k in ("t", "u", "v"):
+        np.testing.assert_array_equal(bits(got[k]), bits(ref[k]), err_msg=k)
+    np.testing.assert_array_equal(bvh.test_visibility(rays, lim), oracle.trace_occluded(nd, tris, rays, lim))
+    return ref
+
+
+def _tree(ctx, tris, morton_bits, rounds):
+    _, _, nd = oracle.lbvh_build(tris, morton_bits)
+    if rounds:
+        oracle.treelet_optimize(nd, rounds)
+    return BVH.build(ctx, tris, optimization_rounds=rounds, morton_bits=morton_bits), nd
+
+
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 8, 9, 10, 31, 33, 257, 4096, 4097, 20000])
+def test_sizes(ctx, n):
+    rng = np.random.default_rng(n)
+    tris = scenes.gmm_triangles(n, seed=n, edge=0.05 if n > 300 else 0.3)
+    bvh, nd = _tree(ctx, tris, 30, 1 if n % 2 else 0)
+    rays = scenes.random_rays(3000, seed=n + 1, lo=0.0, hi=1.0)
+    lim = rng.uniform(0, 2, len(rays)).astype(np.float32)
+    lim[::5] = np.inf
+    _check(bvh, nd, tris, rays, lim, f"n={n}")
+
+
+def _plane_rays(tris, n, seed):
+    """Rays from points of the triangles (half exactly on them), most with one
+    or two zero direction components of either sign."""
+    rng = np.random.default_rng(seed)
+    t = tris[rng.integers(0, len(tris), n)].reshape(n, 3, 3)
+    b = rng.random((n, 2))
+    s = np.sqrt(b[:, :1])
+    p = (t[:, 0] * (1 - s) + t[:, 1] * (s * (1 - b[:, 1:])) + t[:, 2] * (s * b[:, 1:])).astype(np.float32)
+    corner = rng.random(n) < 0.2
+    p[corner] = t[corner, 1]
+    d = rng.normal(size=(n, 3)).astype(np.float32)
+    for share in (0.8, 0.2):
+        k = np.nonzero(rng.random(n) < share)[0]
+        d[k, rng.integers(0, 3, len(k))] = np.where(rng.random(len(k)) < 0.5, 0.0, -0.0)
+    len_ = np.linalg.norm(d, axis=1, keepdims=True)
+    d = np.where(len_ > 0, d / np.maximum(len_, 1e-20), d).astype(np.float32)
+    o = np.where(rng.random((n, 1)) < 0.5, p, p + np.float32(1e-3) * d).astype(np.float32)
+    return np.ascontiguousarray(np.concatenate([o, d], 1), np.float32)
+
+
+@pytest.mark.parametrize("morton_bits,rounds", [(30, 0), (63, 3)])
+def test_rays_along_planes_and_coincident_triangles(ctx, morton_bits, rounds):
+    """The Cornell box (boxes standing on the floor, walls on the scene's own
+    box planes) with some of its triangles doubled, one of them 70 times: rays
+    along box planes, where the slab test meets 0 * inf, and equally near hits."""
+    base = np.ascontiguousarray(scenes.cornell_box(seed=5).tris, np.float32)
+    rng = np.random.default_rng(7)
+    tris = np.concatenate([base, base[:40], base[rng.integers(0, len(base), 300)], np.repeat(base[2:3], 70, 0)])
+    bvh, nd = _tree(ctx, tris, morton_bits, rounds)
+    rays = _plane_rays(np.concatenate([base[:44], base[:44], tris[::37]]), 120000, 3)
+    lim = rng.uniform(0, 2, len(rays)).astype(np.float32)
+    lim[::5] = np.inf
+    ref = _check(bvh, nd, tris, rays, lim, "planes")
+    assert (ref["prim"] >= 0).sum() > 10000
+    f = bvh.trace_fetches()
+    assert f["long_closest_rays"] > 1000  # the finishing pass decided them
+
+
+def test_odd_rays(ctx):
+    """Rays outside what the wide tree's planes take: no direction, NaN,
+    directions from 1e-38 to 1e30 long, origins beyond 2^40."""
+    tris = scenes.gmm_triangles(3000, seed=3, edge=0.1)
+    bvh, nd = _tree(ctx, tris, 30, 0)
+    rays = scenes.random_rays(4000, seed=4, lo=0.0, hi=1.0)
+    scale = np.float32([1e-30, 1e-20, 1e-6, 1e6, 1e20, 1e30])
+    rays[:3000, 3:] *= scale[np.arange(3000) % 6][:, None]
+    rays[3000:3100, 3:] = 0.0
+    rays[3100:3200, 3] = np.nan
+    rays[3200:3300, 0] = np.nan
+    rays[3300:3400, 3:] *= np.float32(1e-38)
+    rays[3400:3500, :3] -= rays[3400:3500, 3:] * np.float32(4e12)
+    lim = np.full(len(rays), np.inf, np.float32)
+    lim[::3] = 1.0
+    lim[1::50] = np.nan
+    _check(bvh, nd, tris, rays, lim, "odd")
+
+
+def test_scene_far_from_the_origin_and_given_bounds(ctx):
+    """Coordinates around 1e5 with small triangles, with scene bounds given
+    that do not hold the triangles (the wide tree uses their own box)."""
+    tris = (scenes.gmm_triangles(5000, seed=8, edge=0.05) + np.float32(1e5)).astype(np.float32)
+    rays = scenes.random_rays(20000, seed=9, lo=0.0, hi=1.0)
+    rays[:, :3] += np.float32(1e5)
+    lim = np.full(len(rays), np.inf, np.float32)
+    sb = np.float32([1e5 + 0.4] * 3 + [1e5 + 0.6] * 3)
+    _, _, nd = oracle.lbvh_build(tris, 30, sb)
+    bvh = BVH.build(ctx, tris, scene_bounds=sb)
+    _check(bvh, nd, tris, rays, lim, "far")
+
+
+def test_more_undecided_rays_than_the_list_holds(ctx):
+    """Every triangle twice: every hit is undecided. 2^20 + 4099 rays, one list
+    of 2^20; the rest are found by scanning. Compared with the reference's
+    order on one lane per ray."""
+    half = scenes.gmm_triangles(500, seed=11, edge=0.3)
+    tris = np.ascontiguousarray(np.concatenate([half, half]), np.float32)
+    n = (1 << 20) + 4099
+    rays = scenes.random_rays(n, seed=12, lo=0.3, hi=0.7)
+    bvh = BVH.build(ctx, tris)
+    got = bvh.intersect(rays)
+    f = bvh.trace_fetches()
+    saved = tune.get_launch(ctx, tune.STANDALONE)
+    try:
+        tune.set_launch(ctx, tune.STANDALONE, dict(saved, handoff_steps=1 << 30))
+        ref = bvh.intersect(rays)
+    finally:
+        tune.set_launch(ctx, tune.STANDALONE, saved)
+    print(f"[wide] undecided: {f}", flush=True)
+    assert (ref["prim"] >= 0).mean() > 0.9
+    np.testing.assert_array_equal(got["prim"], ref["prim"])
+    for k in ("t", "u", "v"):
+        np.testing.assert_array_equal(bits(got[k]), bits(ref[k]), err_msg=k)
+
+
+def test_rebuild_reuses_the_tree(ctx):
+    """Rebuilds of one BVH object over other triangles, with and without
+    rounds, leave no trace of the earlier tree."""
+    import torch
+    n = 30000
+    bvh = None
+    for k, rounds in enumerate((0, 3, 0)):
+        tris = scenes.gmm_triangles(n, seed=40 + k, edge=0.01)
+        dev = torch.from_numpy(tris).cuda()
+        torch.cuda.synchronize()
+        if bvh is None:
+            bvh = BVH.build(ctx, dev, optimization_rounds=rounds, device=True)
+        else:
+            bvh.rebuild(dev, optimization_rounds=rounds)
+        _, _, nd = oracle.lbvh_build(tris, 30)
+        if rounds:
+            oracle.treelet_optimize(nd, rounds)
+        rays = scenes.random_rays(20000, seed=50 + k, lo=0.0, hi=1.0)
+        lim = scenes.shadow_limits(len(rays), seed=60 + k)
+        _check(bvh, nd, tris, rays, lim, f"rebuild {k}")
