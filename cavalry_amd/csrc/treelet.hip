@@ -158,7 +158,7 @@ __device__ __forceinline__ int part6(int lane, int e) {
 // node's height and is kept valid, so no round climbs the tree for it.
 // 4M triangles, one round: 3.7 -> 3.3 ms in the wide levels, 0.49 -> 0.29 in
 // the single-workgroup tail, 0.35 ms of climbing between rounds gone.
-__device__ void optimize_treelet(int root, NodeBox* nbox, int4* topo, uint32_t* hw, GroupLds& L) {
+__device__ __forceinline__ void optimize_treelet(int root, NodeBox* nbox, int4* topo, uint32_t* hw, GroupLds& L) {
     const int lane = threadIdx.x & 31;
     const int half = threadIdx.x & 32;
     LaneNode me;
