@@ -9,10 +9,12 @@
 // over that tree fetched thousands of records (bounce rays over a 1M-triangle
 // interior: 7500 each). What a trace returns does not depend on the tree
 // except through the order of equally near hits (wide_trace.hip), so the
-// traces walk this tree instead: the whole scene box spans the codes, and
-// triangles much larger than the typical one sort into trees of their own
-// (two class bits above the 30 code bits), so that a floor does not inflate
-// every box around it.
+// traces walk this tree instead, whose codes span the whole scene box.
+// Tried and dropped, in records fetched per ray on interiors of 1M triangles
+// (camera / bounce / shadow) and soups of 4M: cubic cells 26 / 64 / 32 and 90
+// against 21 / 59 / 23 and 59 here, 42-bit codes 23 / 62 / 34 and 90 (with the
+// classes that follow), triangles 8 (32) times larger than the typical one in
+// trees of their own 23 / 63 / 36 and 90 (19 / 60 / 30 and 63).
 #include "dev_common.h"
 #include "lbvh.h"
 #include "wide.h"
@@ -21,7 +23,7 @@ namespace cav {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kCodeBits = 32;
+constexpr int kCodeBits = 30;
 constexpr int kCtrTris = 80, kCtrTop = 81;  // words past the level counts
 constexpr int kMaxWideLevels = 78;
 
@@ -54,20 +56,14 @@ __global__ __launch_bounds__(kBlock) void k_wide_codes(const float* __restrict__
     const v3 shi = mk3(ord2f(ob[3]), ord2f(ob[4]), ord2f(ob[5]));
     const v3 se = sub3(shi, slo);
     const v3 inv = mk3(1.f / fmx(se.x, 1e-30f), 1.f / fmx(se.y, 1e-30f), 1.f / fmx(se.z, 1e-30f));
-    // class k: larger than 8^k times the typical triangle, taken as the
-    // scene's extent over sqrt(n) (a surface of n triangles)
-    const float big = 8.f * fmx(se.x, fmx(se.y, se.z)) / sqrtf((float)n);
     for (int64_t i = first; i < n; i += stride) {
         const float* p = tris + i * 9;
         const v3 a = mk3(p[0], p[1], p[2]), b = mk3(p[3], p[4], p[5]), c = mk3(p[6], p[7], p[8]);
         const v3 lo = mk3(fmn(a.x, fmn(b.x, c.x)), fmn(a.y, fmn(b.y, c.y)), fmn(a.z, fmn(b.z, c.z)));
         const v3 hi = mk3(fmx(a.x, fmx(b.x, c.x)), fmx(a.y, fmx(b.y, c.y)), fmx(a.z, fmx(b.z, c.z)));
-        const v3 e = sub3(hi, lo);
-        const float ext = fmx(e.x, fmx(e.y, e.z));
-        const uint32_t cls = ext > big ? (ext > 8.f * big ? (ext > 64.f * big ? 3u : 2u) : 1u) : 0u;
         const v3 m = sub3(scale3(add3(lo, hi), 0.5f), slo);
-        const uint32_t key = (cls << 30) | (spread10(cell10(m.x * inv.x)) << 2) |
-                             (spread10(cell10(m.y * inv.y)) << 1) | spread10(cell10(m.z * inv.z));
+        const uint32_t key = (spread10(cell10(m.x * inv.x)) << 2) | (spread10(cell10(m.y * inv.y)) << 1) |
+                             spread10(cell10(m.z * inv.z));
         keys[i] = key;
         vals[i] = (uint32_t)i;
 #pragma unroll
@@ -170,32 +166,32 @@ __device__ void wide_collapse(const WideBuild& w, uint32_t idx, bool valid, uint
     const bool inner = have && cnt > kWideLeaf;
     const bool leaf = have && !inner;
 
-    // slots: eight rounds of the best remaining (child, free slot) pair
+    // slots: every child asks for the best free one; where several ask for
+    // the same, the best fit has it and the others ask again
     int slot = 0;
     {
         const float cx = (ba.x + bb.x) - (nb.a.x + nb.b.x), cy = (ba.y + bb.y) - (nb.a.y + nb.b.y),
                     cz = (ba.z + bb.z) - (nb.a.z + nb.b.z);
-        float val[8];
-#pragma unroll
-        for (int s = 0; s < 8; ++s) val[s] = (s & 1 ? cx : -cx) + (s & 2 ? cy : -cy) + (s & 4 ? cz : -cz);
         uint32_t free_slots = 0xffu;
         bool todo = have;
-#pragma unroll 1
-        for (int k = 0; k < 8; ++k) {
-            if (__ballot(todo) == 0ull) break;
+        while (__ballot(todo)) {
             float bv = -INFINITY;
             int bs = __ffs((int)free_slots) - 1;
 #pragma unroll
-            for (int s = 0; s < 8; ++s)
-                if (((free_slots >> s) & 1u) && val[s] > bv) { bv = val[s]; bs = s; }
-            const uint32_t key = todo ? ((f2ord(bv) & ~7u) | (uint32_t)(7 - sl) | 8u) : 0u;
-            const uint32_t best = group_max(key);
-            const int src = (lane & 56) | (7 - (int)(best & 7u));
-            const int took = __shfl(bs, src, 64);
-            if (best != 0u) {
-                free_slots &= ~(1u << took);
-                if (lane == src) { slot = took; todo = false; }
+            for (int s = 0; s < 8; ++s) {
+                const float v = (s & 1 ? cx : -cx) + (s & 2 ? cy : -cy) + (s & 4 ? cz : -cz);
+                if (((free_slots >> s) & 1u) && v > bv) { bv = v; bs = s; }
             }
+            // wish: the fit in order, then the lane (so that none are equal), the slot in the low bits
+            const uint32_t wish = todo ? (f2ord(bv) & ~127u) | (uint32_t)(8 | sl) << 3 | (uint32_t)bs : 0u;
+            bool mine = todo;
+#pragma unroll
+            for (int d = 1; d < 8; ++d) {
+                const uint32_t o = (uint32_t)__shfl_xor((int)wish, d, 64);
+                mine = mine && !(o > wish && (o & 7u) == (uint32_t)bs);
+            }
+            if (mine) { slot = bs; todo = false; }
+            free_slots &= ~group_or(mine ? 1u << bs : 0u);
         }
     }
 
@@ -373,7 +369,7 @@ hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, const float* tris, const i
     int nb = (n + kBlock - 1) / kBlock;
     if (nb > kCodeBlocks) nb = kCodeBlocks;
     hipLaunchKernelGGL(k_wide_init, dim3(1), dim3(1024), 0, s, b.hist, kSortHistWords + 16, w.ctr, w.nodes, n);
-    hipLaunchKernelGGL(k_wide_codes, dim3(nb), dim3(kBlock), 0, s, tris, (int64_t)n, bounds, w.keys[0], w.vals[0],
+    hipLaunchKernelGGL(k_wide_codes, dim3(nb), dim3(kBlock), 0, s, tris, (int64_t)n, bounds, ob.keys[0], w.vals[0],
                        b.hist, b.counts, 4 * 256 * tiles);
     mark(mk, "wide_codes");
     hipError_t e = onesweep_sort_pairs(ob, n, kCodeBits, s, nullptr);
@@ -391,7 +387,7 @@ hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, const float* tris, const i
     const bool small = n <= 4096;
     hipLaunchKernelGGL(k_wide_levels, dim3(1), dim3(1024), 0, s, wb, 0, small ? 0xffffffffu : 512u);
     if (!small) {
-        int levels = 2;
+        int levels = 6;  // (an empty one costs 3 us; a skewed tree left to one workgroup cost 1.2 ms)
         for (int64_t left = (int64_t)n / 512; left > 0; left /= 8) ++levels;
         int64_t blocks = (wide_node_capacity(n) + kBlock / 8 - 1) / (kBlock / 8);
         if (blocks > 2048) blocks = 2048;
