@@ -157,3 +157,27 @@ def test_rlpath_deterministic_after_buffers_grow(ctx):
     again, _ = R.render(ctx, scene, 2, integrator="rlpath", max_depth=4, deterministic=True)
     np.testing.assert_array_equal(again.rgb, first.rgb)
     scene.close()
+
+
+@pytest.mark.parametrize("nlights", [15, 16, 17, 64, 69])
+def test_rlpath_light_counts(ctx, nlights):
+    """The light statistics are finished a thread per entry below 16 lights and
+    a wave per entry from there, 64 lights at a time: the deterministic film
+    equals the oracle's bit for bit on both sides of each limit. (The scene's
+    mirrors, glass and plastic take the bin masks of the Q distribution.)"""
+    print(f"[rlpath] {nlights} lights", flush=True)
+    sc = scenes.interior(0, seed=3, width=40, height=32, textures=False)
+    lights = np.flatnonzero(sc.meshes["is_light"])
+    assert len(lights) == 64
+    sc.meshes["is_light"][lights[nlights:]] = 0
+    sc.meshes["is_light"][:max(0, nlights - 64)] = 1  # (walls, above 64)
+    sc.meshes["emission"][:max(0, nlights - 64)] = 1.5
+    sc.meshes["emission"][sc.meshes["is_light"] == 0] = 0
+    cam = for_scene(sc)
+    rgb, w, rays = oracle.render_rlpath(sc, 4, cam, max_depth=6)
+    scene = R.Scene(ctx, sc)
+    film, st = R.render(ctx, scene, 4, integrator="rlpath", camera=cam, max_depth=6, deterministic=True)
+    np.testing.assert_array_equal(film.weight, w)
+    np.testing.assert_array_equal(film.rgb.view(np.uint32), rgb.view(np.uint32))
+    assert st["closest_rays"] + st["shadow_rays"] == rays
+    scene.close()
