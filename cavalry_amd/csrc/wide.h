@@ -11,17 +11,20 @@
 namespace cav {
 
 // One node, 128 bytes (one L2 line), eight 16-byte words:
-//   0: box origin xyz | scale exponents x, y, z (biased, one byte each) and
-//      the mask of slots holding an inner child
+//   0: box origin xyz | scale exponents x, y, z (one byte each, biased by 127
+//      and by kPlaneBits more) and the mask of slots holding an inner child
 //   1: first inner child's node | first triangle | 8 slot bytes (WideSlot)
-//   2, 3, 4: x, y, z: 8 low planes, 8 high planes, in units of 2^exponent
-//      from the origin, rounded outwards
+//   2, 3, 4: x, y, z: planes in units of 2^exponent from the origin, rounded
+//      outwards; two slots to a word: low, low, high, high
 //   5: build only: {binary node, first leaf, last leaf, 0}
 // Inner children lie one after the other in slot order, and so do the
 // triangles of the leaf slots.
 // A slot's byte: 0 empty; inner 1 << 5 | (24 + slot); leaf of c triangles
 // ((1 << c) - 1) << 5 | offset from the first triangle.
 constexpr int kWideWords = 8;
+constexpr int kPlaneBits = 24;  // a plane's byte as the bits of a half float is 2^-24 times its number
+// byte of a slot's low plane of axis k (its high plane: two bytes on)
+__host__ __device__ constexpr int wide_plane(int k, int slot) { return 32 + 16 * k + (slot >> 1) * 4 + (slot & 1); }
 constexpr int kWideLeaf = 3;  // triangles per leaf slot at most
 // nodes for n triangles: a node with inner children has all 8 slots filled,
 // one without holds at least 4 triangles (or is the root)

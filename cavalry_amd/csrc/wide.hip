@@ -225,8 +225,8 @@ __device__ void wide_collapse(const WideBuild& w, uint32_t idx, bool valid, uint
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         uint32_t e = (__float_as_uint(fmx(ext[k], 0.f) * (1.0001f / 254.f)) >> 23) + 1u;
-        e = e < 40u ? 40u : (e > 250u ? 250u : e);
-        ex[k] = e;
+        e = e < 40u ? 40u : (e > 230u ? 230u : e);  // (coordinates up to 2^40 are traced: 161 at most)
+        ex[k] = e + kPlaneBits;
         isc[k] = __uint_as_float((254u - e) << 23);
     }
     uint8_t* mine = reinterpret_cast<uint8_t*>(stage + g * 5);
@@ -239,8 +239,8 @@ __device__ void wide_collapse(const WideBuild& w, uint32_t idx, bool valid, uint
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const float ql = floorf((lo[k] - org[k]) * isc[k] - 1e-4f), qh = ceilf((hi[k] - org[k]) * isc[k] + 1e-4f);
-            mine[32 + 16 * k + slot] = (uint8_t)(int)fmn(fmx(ql, 0.f), 255.f);
-            mine[40 + 16 * k + slot] = (uint8_t)(int)fmn(fmx(qh, 0.f), 255.f);
+            mine[wide_plane(k, slot)] = (uint8_t)(int)fmn(fmx(ql, 0.f), 255.f);
+            mine[wide_plane(k, slot) + 2] = (uint8_t)(int)fmn(fmx(qh, 0.f), 255.f);
         }
         const uint32_t below = counts & ((1u << (2 * slot)) - 1u);
         mine[24 + slot] = inner ? (uint8_t)((1u << 5) | (24u + (uint32_t)slot))

@@ -22,7 +22,11 @@
 // before max(t_M, e_M). A ray that met another hit X with t_X <= max(t_M,
 // e_M) -- coincident surfaces, a box standing on a floor -- goes to
 // k_wide_finish, which collects all hits that close and replays the
-// reference's order among them from the reference's tree.
+// reference's order among them from the reference's tree. The trace keeps the
+// nearest triangle hit and the second's distance and looks at the nearest's
+// own box at the end; where that hit turns out to be no candidate, or a
+// grazing one, the finishing pass decides too (an any-hit ray likewise, by
+// the first triangle hit that blocks it).
 //
 // The wide boxes only have to contain the exact ones. They are rounded
 // outwards, their planes' distances carry a slack of 2^-20 of their terms
@@ -33,10 +37,19 @@
 // assumption, with a margin 16 times wider, that the cooperative passes over
 // the reference's tree make (traverse.hip).
 //
-// Per node and lane: five 16-byte loads from one line and about 230 VALU
+// Per node and lane: five 16-byte loads from one line and about 190 VALU
 // instructions for eight children, against four loads and 90 instructions
 // for the two children of a reference node; a stack entry holds all of a
-// node's remaining children.
+// node's remaining children. The instructions are what bounds the traces
+// (bounce rays: 92% of the issue slots, half of the lanes at work). Planes
+// read as half floats instead of converted bytes, and the nearest hit's own
+// box tested once when the ray is through instead of at every hit (an
+// iteration of 64 rays met some hit three times in four): 2M camera rays 0.56
+// to 0.50 ms, 1M bounce rays 0.97 to 0.89,
+// 2M shadow rays 0.84 to 0.79.
+// Tried and dropped: a second set of pending triangles per lane, tested once
+// 20 to 40 lanes have some (bounce rays 1.34 to 1.52 ms: lanes wait), and all
+// triangles of an iteration before its next node (0.90 to 0.92).
 #include <algorithm>
 #include <cfloat>
 
@@ -62,6 +75,10 @@ constexpr int kWideDeep = 68;                   // entries in all: more than a t
 constexpr int kRefill = 12;
 constexpr int kUndecided = -2;                  // hit id of a ray that the finishing pass still has to find by scanning
 
+// selector of the near planes of an axis (a byte, a zero, a byte, a zero); the far ones' is ^ kFarPlanes
+__device__ __forceinline__ uint32_t near_planes(float inv) { return inv < 0.f ? 0x0c030c02u : 0x0c010c00u; }
+constexpr uint32_t kFarPlanes = 0x00020002u;
+
 // The ray as the node tests use it: direction scaled to a largest component
 // in [1, 2) (a power of two, exact), reciprocals bounded by 2^60 so that an
 // axis the ray runs along gives huge distances instead of infinities.
@@ -69,6 +86,7 @@ struct WideRay {
     v3 o, inv;
     float scale;  // true t * scale = t in the scaled direction
     uint32_t oct;
+    uint32_t nx, ny, nz;  // selectors of the near planes (near_planes)
 };
 __device__ __forceinline__ float wide_rcp(float d) {
     const float r = __builtin_amdgcn_rcpf(d);
@@ -91,6 +109,7 @@ __device__ __forceinline__ RayKind wide_ray(v3 o, v3 d, WideRay& r) {
     r.scale = __uint_as_float(e << 23);
     const float down = __uint_as_float((254u - e) << 23);
     r.inv = mk3(wide_rcp(d.x * down), wide_rcp(d.y * down), wide_rcp(d.z * down));
+    r.nx = near_planes(r.inv.x); r.ny = near_planes(r.inv.y); r.nz = near_planes(r.inv.z);
     r.oct = (r.inv.x < 0.f ? 1u : 0u) | (r.inv.y < 0.f ? 2u : 0u) | (r.inv.z < 0.f ? 4u : 0u);
     return dead ? kRayDead : (fine ? kRayFine : kRayOdd);
 }
@@ -102,7 +121,7 @@ __device__ __forceinline__ uint32_t order_slots(uint32_t meta, uint32_t oct4) {
     return meta ^ (oct4 & ((inner >> 1) - (inner >> 4)));  // 7 in the low bits of the inner ones' bytes
 }
 
-// One axis of one node: plane distances are q * a + b.
+// One axis of one node: plane distances are (the byte's half float) * a + b.
 struct AxisPlanes {
     float an, af, bn, bf;
 };
@@ -115,8 +134,15 @@ __device__ __forceinline__ AxisPlanes axis_planes(float p, uint32_t e, float o, 
     r.bf = __builtin_fmaf(kSlack, fabsf(b), b);
     return r;
 }
-__device__ __forceinline__ float ubyte(uint32_t w, int k) { return (float)((w >> (8 * k)) & 255u); }
 
+// The planes of two slots as two half floats, near or far ones by the
+// selector: one byte permutation in place of two conversions and half a
+// select, and the fused multiply-add takes halves as they are (denormal ones
+// included: byte * 2^-24 exactly, as the exponents are kPlaneBits up).
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ half2v plane_pair(uint32_t word, uint32_t sel) {
+    return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(word, word, sel));
+}
 // Tests a node's children against the ray up to `cut` (scaled units): bits
 // 0..23 the triangles of hit leaf slots, 24..31 the hit inner children in
 // front-to-back order.
@@ -125,27 +151,31 @@ __device__ __forceinline__ uint32_t test_children(const uint4& w0, const uint4& 
     const AxisPlanes x = axis_planes(__uint_as_float(w0.x), w0.w & 255u, r.o.x, r.inv.x);
     const AxisPlanes y = axis_planes(__uint_as_float(w0.y), (w0.w >> 8) & 255u, r.o.y, r.inv.y);
     const AxisPlanes z = axis_planes(__uint_as_float(w0.z), (w0.w >> 16) & 255u, r.o.z, r.inv.z);
-    const bool nx = r.inv.x < 0.f, ny = r.inv.y < 0.f, nz = r.inv.z < 0.f;
+    const uint32_t fx = r.nx ^ kFarPlanes, fy = r.ny ^ kFarPlanes, fz = r.nz ^ kFarPlanes;
     const uint32_t oct4 = r.oct * 0x01010101u;
+    const uint32_t px[4] = {w2.x, w2.y, w2.z, w2.w}, py[4] = {w3.x, w3.y, w3.z, w3.w}, pz[4] = {w4.x, w4.y, w4.z, w4.w};
     uint32_t mask = 0;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
-        const uint32_t lx = half ? w2.y : w2.x, hx = half ? w2.w : w2.z;
-        const uint32_t ly = half ? w3.y : w3.x, hy = half ? w3.w : w3.z;
-        const uint32_t lz = half ? w4.y : w4.x, hz = half ? w4.w : w4.z;
-        const uint32_t xn = nx ? hx : lx, xf = nx ? lx : hx;
-        const uint32_t yn = ny ? hy : ly, yf = ny ? ly : hy;
-        const uint32_t zn = nz ? hz : lz, zf = nz ? lz : hz;
         const uint32_t meta = order_slots(half ? w1.w : w1.z, oct4);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float tn = fmx(fmx(__builtin_fmaf(ubyte(xn, k), x.an, x.bn), __builtin_fmaf(ubyte(yn, k), y.an, y.bn)),
-                                 fmx(__builtin_fmaf(ubyte(zn, k), z.an, z.bn), 0.f));
-            const float tf = fmn(fmn(__builtin_fmaf(ubyte(xf, k), x.af, x.bf), __builtin_fmaf(ubyte(yf, k), y.af, y.bf)),
-                                 fmn(__builtin_fmaf(ubyte(zf, k), z.af, z.bf), cut));
-            const uint32_t m = meta >> (8 * k);
-            const uint32_t bits = ((m >> 5) & 7u) << (m & 31u);
-            mask |= tn <= tf ? bits : 0u;
+        for (int pair = 0; pair < 2; ++pair) {
+            const int w = 2 * half + pair;
+            const half2v xn = plane_pair(px[w], r.nx), xf = plane_pair(px[w], fx);
+            const half2v yn = plane_pair(py[w], r.ny), yf = plane_pair(py[w], fy);
+            const half2v zn = plane_pair(pz[w], r.nz), zf = plane_pair(pz[w], fz);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const float tn =
+                    fmx(fmx(__builtin_fmaf((float)xn[c], x.an, x.bn), __builtin_fmaf((float)yn[c], y.an, y.bn)),
+                        fmx(__builtin_fmaf((float)zn[c], z.an, z.bn), 0.f));
+                const float tf =
+                    fmn(fmn(__builtin_fmaf((float)xf[c], x.af, x.bf), __builtin_fmaf((float)yf[c], y.af, y.bf)),
+                        fmn(__builtin_fmaf((float)zf[c], z.af, z.bf), cut));
+                const uint32_t m = meta >> (8 * (2 * pair + c));
+                const uint32_t bits = ((m >> 5) & 7u) << (m & 31u);
+                mask |= tn <= tf ? bits : 0u;
+            }
         }
     }
     return mask;
@@ -266,52 +296,83 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
     WideRay r;
     r.o = r.inv = mk3(0, 0, 0);
     r.scale = 1.f;
-    r.oct = 0;
+    r.oct = r.nx = r.ny = r.nz = 0;
     v3 d = mk3(0, 0, 0);
-    float best = FLT_MAX, own = 0.f, bu = 0.f, bv = 0.f, cut = 0.f;  // own: where the nearest hit's box starts
-    int bp = -1, sm = -1, dm = -1, steps = 0;
-    bool unsure = false, grazed = false, may_list = false, drained = false;
+    float best = FLT_MAX, rival = FLT_MAX, bu = 0.f, bv = 0.f, cut = 0.f;  // rival: the second nearest hit
+    int bt = -1, sm = -1, dm = -1, steps = 0;  // bt: the nearest hit's triangle record
+    bool odd = false, over = false, may_list = false, drained = false;  // over: traversed, result still to be written
     uint32_t cbase = 0, group = 0;  // the current node's inner children: first one, slot mask << 8 | bits to visit
     uint32_t tbase = 0, tbits = 0;  // triangles to test
     int sp = 0, maxsp = 0;
     uint32_t deep[2 * (kWideDeep - kWideStack)];
-    uint64_t nfetch = 0;
+    uint32_t nfetch = 0;
     Dispenser disp(nrays, most);
 
     while (true) {
-        const uint64_t need = __ballot(ri == -1);
-        if (need && (__popcll(need) >= kRefill || !__ballot(ri >= 0))) {
-            const int64_t mine = disp.next(need, lane, next_ray);
-            if (ri == -1) {
-                ri = mine < nrays ? mine : -2;
-                if (ri >= 0) {
-                    v3 o;
-                    load_ray(rays, ri, o, d);
-                    const RayKind kind = wide_ray(o, d, r);
-                    best = FLT_MAX; own = 0.f; bp = -1; bu = 0.f; bv = 0.f;
-                    unsure = kind == kRayOdd;
-                    grazed = false;
-                    may_list = wl.after > 0;
-                    steps = 0; sp = 0; tbits = 0;
-                    cbase = 0;
-                    group = (1u << 8) | (1u << r.oct);  // the root, as slot 0 of a node of one child
-                    cut = FLT_MAX;
-                    if (kAny) {
-                        best = limit[ri];
-                        const bool use = !(best == INFINITY);
-                        if (use) cut = best * kReach * r.scale;
-                        if (use && !(best > 0.f)) group = 0;  // nothing lies before it
-                        sm = src ? src[ri] : -1;
-                        dm = dst ? dst[ri] : -1;
+        const uint64_t idle = __ballot(ri == -1 || over);
+        if (idle && (__popcll(idle) >= kRefill || !__ballot(ri >= 0 && !over))) {
+            if (over) {
+                bool ask = odd;  // the finishing pass has to decide
+                int prim = -1;
+                if (bt >= 0) {
+                    const float4* tp = tris + (int64_t)bt * 3;
+                    const float4 a = tp[0], b = tp[1], c = tp[2];
+                    prim = __float_as_int(a.w);
+                    bool touch;
+                    const float e = leaf_entry(a, b, c, r.o, d, touch);
+                    ask = ask || touch || !(e >= 0.f);
+                    if (!kAny) ask = ask || rival <= fmx(best, e) || e > best * kOwnBox;
+                }
+                if (kAny) {
+                    ovis[ri] = prim >= 0 ? 0 : 1;
+                } else {
+                    oprim[ri] = prim;
+                    ot[ri] = prim >= 0 ? best : 0.f;
+                    if (ou) ou[ri] = bu;
+                    if (ov) ov[ri] = bv;
+                }
+                if (ask) {
+                    const uint32_t slot = atomicAdd(wl.n, 1u);
+                    if (slot < wl.cap) wl.ids[slot] = (uint32_t)ri;
+                    else if (kAny) ovis[ri] = 255;
+                    else oprim[ri] = kUndecided;
+                }
+                over = false;
+                ri = -1;
+            }
+            const uint64_t need = __ballot(ri == -1);
+            if (need) {
+                const int64_t mine = disp.next(need, lane, next_ray);
+                if (ri == -1) {
+                    ri = mine < nrays ? mine : -2;
+                    if (ri >= 0) {
+                        v3 o;
+                        load_ray(rays, ri, o, d);
+                        const RayKind kind = wide_ray(o, d, r);
+                        best = rival = FLT_MAX; bt = -1; bu = 0.f; bv = 0.f;
+                        odd = kind == kRayOdd;
+                        may_list = wl.after > 0;
+                        steps = 0; sp = 0; tbits = 0;
+                        cbase = 0;
+                        group = (1u << 8) | (1u << r.oct);  // the root, as slot 0 of a node of one child
+                        cut = FLT_MAX;
+                        if (kAny) {
+                            best = limit[ri];
+                            const bool use = !(best == INFINITY);
+                            if (use) cut = best * kReach * r.scale;
+                            if (use && !(best > 0.f)) group = 0;  // nothing lies before it
+                            sm = src ? src[ri] : -1;
+                            dm = dst ? dst[ri] : -1;
+                        }
+                        if (kind != kRayFine) group = 0;
                     }
-                    if (kind != kRayFine) group = 0;
                 }
             }
         }
         if (!__ballot(ri >= 0)) break;  // every lane is out of rays
-        if (ri < 0) continue;
+        if (ri < 0 || over) continue;
 
-        bool done = false, listed = false, hit = false;
+        bool done = false, listed = false;
         if (may_list && steps >= wl.after) {
             if (!drained && ((steps - wl.after) & 255) == 0)
                 drained = disp.drained(next_ray, nrays);
@@ -378,59 +439,30 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                 const int mesh = __float_as_int(b.w);
                 if (mesh != sm && mesh != dm && wide_tri_hit(a, b, c, r.o, d, t, u, v) &&
                     (best == INFINITY || t < best)) {
-                    bool touch;
-                    const bool in = leaf_entry(a, b, c, r.o, d, touch) >= 0.f;
-                    if (in && touch) unsure = true;
-                    else if (in) done = hit = true;
+                    bt = (int)(tbase + k);
+                    done = true;
                 }
-            } else if (wide_tri_hit(a, b, c, r.o, d, t, u, v) && t <= fmx(best, own)) {
-                bool touch;
-                const float e = leaf_entry(a, b, c, r.o, d, touch);
-                if (e >= 0.f) {
-                    if (touch) {
-                        grazed = true;
-                    } else if (t < best) {
-                        // the earlier nearest hit is this one's only possible rival so far
-                        unsure = best <= fmx(t, e) || e > t * kOwnBox;
-                        best = t; own = e; bu = u; bv = v; bp = __float_as_int(a.w);
-                        cut = t * kReach * r.scale;
-                    } else {
-                        unsure = true;
-                    }
+            } else if (wide_tri_hit(a, b, c, r.o, d, t, u, v)) {
+                rival = fmn(rival, fmx(t, best));
+                if (t < best) {
+                    best = t; bu = u; bv = v; bt = (int)(tbase + k);
+                    cut = t * kReach * r.scale;
                 }
             }
         }
         if (done) {
-            if (listed) {
-                // nothing to write
-            } else if (kAny) {
-                ovis[ri] = hit ? 0 : 1;
-                if (unsure && !hit) {
-                    const uint32_t slot = atomicAdd(wl.n, 1u);
-                    if (slot < wl.cap) wl.ids[slot] = (uint32_t)ri;
-                    else ovis[ri] = 255;
-                }
-            } else {
-                oprim[ri] = bp;
-                ot[ri] = bp >= 0 ? best : 0.f;
-                if (ou) ou[ri] = bu;
-                if (ov) ov[ri] = bv;
-                if (unsure || grazed) {
-                    const uint32_t slot = atomicAdd(wl.n, 1u);
-                    if (slot < wl.cap) wl.ids[slot] = (uint32_t)ri;
-                    else oprim[ri] = kUndecided;
-                }
-            }
-            ri = -1;
+            if (listed) ri = -1;
+            else over = true;
         }
     }
+    uint64_t fetches = nfetch;
 #pragma unroll
     for (int dd = 32; dd >= 1; dd >>= 1) {
         maxsp = max(maxsp, __shfl_xor(maxsp, dd, 64));
-        nfetch += __shfl_xor(nfetch, dd, 64);
+        fetches += __shfl_xor(fetches, dd, 64);
     }
     if (lane == 0 && maxsp > 0) atomicMax(overflow + 6, (uint32_t)maxsp);
-    if (lane == 0 && nfetch > 0) atomicAdd(fetched, (unsigned long long)nfetch);
+    if (lane == 0 && fetches > 0) atomicAdd(fetched, (unsigned long long)fetches);
 }
 
 // ------------------------------------------------------------- finishing pass
@@ -583,7 +615,8 @@ __device__ __forceinline__ void lane_child(const uint4* nd, int slot, const Wide
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         const AxisPlanes ap = axis_planes(org[k], (w0.w >> (8 * k)) & 255u, ro[k], ri[k]);
-        const float lo = (float)by[32 + 16 * k + slot], hi = (float)by[40 + 16 * k + slot];
+        constexpr float kByte = 1.f / (float)(1 << kPlaneBits);
+        const float lo = (float)by[wide_plane(k, slot)] * kByte, hi = (float)by[wide_plane(k, slot) + 2] * kByte;
         tn = fmx(tn, __builtin_fmaf(ri[k] < 0.f ? hi : lo, ap.an, ap.bn));
         tf = fmn(tf, __builtin_fmaf(ri[k] < 0.f ? lo : hi, ap.af, ap.bf));
     }
