@@ -7,15 +7,17 @@
 
 namespace cav {
 
+// Sort of the first min(cap, *n_dev) pairs.
+constexpr int kCountedSortWords = 8 * 256 + 8;  // digit counts and tile counters of up to 8 passes
 template <typename K>
-struct SortBuffers {
-    K* keys[2] = {nullptr, nullptr};        // keys[0] holds the input
-    uint32_t* vals[2] = {nullptr, nullptr};  // vals[0] holds the input
-    uint32_t* hist = nullptr;                // passes * 256
-    uint32_t* counts = nullptr;              // 256 * tiles
-    uint32_t* offsets = nullptr;             // 256 * tiles
-    const uint32_t* n_dev = nullptr;         // optional: sort only the first min(n, *n_dev) pairs
-    int result = 0;                          // index of the buffer holding the output
+struct CountedSort {
+    K* keys[2] = {nullptr, nullptr};              // keys[0] holds the input
+    uint32_t* vals[2] = {nullptr, nullptr};       // vals[0] holds the input
+    uint32_t* work = nullptr;                     // kCountedSortWords, zero before the sort
+    uint64_t* status[2] = {nullptr, nullptr};     // counted_sort_status_bytes(cap) each
+    const uint32_t* n_dev = nullptr;
+    uint32_t* err = nullptr;                      // nonzero: a look-back wait exceeded its bound
+    int result = 0;                               // index of the buffer holding the output
 };
 
 // Onesweep sort (one kernel per 8-bit digit pass, decoupled look-back).
@@ -33,16 +35,13 @@ struct OnesweepBuffers {
 struct Marker;
 int64_t sort_tiles(int64_t n);
 int64_t onesweep_tiles(int64_t n);  // look-back tiles of the onesweep sort (at most sort_tiles)
-int sort_radix();
-hipError_t radix_sort_pairs(SortBuffers<uint32_t>& b, int64_t n, int key_bits, hipStream_t s,
-                            Marker* mk);
-hipError_t radix_sort_pairs(SortBuffers<uint64_t>& b, int64_t n, int key_bits, hipStream_t s,
-                            Marker* mk);
+int64_t counted_sort_status_bytes(int64_t cap);
 hipError_t onesweep_sort_pairs(OnesweepBuffers<uint32_t>& b, int64_t n, int key_bits, hipStream_t s,
                                Marker* mk);
 hipError_t onesweep_sort_pairs(OnesweepBuffers<uint64_t>& b, int64_t n, int key_bits, hipStream_t s,
                                Marker* mk);
 // launched through a sink (a stream or a graph under construction)
-hipError_t radix_sort_pairs(SortBuffers<uint64_t>& b, int64_t n, int key_bits, LaunchSink& ls);
+hipError_t sort_pairs_counted(CountedSort<uint32_t>& b, int64_t cap, int key_bits, LaunchSink& ls);
+hipError_t sort_pairs_counted(CountedSort<uint64_t>& b, int64_t cap, int key_bits, LaunchSink& ls);
 
 }  // namespace cav

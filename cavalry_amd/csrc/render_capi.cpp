@@ -161,7 +161,7 @@ int ensure_rl_rec(cav_ctx* ctx, RenderState* rs, int64_t cap) {
     free_list(rs->rl_rec);
     rs->rl_rec_cap = 0;
     auto& L = rs->rl_rec;
-    const size_t C = (size_t)cap, T = (size_t)sort_tiles(cap);
+    const size_t C = (size_t)cap, T = (size_t)counted_sort_status_bytes(cap);
     int rc = CAV_OK;
     for (int k = 0; k < 2 && rc == CAV_OK; ++k) {
         rc = grab_into(ctx, L, r.rec_keys[k], 8 * C, "rl update keys");
@@ -169,9 +169,9 @@ int ensure_rl_rec(cav_ctx* ctx, RenderState* rs, int64_t cap) {
     }
     if (rc == CAV_OK) rc = grab_into(ctx, L, r.rec_val, 4 * C, "rl update values");
     if (rc == CAV_OK) rc = grab_into(ctx, L, r.rec_count, 256, "rl update count");
-    if (rc == CAV_OK) rc = grab_into(ctx, L, r.rec_hist, 4 * 8 * 256, "rl update sort histogram");
-    if (rc == CAV_OK) rc = grab_into(ctx, L, r.rec_counts, 4 * 256 * T, "rl update sort counts");
-    if (rc == CAV_OK) rc = grab_into(ctx, L, r.rec_offsets, 4 * 256 * T, "rl update sort offsets");
+    if (rc == CAV_OK) rc = grab_into(ctx, L, r.rec_work, 4 * kCountedSortWords, "rl update sort histogram");
+    if (rc == CAV_OK) rc = grab_into(ctx, L, r.rec_status[0], T, "rl update sort counts");
+    if (rc == CAV_OK) rc = grab_into(ctx, L, r.rec_status[1], T, "rl update sort offsets");
     if (rc != CAV_OK) { free_list(L); return rc; }
     rs->rl_rec_cap = cap;
     r.rec_cap = cap;
@@ -207,14 +207,14 @@ int ensure_rl(cav_ctx* ctx, RenderState* rs, int64_t nsamp, int64_t cells, int64
         if (rc == CAV_OK) rc = grab_into(ctx, L, sl.npdf, 4 * S, "rl next pdf");
         if (rc == CAV_OK) rc = grab_into(ctx, L, sl.ncell, 4 * S, "rl next bin");
         if (rc == CAV_OK) rc = grab_into(ctx, L, r.dims, 64, "rl dimensions");
-        const size_t T = (size_t)sort_tiles(nsamp);
+        const size_t T = (size_t)counted_sort_status_bytes(nsamp);
         for (int k = 0; k < 2 && rc == CAV_OK; ++k) {
             rc = grab_into(ctx, L, r.skeys[k], 4 * S, "rl shading-order keys");
             if (rc == CAV_OK) rc = grab_into(ctx, L, r.svals[k], 4 * S, "rl shading order");
         }
-        if (rc == CAV_OK) rc = grab_into(ctx, L, r.shist, 4 * 8 * 256, "rl shading-order histogram");
-        if (rc == CAV_OK) rc = grab_into(ctx, L, r.scounts, 4 * 256 * T, "rl shading-order counts");
-        if (rc == CAV_OK) rc = grab_into(ctx, L, r.soffsets, 4 * 256 * T, "rl shading-order offsets");
+        if (rc == CAV_OK) rc = grab_into(ctx, L, r.swork, 4 * kCountedSortWords, "rl shading-order histogram");
+        if (rc == CAV_OK) rc = grab_into(ctx, L, r.sstatus[0], T, "rl shading-order counts");
+        if (rc == CAV_OK) rc = grab_into(ctx, L, r.sstatus[1], T, "rl shading-order offsets");
         if (rc != CAV_OK) { free_list(L); return rc; }
         rs->rl_cap = nsamp;
     }

@@ -1159,10 +1159,16 @@ __global__ __launch_bounds__(kBlock) void k_gather(const uint32_t* __restrict__ 
     }
 }
 
-// Deterministic mode, before k_qdist: no records yet (k_qdist appends them;
-// the sort takes only the appended ones).
-__global__ void k_rec_reset(uint32_t* count) {
-    if (threadIdx.x == 0) *count = 0u;
+// Zeroes for a counted sort. Deterministic mode, before k_qdist: no records
+// yet either (count; k_qdist appends them, the sort takes only the appended
+// ones).
+// A look-back that waits past its bound counts as a traversal failure: the
+// render (the served request) ends with an error.
+inline uint32_t* sort_err(uint32_t* trace_counters) { return trace_counters + 1; }
+constexpr int kResetBlock = 1024;
+__global__ __launch_bounds__(kResetBlock) void k_sort_reset(uint32_t* work, uint32_t* count) {
+    for (int i = threadIdx.x; i < kCountedSortWords; i += kResetBlock) work[i] = 0u;
+    if (count && threadIdx.x == 0) *count = 0u;
 }
 
 // The tables a record's request index selects.
@@ -1209,14 +1215,15 @@ __global__ __launch_bounds__(kBlock) void k_rec_sum(const uint64_t* __restrict__
 // Sorts a bounce's records by key (only the appended ones) and sums them.
 template <class Tab>
 hipError_t rec_sort_sum(uint64_t* const keys[2], uint32_t* const idx[2], float* val, uint32_t* count,
-                        uint32_t* hist, uint32_t* counts, uint32_t* offsets, int64_t cap, Tab tab,
+                        uint32_t* work, uint64_t* status0, uint64_t* status1, uint32_t* err, int64_t cap, Tab tab,
                         LaunchSink& ls) {
-    SortBuffers<uint64_t> sb;
+    CountedSort<uint64_t> sb;
     sb.keys[0] = keys[0]; sb.keys[1] = keys[1];
     sb.vals[0] = idx[0]; sb.vals[1] = idx[1];
-    sb.hist = hist; sb.counts = counts; sb.offsets = offsets;
+    sb.work = work; sb.status[0] = status0; sb.status[1] = status1;
     sb.n_dev = count;
-    hipError_t e = radix_sort_pairs(sb, cap, 64, ls);
+    sb.err = err;
+    hipError_t e = sort_pairs_counted(sb, cap, 64, ls);
     if (e != hipSuccess) return e;
     ls.launch("k_rec_sum", &k_rec_sum<Tab>, dim3((unsigned)((cap + kBlock - 1) / kBlock)), dim3(kBlock),
               sb.keys[sb.result], sb.vals[sb.result], val, count, cap, tab);
@@ -1268,14 +1275,16 @@ hipError_t render_rlpath(const RenderArgs& a, const RlArgs& rl, bool init_tables
             const unsigned kb = (unsigned)((nsamp + kBlock - 1) / kBlock);
             hipLaunchKernelGGL(k_entry_keys, dim3(kb), dim3(kBlock), 0, s, a.scene, gr, a.q[from], a.hit_prim,
                                a.hit_t, a.counts + qin, nsamp, rl.skeys[0], rl.svals[0]);
-            SortBuffers<uint32_t> sb;
+            ls.launch("k_sort_reset", &k_sort_reset, dim3(1), dim3(kResetBlock), rl.swork, (uint32_t*)nullptr);
+            CountedSort<uint32_t> sb;
             sb.keys[0] = rl.skeys[0]; sb.keys[1] = rl.skeys[1];
             sb.vals[0] = rl.svals[0]; sb.vals[1] = rl.svals[1];
-            sb.hist = rl.shist; sb.counts = rl.scounts; sb.offsets = rl.soffsets;
+            sb.work = rl.swork; sb.status[0] = rl.sstatus[0]; sb.status[1] = rl.sstatus[1];
             sb.n_dev = a.counts + qin;
+            sb.err = sort_err(a.trace_counters);
             int bits = 1;
             while (((int64_t)1 << bits) < 8 * nent) ++bits;
-            if ((e = radix_sort_pairs(sb, nsamp, bits, s, nullptr)) != hipSuccess) return e;
+            if ((e = sort_pairs_counted(sb, nsamp, bits, ls)) != hipSuccess) return e;
             at = from ^ 1;
             hit = RlHits{(int32_t*)rl.svals[0], (float*)rl.svals[1], hu ? (float*)rl.skeys[0] : nullptr,
                          hu ? (float*)rl.skeys[1] : nullptr};
@@ -1290,12 +1299,14 @@ hipError_t render_rlpath(const RenderArgs& a, const RlArgs& rl, bool init_tables
                                       a.sh.limit, a.sh.src, a.sh.dst, a.vis, a.trace_counters, a.launch, s, &a.coop)) != hipSuccess)
             return e;
         const RlRecords rec{rl.rec_keys[0], rl.rec_val, rl.rec_count, rl.rec_idx[0]};
-        if (rec.keys) ls.launch("k_rec_reset", &k_rec_reset, dim3(1), dim3(64), rl.rec_count);
+        if (rec.keys)
+            ls.launch("k_sort_reset", &k_sort_reset, dim3(1), dim3(kResetBlock), rl.rec_work, rl.rec_count);
         launch_qdist<RenderSrc>("k_qdist", a.launch.shade_block, nsamp, ls, src, a.scene, a.halton, a.q[at],
                                 rl.q[at], rl.slots, a.vis, hit.prim, hit.t, hit.u, hit.v, a.counts, qin, rec);
         if (rec.keys &&
-            (e = rec_sort_sum(rl.rec_keys, rl.rec_idx, rl.rec_val, rl.rec_count, rl.rec_hist, rl.rec_counts,
-                              rl.rec_offsets, rl.rec_cap, RenderTables{t}, ls)) != hipSuccess)
+            (e = rec_sort_sum(rl.rec_keys, rl.rec_idx, rl.rec_val, rl.rec_count, rl.rec_work, rl.rec_status[0],
+                              rl.rec_status[1], sort_err(a.trace_counters), rl.rec_cap, RenderTables{t}, ls)) !=
+                hipSuccess)
             return e;
         hipLaunchKernelGGL(k_finish_q, dim3((unsigned)((nent + kEntryWaves - 1) / kEntryWaves)),
                            dim3(64 * kEntryWaves), 0, s, t, nent, rl.alpha_scale);
@@ -1343,13 +1354,13 @@ void pool_rl_learn(const PoolDev& p, int qin, bool det, LaunchSink& ls) {
     RlRecords rec{nullptr, nullptr, nullptr, nullptr};
     if (det) {
         rec = RlRecords{p.rl.rec_keys[0], p.rl.rec_val, p.rl.rec_count, p.rl.rec_idx[0]};
-        ls.launch("k_rec_reset", &k_rec_reset, dim3(1), dim3(64), p.rl.rec_count);
+        ls.launch("k_sort_reset", &k_sort_reset, dim3(1), dim3(kResetBlock), p.rl.rec_work, p.rl.rec_count);
     }
     launch_qdist<PoolSrc>("k_qdist<pool>", p.launch.shade_block, p.cap, ls, src, p.scene, p.halton, p.q[qin],
                           p.rl.q[qin], p.rl.sl, p.vis, p.hit_prim, p.hit_t, hu, hv, p.counts, qin, rec);
     if (det)
-        (void)rec_sort_sum(p.rl.rec_keys, p.rl.rec_idx, p.rl.rec_val, p.rl.rec_count, p.rl.rec_hist, p.rl.rec_counts,
-                           p.rl.rec_offsets, p.rl.rec_cap, PoolTables{p.rl.req}, ls);
+        (void)rec_sort_sum(p.rl.rec_keys, p.rl.rec_idx, p.rl.rec_val, p.rl.rec_count, p.rl.rec_work, p.rl.rec_status[0],
+                           p.rl.rec_status[1], sort_err(p.trace_counters), p.rl.rec_cap, PoolTables{p.rl.req}, ls);
     // the updates of every request with hits; a fixed grid, so that the
     // launch does not depend on which requests are in the pool
     ls.launch("k_pool_finish_q", &k_pool_finish_q, dim3(2048), dim3(64 * kEntryWaves), (const RlReqState*)p.rl.req,

@@ -44,7 +44,8 @@ struct PoolRl {
     uint32_t* rec_idx[2];
     float* rec_val;
     uint32_t* rec_count;
-    uint32_t *rec_hist, *rec_counts, *rec_offsets;
+    uint32_t* rec_work;
+    uint64_t* rec_status[2];
     int64_t rec_cap;
 };
 

@@ -276,10 +276,10 @@ int make_pool(cav_server* sv, cav_scene* sc, Pool*& out) {
     A(R.sl.ldir, 12 * C); A(R.sl.inc, 12 * C); A(R.sl.sh_idx, 4 * C); A(R.sl.ndir, 12 * C); A(R.sl.npdf, 4 * C);
     A(R.sl.ncell, 4 * C);
     R.rec_cap = 3 * (int64_t)C;  // at most 3 updates per task
-    const size_t RC = (size_t)R.rec_cap, RT = (size_t)sort_tiles(R.rec_cap);
+    const size_t RC = (size_t)R.rec_cap, RT = (size_t)counted_sort_status_bytes(R.rec_cap);
     for (int k = 0; k < 2; ++k) { A(R.rec_keys[k], 8 * RC); A(R.rec_idx[k], 4 * RC); }
-    A(R.rec_val, 4 * RC); A(R.rec_count, 256); A(R.rec_hist, 4 * 8 * 256); A(R.rec_counts, 4 * 256 * RT);
-    A(R.rec_offsets, 4 * 256 * RT);
+    A(R.rec_val, 4 * RC); A(R.rec_count, 256); A(R.rec_work, 4 * kCountedSortWords); A(R.rec_status[0], RT);
+    A(R.rec_status[1], RT);
     A(p->d_reqs, sizeof(ReqDev) * kSlots);
     const int ring = sv->cfg.max_steps_ahead + 2;
     A(p->d_chunks, sizeof(Chunk) * kSlots * ring);
