@@ -776,6 +776,17 @@ __device__ inline float lane_f(float v, int k) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
 }
 
+// A deterministic request's entries with updates are marked by k_rec_sum, in
+// the sign of a count that is never negative (the first bin's total, the first
+// light's count): finishing them then reads a word per entry of the pool's
+// requests instead of all their counts. (Marked by k_qdist's lanes instead,
+// atomic updates cost it 620 to 730 us a bounce of the guided render.)
+constexpr int32_t kMark = INT32_MIN;
+__device__ inline void mark(int32_t* p) {
+    const int32_t v = *p;
+    if (v >= 0) *p = v | kMark;  // (several threads may: they store the same word)
+}
+
 __device__ inline void finish_q_entry(const RlTables& t, int64_t e, float alpha_scale) {
     const int lane = threadIdx.x & 63;
     const int64_t base = e * kXY;
@@ -783,7 +794,7 @@ __device__ inline void finish_q_entry(const RlTables& t, int64_t e, float alpha_
     const int n0 = t.cnt[base + c0], n1 = t.cnt[base + c1];
     if (__ballot(n0 != 0 || n1 != 0) == 0) return;
     float q0 = t.Q[base + c0], q1 = t.Q[base + c1];
-    int tot0 = t.total[base + c0], tot1 = t.total[base + c1];
+    int tot0 = t.total[base + c0] & ~kMark, tot1 = t.total[base + c1];
     if (n0 != 0) {
         float a = (float)n0 / (float)(tot0 + n0);
         a = a * alpha_scale;
@@ -822,24 +833,70 @@ __device__ inline void finish_q_entry(const RlTables& t, int64_t e, float alpha_
     t.Q[base + c1] = q1;
 }
 
+// The marked ones of a wave's entries (first, first + step, ... below nent, 64
+// at most), one after the other; counts: the marks, `stride` words apart.
+template <typename F>
+__device__ inline void marked_entries(const int32_t* counts, int64_t stride, int64_t first, int64_t step, int64_t nent,
+                                      F&& finish) {
+    const int64_t mine = first + step * (threadIdx.x & 63);
+    for (uint64_t m = __ballot(mine < nent && counts[mine * stride] < 0); m != 0ull; m &= m - 1ull)
+        finish(first + step * (__ffsll((unsigned long long)m) - 1));
+}
+
 __global__ __launch_bounds__(64 * kEntryWaves) void k_finish_q(RlTables t, int64_t nent, float alpha_scale) {
     const int64_t e = (int64_t)blockIdx.x * kEntryWaves + (threadIdx.x >> 6);
     if (e < nent) finish_q_entry(t, e, alpha_scale);
 }
 
-// The same over the tables of every pool request with hits this bounce
-// (live[slot]), one entry per wave on a fixed grid.
-__global__ __launch_bounds__(64 * kEntryWaves) void k_pool_finish_q(const RlReqState* __restrict__ rl,
-                                                                    const uint8_t* __restrict__ live, int nslots) {
-    const int64_t w0 = (int64_t)blockIdx.x * kEntryWaves + (threadIdx.x >> 6);
-    const int64_t nw = (int64_t)gridDim.x * kEntryWaves;
-    for (int sl = 0; sl < nslots; ++sl) {
-        if (!live[sl]) continue;
-        const RlReqState& R = rl[sl];
-        const int64_t nent = (int64_t)R.gr.g * R.gr.g * R.gr.g;
-        for (int64_t e = w0; e < nent; e += nw) finish_q_entry(R.t, e, R.alpha_scale);
+// Pool: the waves of the launch are dealt out in turn to the requests with
+// hits this bounce (live[slot]), so the launch does not depend on which are in
+// the pool. A wave's request (-1: none), which of that request's waves it is
+// and how many there are. With 12 requests of 32^3 entries and 64 lights, a
+// step: the Q tables 37 to 11 us, the light statistics 35 to 8.4.
+struct PoolPart {
+    int slot, part, parts;
+};
+__device__ inline PoolPart pool_part(const uint8_t* live) {
+    static_assert(kPoolSlots == 256, "four slots to a lane");
+    const int per = blockDim.x >> 6, lane = threadIdx.x & 63;
+    const int w = (int)blockIdx.x * per + (int)(threadIdx.x >> 6), nw = (int)gridDim.x * per;
+    const uint32_t four = reinterpret_cast<const uint32_t*>(live)[lane];
+    uint64_t m[4];
+    int n = 0;
+    for (int k = 0; k < 4; ++k) {
+        m[k] = __ballot(((four >> (8 * k)) & 255u) != 0u);
+        n += __popcll(m[k]);
     }
+    if (n == 0) return PoolPart{-1, 0, 1};
+    int r = w % n;
+    PoolPart p{-1, w / n, (nw - 1 - r) / n + 1};
+    for (int k = 0; k < 4 && p.slot < 0; ++k) {
+        const int c = __popcll(m[k]);
+        if (r >= c) {
+            r -= c;
+            continue;
+        }
+        uint64_t left = m[k];
+        for (; r > 0; --r) left &= left - 1ull;
+        p.slot = 4 * (__ffsll((unsigned long long)left) - 1) + k;
+    }
+    return p;
 }
+__global__ __launch_bounds__(64 * kEntryWaves) void k_pool_finish_q(const RlReqState* __restrict__ rl,
+                                                                    const uint8_t* __restrict__ live) {
+    const PoolPart p = pool_part(live);
+    if (p.slot < 0) return;
+    const RlReqState& R = rl[p.slot];
+    const int64_t nent = (int64_t)R.gr.g * R.gr.g * R.gr.g;
+    if (!R.det) {
+        for (int64_t e = p.part; e < nent; e += p.parts) finish_q_entry(R.t, e, R.alpha_scale);
+        return;
+    }
+    for (int64_t first = p.part; first < nent; first += 64 * (int64_t)p.parts)
+        marked_entries(R.t.total, kXY, first, p.parts, nent, [&](int64_t e) { finish_q_entry(R.t, e, R.alpha_scale); });
+}
+
+constexpr unsigned kPoolFinishBlocks = 2048;
 
 // finishLightingTraining (:463-514) per entry, clearing the new statistics
 // (prepareLightingTraining).
@@ -849,6 +906,7 @@ __device__ inline void finish_light_entry(const RlTables& t, int64_t e, int L) {
     int32_t* cnt = t.lcount + e * L;
     int32_t* ncnt = t.lnewc + e * L;
     float* cdf = t.ldist + e * L;
+    if (cnt[0] < 0) cnt[0] &= ~kMark;
     float sum_r = 0, valid = 0;
     bool any = false;
     for (int k = 0; k < L; ++k) {
@@ -895,8 +953,12 @@ __device__ inline void finish_light_wave(const RlTables& t, int64_t e, int L) {
         const int64_t at = base + k0 + lane;
         const int nc = k0 + lane < L ? t.lnewc[at] : 0;
         float r = 0.f;
+        if (nc > 0 || k0 + lane == 0) {
+            const int c = t.lcount[at] & ~kMark;
+            if (nc <= 0) t.lcount[at] = c;  // (the first light's: takes the mark off)
+        }
         if (nc > 0) {
-            const int c = t.lcount[at];
+            const int c = t.lcount[at] & ~kMark;
             const float tc = (float)(c + nc);
             r = ((float)c / tc) * t.lres[at] + ((float)nc / tc) * (t.lnew[at] / (float)nc);
             t.lres[at] = r;
@@ -959,17 +1021,19 @@ unsigned finish_light_blocks(int64_t nent, int L) {
 }
 
 __global__ __launch_bounds__(kBlock) void k_pool_finish_light(const RlReqState* __restrict__ rl,
-                                                              const uint8_t* __restrict__ live, int nslots, int L) {
-    const int64_t t0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int64_t nt = (int64_t)gridDim.x * kBlock;
-    for (int sl = 0; sl < nslots; ++sl) {
-        if (!live[sl]) continue;
-        const RlReqState& R = rl[sl];
-        const int64_t nent = (int64_t)R.gr.g * R.gr.g * R.gr.g;
-        if (L >= kLightWave) {
-            for (int64_t e = t0 >> 6; e < nent; e += nt >> 6) finish_light_wave(R.t, e, L);
-        } else {
-            for (int64_t e = t0; e < nent; e += nt) finish_light_entry(R.t, e, L);
+                                                              const uint8_t* __restrict__ live, int L) {
+    const PoolPart p = pool_part(live);
+    if (p.slot < 0) return;
+    const RlReqState& R = rl[p.slot];
+    const int64_t nent = (int64_t)R.gr.g * R.gr.g * R.gr.g, parts = p.parts;
+    for (int64_t first = p.part; first < nent; first += 64 * parts) {
+        const int64_t e = first + parts * (threadIdx.x & 63);
+        if (L >= kLightWave && R.det) {
+            marked_entries(R.t.lcount, L, first, parts, nent, [&](int64_t at) { finish_light_wave(R.t, at, L); });
+        } else if (L >= kLightWave) {
+            for (int64_t at = first; at < nent && at < first + 64 * parts; at += parts) finish_light_wave(R.t, at, L);
+        } else if (e < nent && (!R.det || R.t.lcount[e * L] < 0)) {
+            finish_light_entry(R.t, e, L);
         }
     }
 }
@@ -1173,10 +1237,12 @@ __global__ __launch_bounds__(kResetBlock) void k_sort_reset(uint32_t* work, uint
 
 // The tables a record's request index selects.
 struct RenderTables {
+    static constexpr bool kMarks = false;
     RlTables t;
     __device__ const RlTables& of(uint32_t) const { return t; }
 };
 struct PoolTables {
+    static constexpr bool kMarks = true;
     const RlReqState* rl;
     __device__ const RlTables& of(uint32_t x) const { return rl[x].t; }
 };
@@ -1188,7 +1254,7 @@ template <class Tab>
 __global__ __launch_bounds__(kBlock) void k_rec_sum(const uint64_t* __restrict__ keys,
                                                     const uint32_t* __restrict__ idx,
                                                     const float* __restrict__ val, const uint32_t* count,
-                                                    int64_t cap, Tab tab) {
+                                                    int64_t cap, Tab tab, int nlights) {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int64_t n = (int64_t)*count < cap ? (int64_t)*count : cap;
     if (i >= n) return;
@@ -1206,9 +1272,11 @@ __global__ __launch_bounds__(kBlock) void k_rec_sum(const uint64_t* __restrict__
     if ((seg >> kRecKeyBits) & 1ull) {
         t.lnew[key] = sum;
         t.lnewc[key] = c;
+        if (Tab::kMarks) mark(t.lcount + (int64_t)((uint32_t)key / (uint32_t)nlights) * nlights);
     } else {
         t.newQ[key] = sum;
         t.cnt[key] = c;
+        if (Tab::kMarks) mark(t.total + (key & ~(int64_t)(kXY - 1)));
     }
 }
 
@@ -1216,7 +1284,7 @@ __global__ __launch_bounds__(kBlock) void k_rec_sum(const uint64_t* __restrict__
 template <class Tab>
 hipError_t rec_sort_sum(uint64_t* const keys[2], uint32_t* const idx[2], float* val, uint32_t* count,
                         uint32_t* work, uint64_t* status0, uint64_t* status1, uint32_t* err, int64_t cap, Tab tab,
-                        LaunchSink& ls) {
+                        int nlights, LaunchSink& ls) {
     CountedSort<uint64_t> sb;
     sb.keys[0] = keys[0]; sb.keys[1] = keys[1];
     sb.vals[0] = idx[0]; sb.vals[1] = idx[1];
@@ -1226,7 +1294,7 @@ hipError_t rec_sort_sum(uint64_t* const keys[2], uint32_t* const idx[2], float* 
     hipError_t e = sort_pairs_counted(sb, cap, 64, ls);
     if (e != hipSuccess) return e;
     ls.launch("k_rec_sum", &k_rec_sum<Tab>, dim3((unsigned)((cap + kBlock - 1) / kBlock)), dim3(kBlock),
-              sb.keys[sb.result], sb.vals[sb.result], val, count, cap, tab);
+              sb.keys[sb.result], sb.vals[sb.result], val, count, cap, tab, nlights);
     return ls.err;
 }
 
@@ -1305,7 +1373,7 @@ hipError_t render_rlpath(const RenderArgs& a, const RlArgs& rl, bool init_tables
                                 rl.q[at], rl.slots, a.vis, hit.prim, hit.t, hit.u, hit.v, a.counts, qin, rec);
         if (rec.keys &&
             (e = rec_sort_sum(rl.rec_keys, rl.rec_idx, rl.rec_val, rl.rec_count, rl.rec_work, rl.rec_status[0],
-                              rl.rec_status[1], sort_err(a.trace_counters), rl.rec_cap, RenderTables{t}, ls)) !=
+                              rl.rec_status[1], sort_err(a.trace_counters), rl.rec_cap, RenderTables{t}, L, ls)) !=
                 hipSuccess)
             return e;
         hipLaunchKernelGGL(k_finish_q, dim3((unsigned)((nent + kEntryWaves - 1) / kEntryWaves)),
@@ -1360,13 +1428,13 @@ void pool_rl_learn(const PoolDev& p, int qin, bool det, LaunchSink& ls) {
                           p.rl.q[qin], p.rl.sl, p.vis, p.hit_prim, p.hit_t, hu, hv, p.counts, qin, rec);
     if (det)
         (void)rec_sort_sum(p.rl.rec_keys, p.rl.rec_idx, p.rl.rec_val, p.rl.rec_count, p.rl.rec_work, p.rl.rec_status[0],
-                           p.rl.rec_status[1], sort_err(p.trace_counters), p.rl.rec_cap, PoolTables{p.rl.req}, ls);
-    // the updates of every request with hits; a fixed grid, so that the
-    // launch does not depend on which requests are in the pool
-    ls.launch("k_pool_finish_q", &k_pool_finish_q, dim3(2048), dim3(64 * kEntryWaves), (const RlReqState*)p.rl.req,
-              (const uint8_t*)p.rl.live, kPoolSlots);
-    ls.launch("k_pool_finish_light", &k_pool_finish_light, dim3(2048), dim3(kBlock), (const RlReqState*)p.rl.req,
-              (const uint8_t*)p.rl.live, kPoolSlots, p.scene.nlights);
+                           p.rl.rec_status[1], sort_err(p.trace_counters), p.rl.rec_cap, PoolTables{p.rl.req},
+                           p.scene.nlights, ls);
+    // the updates of every request with hits
+    ls.launch("k_pool_finish_q", &k_pool_finish_q, dim3(kPoolFinishBlocks), dim3(64 * kEntryWaves),
+              (const RlReqState*)p.rl.req, (const uint8_t*)p.rl.live);
+    ls.launch("k_pool_finish_light", &k_pool_finish_light, dim3(kPoolFinishBlocks), dim3(kBlock),
+              (const RlReqState*)p.rl.req, (const uint8_t*)p.rl.live, p.scene.nlights);
     ls.launch("k_next<pool>", &k_next<PoolSrc>, dim3(nb), dim3(kBlock), src, p.scene, p.halton, p.q[qin], p.q[qout],
               p.rl.q[qout], p.rl.sl, p.hit_prim, p.hit_t, hu, hv, p.counts, qin, qout, p.rid[qout],
               p.depth[qout]);

@@ -1019,10 +1019,11 @@ __global__ __launch_bounds__(64) void k_closest_coop(const TRec* __restrict__ re
     if (lane == 0 && nfetch > 0) atomicAdd(fetched, (unsigned long long)nfetch);
 }
 
-// zeroes n words; a kernel rather than hipMemsetAsync so the launch sequence
-// can be captured into a hipGraph
-__global__ void k_clear_words(uint32_t* p, int n) {
+// zeroes n words at p and m at q; a kernel rather than hipMemsetAsync so the
+// launch sequence can be captured into a hipGraph
+__global__ void k_clear_words(uint32_t* p, int n, uint32_t* q, int m) {
     if ((int)threadIdx.x < n) p[threadIdx.x] = 0u;
+    if ((int)threadIdx.x < m) q[threadIdx.x] = 0u;
 }
 
 // Workgroups of a persistent launch of `threads`-thread workgroups:
@@ -1236,9 +1237,8 @@ hipError_t trace_occluded(const TraceBvh& bvh, const float* rays,
 void trace_closest_queue(const TraceBvh& bvh, const float* rays,
                          const uint32_t* nrays_dev, int64_t capacity, int32_t* prim, float* t, float* u, float* v,
                          uint32_t* counters, const TraceLaunch& L, LaunchSink& ls, const TraceCoop* coop) {
-    ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 2, 2);
-    if (coop && coop->longs && L.handoff < kNoHandoff)
-        ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 26, 5);
+    const bool pass = coop && coop->longs && L.handoff < kNoHandoff;
+    ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 2, 2, counters + 26, pass ? 5 : 0);
     trace_near(bvh, rays, capacity, nrays_dev, prim, t, u, v, counters, L, coop, ls);
 }
 
@@ -1246,9 +1246,8 @@ void trace_occluded_queue(const TraceBvh& bvh, const float* rays, const uint32_t
                           int64_t capacity, const float* limit, const int32_t* src, const int32_t* dst,
                           uint8_t* visible, uint32_t* counters, const TraceLaunch& L, LaunchSink& ls,
                           const TraceCoop* coop) {
-    ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 4, 2);
-    if (coop && coop->spill && L.handoff < kNoHandoff)
-        ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 20, 6);
+    const bool pass = coop && coop->spill && L.handoff < kNoHandoff;
+    ls.launch("k_clear_words", &k_clear_words, dim3(1), dim3(64), counters + 4, 2, counters + 20, pass ? 6 : 0);
     trace_any(bvh, rays, capacity, nrays_dev, limit, src, dst, visible, counters, L, coop, ls);
 }
 
