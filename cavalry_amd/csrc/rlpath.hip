@@ -560,7 +560,9 @@ __global__ __launch_bounds__(B) void k_qdist(Src src, SceneDev sc, HaltonDev h, 
         // and one specular lane held its wave for all 128 bins. Adding 0
         // changes no sum as long as every Q is finite. rlpath on a 400K
         // interior, whole kernel per bounce: 980 us before, 788 us with this and the shorter sincos,
-        // 607 us since the tasks are copied into shading order (k_gather).
+        // 607 us once the tasks were copied into shading order (k_gather),
+        // 462 us with the sampled row below free of branches and with one
+        // lane per request telling that a sample was taken.
         uint32_t up[4] = {~0u, ~0u, ~0u, ~0u};
         bool skip = !matte;
         if (skip) {
@@ -668,31 +670,70 @@ __global__ __launch_bounds__(B) void k_qdist(Src src, SceneDev sc, HaltonDev h, 
             if (mono) {
                 // non-decreasing, NaN-free CDF: the binary search returns the
                 // first bin with cdf >= f (the last bin if none)
+                // (x / sum >= f without the division but near f * sum: the
+                // three roundings are 2^-24 each)
+                const float fs = f * sum;
+                const bool far = fs > 1e-30f && sum < 1e30f;
+                const float lo = far ? fs * (1.f - 0x1p-21f) : -INFINITY, hi = far ? fs * (1.f + 0x1p-21f) : INFINITY;
+                const auto reaches = [=](float x) {
+                    bool ge = x > hi;
+                    if (!ge && !(x < lo)) ge = x / sum >= f;
+                    return ge;
+                };
                 int r = 0;
 #pragma unroll
-                for (int k = 0; k < kNY - 1; ++k) r += rows[k] / sum < f ? 1 : 0;
+                for (int k = 0; k < kNY - 1; ++k) r += reaches(rows[k]) ? 0 : 1;
                 float pre = 0.f;
 #pragma unroll
                 for (int k = 0; k < kNY - 1; ++k) pre = k == r - 1 ? rows[k] : pre;
                 float u, xy;
                 be.row(r, u, xy);
-                float prevc = r == 0 ? 0.f : pre / sum;
                 int found = kNX - 1;
-                bool hit = false;
-                const uint32_t upw = r < 2 ? up[0] : (r < 4 ? up[1] : (r < 6 ? up[2] : up[3]));
-                const uint32_t upr = upw >> ((r & 1) * kNX);
-                for (int p = 0; p < kNX && !hit; ++p) {
-                    if ((upr >> p) & 1u) pre += be.bin(u, xy, p, Qe[r * kNX + p]);
-                    const float cm = pre / sum;
-                    if (cm >= f || p == kNX - 1) {
-                        found = p;
-                        b0 = cm;
-                        b1 = prevc;
-                        hit = true;
-                    } else {
-                        prevc = cm;
+                float at = pre, below = pre;  // the prefixes at the bin found and before it
+                if (matte) {
+                    float4v qr[kNX / 4];
+                    be.q_row(r, qr);
+                    float pf[kNX];
+#pragma unroll
+                    for (int p = 0; p < kNX; ++p) {
+                        pre = pre + be.matte_bin(u, xy, p, qr[p / 4][p % 4]);
+                        pf[p] = pre;
+                    }
+                    // the sums do not decrease: past those surely short of it, to the first that is not
+                    found = 0;
+#pragma unroll
+                    for (int p = 0; p < kNX - 1; ++p) found += pf[p] < lo ? 1 : 0;
+                    while (true) {
+#pragma unroll
+                        for (int p = 0; p < kNX; ++p) {
+                            below = p == found - 1 ? pf[p] : below;
+                            at = p == found ? pf[p] : at;
+                        }
+                        if (found == kNX - 1 || reaches(at)) break;
+                        ++found;
+                    }
+                } else {
+                    // (a bin of weight 0 has its predecessor's prefix, which fell
+                    // short, but for the first one's when f is 0)
+                    const uint32_t upw = r < 2 ? up[0] : (r < 4 ? up[1] : (r < 6 ? up[2] : up[3]));
+                    uint32_t bins = (upw >> ((r & 1) * kNX)) & 0xffffu;
+                    if (!(bins & 1u) && reaches(at)) {  // f = 0
+                        found = 0;
+                        bins = 0u;
+                    }
+                    for (; bins != 0u; bins &= bins - 1u) {
+                        const int p = __ffs((int)bins) - 1;
+                        below = at;
+                        at += be.bin(u, xy, p, Qe[r * kNX + p]);
+                        if (reaches(at)) {
+                            found = p;
+                            break;
+                        }
+                        if (p < kNX - 1) below = at;
                     }
                 }
+                b0 = at / sum;
+                b1 = below / sum;
                 cell = r * kNX + found;
             } else {
                 // the reference's binary search, recomputing the prefix sums
@@ -764,8 +805,16 @@ __global__ __launch_bounds__(B) void k_qdist(Src src, SceneDev sc, HaltonDev h, 
     wave_add(up_fl, up_cl, v_l, up_l && !use_rec);
     wave_add(up_fp, up_cp, v_p, up_p && !use_rec);
     wave_add(up_fd, up_cd, v_d, up_d && !use_rec);
-    if (valid && __hip_atomic_load(&dims[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-        atomicMax(&dims[1], 1);
+    // one lane per request tells it: waves that end together and find the word
+    // still 0 sent an atomic per lane (the first bounce: 2.1 ms, 0.69 now)
+    const unsigned long long key = reinterpret_cast<unsigned long long>(dims);
+    for (uint64_t todo = __ballot(valid); todo != 0ull;) {
+        const int lead = __ffsll((unsigned long long)todo) - 1;
+        todo &= ~__ballot(valid && key == __shfl(key, lead, 64));
+        if ((int)(threadIdx.x & 63) == lead &&
+            __hip_atomic_load(&dims[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+            atomicMax(&dims[1], 1);
+    }
 }
 
 // finishUpdateQ (:97-110, 753-762) and averageQ (:52-72, 765-772) for one
