@@ -637,28 +637,33 @@ def main() -> int:
         "build_frac": round(ALG_BYTES_PER_TRI_30 * n / (lbvh_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
         "build_alg_bytes_per_tri": ALG_BYTES_PER_TRI_30,
     }
-    # roofline of the step's dominant kernel, the traversal: algorithmic bytes
-    # = the 64-byte records the reference's visiting order fetches (counted by
-    # the kernel over the timed steps) + the rays read and the hits written
+    # roofline of the step's dominant kernel, the traversal: the records its
+    # timed launches fetched (64 bytes each: a wide node is 80, a wide triangle
+    # 48, a record of the reference's tree 64) + the rays read and the hits
+    # written; launches that walk the reference's tree count the records of its
+    # visiting order instead, which are fewer than the wave passes fetch
     fetch = {k: v / args.steps for k, v in fetches.items()}
+    wide = {k: fetch[k] < ref_fetch[k] for k in fetch}
+    counted = {k: fetch[k] if wide[k] else ref_fetch[k] for k in fetch}
     trav_bytes = {
-        "closest": ref_fetch["closest"] * TRACE_RECORD_BYTES + r * (24 + 8),
-        "occluded": ref_fetch["occluded"] * TRACE_RECORD_BYTES + r * (24 + 4 + 1),
+        "closest": counted["closest"] * TRACE_RECORD_BYTES + r * (24 + 8),
+        "occluded": counted["occluded"] * TRACE_RECORD_BYTES + r * (24 + 4 + 1),
     }
     trav_ms = {"closest": stages["trace_closest"], "occluded": stages["trace_shadow"]}
     tdom = max(trav_ms, key=lambda k: trav_ms[k])
     t_ach = trav_bytes[tdom] / (trav_ms[tdom] * 1e-3) / 1e9
     roofline = {
-        "bound": "hbm", "kernel": f"k_trace<{'closest' if tdom == 'closest' else 'any'}>",
+        "bound": "hbm",
+        "kernel": f"{'k_wide_trace' if wide[tdom] else 'k_trace'}<{'closest' if tdom == 'closest' else 'any'}>",
         "achieved": round(t_ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": round(t_ach / HBM_PEAK_GBS, 4), "traffic": None,
         "avg_launch_ms": round(trav_ms[tdom], 4), "alg_bytes_per_launch": int(trav_bytes[tdom]),
         "records_per_ray": round(ref_fetch[tdom] / r, 1),
         "records_fetched_per_ray": round(fetch[tdom] / r, 1),
-        "note": "algorithmic bytes count every record the visiting order fetches (closest-hit: the "
-                "reference's; any-hit: the reference's up to the ray's limit), records_per_ray, counted "
-                "on an untimed trace without the cooperative passes, whether L2 or HBM serves it; "
-                "records_fetched_per_ray is what the timed traces fetched",
+        "note": "algorithmic bytes count every record the timed traces of the wide tree fetched, whether "
+                "L2 or HBM serves it (records_fetched_per_ray); records_per_ray is what the reference's "
+                "visiting order fetches (closest-hit; any-hit up to the ray's limit), counted on an untimed "
+                "trace without the cooperative passes",
         "lbvh_build_frac": lbvh_roofline["build_frac"],
     }
     traffic_file = os.path.join(ROOT, "profiles", "traffic.json")
