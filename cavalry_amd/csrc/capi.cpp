@@ -181,7 +181,12 @@ static int bvh_run(cav_ctx* ctx, cav_bvh* h, const float* tris_dev, const float*
     // within 2^40 (its planes' distances then stay finite) and no traversal of
     // the reference's tree can outgrow its 64-entry stack.
     h->wide_ok = h->wide.base != nullptr && (height & 0xffffu) <= 64u && wide_err == 0;
-    for (int k = 0; k < 6; ++k) h->wide_ok = h->wide_ok && std::fabs(ord_to_float(box[k])) <= 1099511627776.f;
+    float boxf[6];
+    for (int k = 0; k < 6; ++k) {
+        boxf[k] = ord_to_float(box[k]);
+        h->wide_ok = h->wide_ok && std::fabs(boxf[k]) <= 1099511627776.f;
+    }
+    if (h->wide_ok) h->wide_scale = wide_scale(boxf);
     if (sort_err) return fail(ctx, CAV_ERR_HIP, "radix sort: a look-back wait exceeded its bound");
     cav_bvh_stats st{};
     st.n = n;

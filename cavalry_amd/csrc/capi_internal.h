@@ -31,6 +31,7 @@ struct cav_bvh {
     int32_t* mesh = nullptr;    // n, original order (may be null)
     cav::WideBuffers wide;      // wide traversal tree (base null: no memory for it)
     bool wide_ok = false;       // the last build's wide tree can stand in for the reference's
+    cav::WideScale wide_scale{};  // of the last build's triangles
     // long-ray pass buffers (cav::trace_coop_bytes(spill_cap, spill_cap)),
     // grown to the largest batch traced
     mutable void* spill = nullptr;
@@ -50,7 +51,9 @@ int dev_alloc(cav_ctx* ctx, void** p, size_t bytes, const char* what);
 // what the traces of a BVH read
 inline TraceBvh bvh_trace(const cav_bvh* h) {
     TraceBvh t{h->rec, h->n, h->root, WideDev{}};
-    if (h->wide_ok) t.wide = WideDev{h->wide.nodes, h->wide.tris, h->b.nbox, h->b.topo, h->wide.leaf_of};
+    if (h->wide_ok)
+        t.wide = WideDev{h->wide.nodes, h->wide.tris, h->b.nbox, h->b.topo, h->wide.leaf_of, h->wide_scale.far_origin,
+                         h->wide_scale.rcp_max};
     return t;
 }
 // frees context-owned state of other subsystems before the stream goes away

@@ -181,6 +181,8 @@ struct WideDev {
     const NodeBox* nbox = nullptr;
     const int4* topo = nullptr;
     const int32_t* leaf_of = nullptr;
+    float far_origin = 0.f;  // WideScale of the scene
+    float rcp_max = 0.f;
 };
 // A flattened BVH of ntris triangles with its wide tree, if it has one.
 struct TraceBvh {

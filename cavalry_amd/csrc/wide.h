@@ -30,6 +30,29 @@ constexpr int kWideLeaf = 3;  // triangles per leaf slot at most
 // one without holds at least 4 triangles (or is the root)
 inline int64_t wide_node_capacity(int64_t n) { return 2 * n / 7 + 16; }
 
+// Limits that follow from the largest coordinate of a scene, 2^k at most
+// (k from -20 to 40). A ray that hardly moves along an axis has a reciprocal
+// there that is cut off at rcp_max, which brings the planes of that axis
+// closer than they are. That must not end a box early: a ray that starts
+// inside (or on the edge of) an exact box starts at least 2^-14 units inside
+// the planes that hold it, or 2^(2k - 81), which rcp_max takes to 2^(k + 23);
+// and a ray from within 2^(k + 20) has left the scene along its main axis
+// before 2^(k + 21). Sums of two coordinates times rcp_max stay below 2^126.
+struct WideScale {
+    float far_origin;   // rays from beyond go to the reference's traversal
+    float rcp_max;
+    uint32_t min_unit;  // exponent (biased by 127) of the smallest unit, 2^(2k - 67)
+};
+__host__ __device__ inline WideScale wide_scale(const float* box6) {
+    float m = 0.f;
+    for (int i = 0; i < 6; ++i) m = __builtin_fmaxf(m, __builtin_fabsf(box6[i]));
+    int k = (int)((__builtin_bit_cast(uint32_t, m) + 0x7fffffu) >> 23) - 127;
+    k = k < -20 ? -20 : (k > 40 ? 40 : k);
+    const auto pow2 = [](int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); };
+    const int e = 60 + 2 * k;
+    return WideScale{pow2(k + 20), pow2(104 - k), (uint32_t)(e < 40 ? 40 : e)};
+}
+
 // Scratch and results of one build (library-owned, sized for n triangles).
 struct WideBuffers {
     void* base = nullptr;  // the one allocation that holds the rest

@@ -87,6 +87,7 @@ struct WideBuild {
     const uint32_t* order;
     const float* tris;
     const int32_t* mesh;
+    const uint32_t* bounds;  // the triangles' box (order-preserving ints)
     uint4* nodes;
     float4* wtris;
     uint32_t* ctr;
@@ -117,7 +118,7 @@ __device__ __forceinline__ uint32_t group_or(uint32_t v) {
 // nodes take their children's places with one atomic. Every lane of the wave
 // calls it; groups without a node pass valid = false.
 __device__ void wide_collapse(const WideBuild& w, uint32_t idx, bool valid, uint32_t next_start, uint32_t* next_ctr,
-                              uint4* stage) {
+                              uint32_t min_unit, uint4* stage) {
     const int lane = threadIdx.x & 63, g = lane >> 3, sl = lane & 7;
     const int n = w.n;
     uint4 it = make_uint4(0u, 0u, 0u, 0u);
@@ -218,14 +219,18 @@ __device__ void wide_collapse(const WideBuild& w, uint32_t idx, bool valid, uint
     const uint32_t child_base = next_start + base_n + (uint32_t)__popcll(innb & ((1ull << (lane & 56)) - 1ull));
     const uint32_t tri_base = base_t + tpre - ntri;
 
-    // the node's scale: the smallest power of two with the box inside 254 units
+    // the node's origin, a step of its coordinates (and the smallest unit)
+    // below the box, and its scale: the smallest power of two with the box
+    // inside 254 units
     uint32_t ex[3];
-    float isc[3];
-    const float ext[3] = {nb.b.x - nb.a.x, nb.b.y - nb.a.y, nb.b.z - nb.a.z};
+    float org[3], isc[3];
+    const float blo[3] = {nb.a.x, nb.a.y, nb.a.z}, bhi[3] = {nb.b.x, nb.b.y, nb.b.z};
+    const float least = __uint_as_float(min_unit << 23);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        uint32_t e = (__float_as_uint(fmx(ext[k], 0.f) * (1.0001f / 254.f)) >> 23) + 1u;
-        e = e < 40u ? 40u : (e > 230u ? 230u : e);  // (coordinates up to 2^40 are traced: 161 at most)
+        org[k] = blo[k] - fmx(fabsf(blo[k]) * 0x1p-23f, least);
+        uint32_t e = (__float_as_uint(fmx(bhi[k] - org[k], 0.f) * (1.0001f / 254.f)) >> 23) + 1u;
+        e = e < min_unit ? min_unit : (e > 230u ? 230u : e);  // (coordinates up to 2^40 are traced: 161 at most)
         ex[k] = e + kPlaneBits;
         isc[k] = __uint_as_float((254u - e) << 23);
     }
@@ -233,7 +238,7 @@ __device__ void wide_collapse(const WideBuild& w, uint32_t idx, bool valid, uint
     if (sl < 5) stage[g * 5 + sl] = make_uint4(0u, 0u, 0u, 0u);
     lds_sync();
     if (have) {
-        const float lo[3] = {ba.x, ba.y, ba.z}, hi[3] = {bb.x, bb.y, bb.z}, org[3] = {nb.a.x, nb.a.y, nb.a.z};
+        const float lo[3] = {ba.x, ba.y, ba.z}, hi[3] = {bb.x, bb.y, bb.z};
         // rounded outwards; the 1e-4 units cover the rounding of the two
         // operations (255 units times 2^-23 at most)
 #pragma unroll
@@ -248,9 +253,9 @@ __device__ void wide_collapse(const WideBuild& w, uint32_t idx, bool valid, uint
     }
     if (sl == 0) {
         uint32_t* hd = reinterpret_cast<uint32_t*>(mine);
-        hd[0] = __float_as_uint(nb.a.x);
-        hd[1] = __float_as_uint(nb.a.y);
-        hd[2] = __float_as_uint(nb.a.z);
+        hd[0] = __float_as_uint(org[0]);
+        hd[1] = __float_as_uint(org[1]);
+        hd[2] = __float_as_uint(org[2]);
         hd[3] = ex[0] | (ex[1] << 8) | (ex[2] << 16) | (imask << 24);
         hd[4] = child_base;
         hd[5] = tri_base;
@@ -275,6 +280,12 @@ __device__ void wide_collapse(const WideBuild& w, uint32_t idx, bool valid, uint
     }
 }
 
+__device__ __forceinline__ uint32_t min_unit_of(const uint32_t* bounds) {
+    float box[6];
+    for (int k = 0; k < 6; ++k) box[k] = ord2f(bounds[k]);
+    return wide_scale(box).min_unit;
+}
+
 __device__ __forceinline__ uint32_t ctr_load(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -287,6 +298,7 @@ __device__ __forceinline__ uint32_t ctr_load(const uint32_t* p) {
 __global__ __launch_bounds__(1024) void k_wide_levels(WideBuild w, int skip, uint32_t limit) {
     __shared__ uint4 stage[16][40];
     const int wave = threadIdx.x >> 6, g = (threadIdx.x & 63) >> 3;
+    const uint32_t min_unit = min_unit_of(w.bounds);
     int lvl = (int)ctr_load(w.ctr + kCtrTop) + skip;
     uint32_t start = 0;
     for (int k = 0; k < lvl; ++k) start += ctr_load(w.ctr + k);
@@ -295,7 +307,7 @@ __global__ __launch_bounds__(1024) void k_wide_levels(WideBuild w, int skip, uin
         if (cnt == 0u || cnt > limit) break;
         for (uint32_t b = 0; b < cnt; b += 128u) {
             const uint32_t i = b + (uint32_t)(wave * 8 + g);
-            wide_collapse(w, start + (i < cnt ? i : 0u), i < cnt, start + cnt, w.ctr + lvl + 1, stage[wave]);
+            wide_collapse(w, start + (i < cnt ? i : 0u), i < cnt, start + cnt, w.ctr + lvl + 1, min_unit, stage[wave]);
         }
         __syncthreads();
         start += cnt;
@@ -312,11 +324,11 @@ __global__ __launch_bounds__(kBlock) void k_wide_level(WideBuild w, int j) {
     if (lvl >= kMaxWideLevels) return;
     uint32_t start = 0;
     for (int k = 0; k < lvl; ++k) start += w.ctr[k];
-    const uint32_t cnt = w.ctr[lvl];
+    const uint32_t cnt = w.ctr[lvl], min_unit = min_unit_of(w.bounds);
     const uint32_t per = gridDim.x * (kBlock / 8);
     for (uint32_t b = blockIdx.x * (kBlock / 8) + (uint32_t)(wave * 8); b < cnt; b += per) {
         const uint32_t i = b + (uint32_t)g;
-        wide_collapse(w, start + (i < cnt ? i : 0u), i < cnt, start + cnt, w.ctr + lvl + 1, stage[wave]);
+        wide_collapse(w, start + (i < cnt ? i : 0u), i < cnt, start + cnt, w.ctr + lvl + 1, min_unit, stage[wave]);
     }
 }
 
@@ -381,7 +393,7 @@ hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, const float* tris, const i
     e = bottom_up_tree(ob.keys[ob.result], kCodeBits, tris, n, out, s, nullptr);
     if (e != hipSuccess) return e;
     mark(mk, "wide_tree");
-    const WideBuild wb{w.nbox, w.topo, order, tris, mesh, w.nodes, w.tris, w.ctr, n};
+    const WideBuild wb{w.nbox, w.topo, order, tris, mesh, bounds, w.nodes, w.tris, w.ctr, n};
     // up to 512 nodes per level in one workgroup; then a launch per level
     // until all but a skewed tree's last few nodes are done; then those
     const bool small = n <= 4096;

@@ -66,7 +66,6 @@ namespace {
 constexpr float kReach = 1.0f + 1.0f / 32.0f;
 constexpr float kOwnBox = 1.0f + 1.0f / 64.0f;  // a box starting further beyond its hit: the reference decides
 constexpr float kSlack = 1.0f / 1048576.0f;     // 2^-20
-constexpr float kFarthest = 1099511627776.f;    // 2^40: origins beyond go to the reference's traversal
 constexpr int kWideStack = 12;                  // stack entries in LDS
 constexpr int kWideDeep = 68;                   // entries in all: more than a tree over 32-bit codes has levels
 // Idle lanes a wave collects before it hands out rays: setting a ray up costs
@@ -80,35 +79,35 @@ __device__ __forceinline__ uint32_t near_planes(float inv) { return inv < 0.f ? 
 constexpr uint32_t kFarPlanes = 0x00020002u;
 
 // The ray as the node tests use it: direction scaled to a largest component
-// in [1, 2) (a power of two, exact), reciprocals bounded by 2^60 so that an
-// axis the ray runs along gives huge distances instead of infinities.
+// in [1, 2) (a power of two, exact), reciprocals bounded so that an axis the
+// ray runs along gives huge distances instead of infinities (WideScale).
 struct WideRay {
     v3 o, inv;
     float scale;  // true t * scale = t in the scaled direction
     uint32_t oct;
     uint32_t nx, ny, nz;  // selectors of the near planes (near_planes)
 };
-__device__ __forceinline__ float wide_rcp(float d) {
+__device__ __forceinline__ float wide_rcp(float d, float most) {
     const float r = __builtin_amdgcn_rcpf(d);
-    return __builtin_copysignf(fmn(fabsf(r), 1152921504606846976.f), d);
+    return __builtin_copysignf(fmn(fabsf(r), most), d);
 }
 enum RayKind {
     kRayFine,
-    kRayOdd,  // only the reference's traversal takes it: from beyond 2^40, or a direction near float's limits
+    kRayOdd,  // only the reference's traversal takes it: from far beyond the scene, or a direction near float's limits
     kRayDead  // hits nothing: a zero direction (every determinant is 0) or one that is not finite, or a NaN
               // origin (Moller-Trumbore's t is 0 or NaN for every finite triangle)
 };
-__device__ __forceinline__ RayKind wide_ray(v3 o, v3 d, WideRay& r) {
+__device__ __forceinline__ RayKind wide_ray(v3 o, v3 d, float farthest, float rcp_max, WideRay& r) {
     const float m = fmx(fabsf(d.x), fmx(fabsf(d.y), fabsf(d.z)));
     const uint32_t e = __float_as_uint(m) >> 23;
     const bool dead = !(fabsf(d.x) <= FLT_MAX && fabsf(d.y) <= FLT_MAX && fabsf(d.z) <= FLT_MAX) || m == 0.f ||
                       !(o.x == o.x && o.y == o.y && o.z == o.z);
-    const bool fine = fabsf(o.x) <= kFarthest && fabsf(o.y) <= kFarthest && fabsf(o.z) <= kFarthest && e >= 2u &&
+    const bool fine = fabsf(o.x) <= farthest && fabsf(o.y) <= farthest && fabsf(o.z) <= farthest && e >= 2u &&
                       e <= 252u;
     r.o = o;
     r.scale = __uint_as_float(e << 23);
     const float down = __uint_as_float((254u - e) << 23);
-    r.inv = mk3(wide_rcp(d.x * down), wide_rcp(d.y * down), wide_rcp(d.z * down));
+    r.inv = mk3(wide_rcp(d.x * down, rcp_max), wide_rcp(d.y * down, rcp_max), wide_rcp(d.z * down, rcp_max));
     r.nx = near_planes(r.inv.x); r.ny = near_planes(r.inv.y); r.nz = near_planes(r.inv.z);
     r.oct = (r.inv.x < 0.f ? 1u : 0u) | (r.inv.y < 0.f ? 2u : 0u) | (r.inv.z < 0.f ? 4u : 0u);
     return dead ? kRayDead : (fine ? kRayFine : kRayOdd);
@@ -287,7 +286,8 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                                                   const int32_t* __restrict__ dst, uint8_t* __restrict__ ovis,
                                                   uint32_t* __restrict__ overflow,
                                                   unsigned long long* __restrict__ next_ray,
-                                                  unsigned long long* __restrict__ fetched, WideList wl, int most) {
+                                                  unsigned long long* __restrict__ fetched, WideList wl,
+                                                  float farthest, float rcp_max, int most) {
     __shared__ WideStackLds<B> lds;
     const int lane = threadIdx.x & 63;
     const int64_t nrays = nrays_dev ? (int64_t)*nrays_dev : nrays_arg;
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                     if (ri >= 0) {
                         v3 o;
                         load_ray(rays, ri, o, d);
-                        const RayKind kind = wide_ray(o, d, r);
+                        const RayKind kind = wide_ray(o, d, farthest, rcp_max, r);
                         best = rival = FLT_MAX; bt = -1; bu = 0.f; bv = 0.f;
                         odd = kind == kRayOdd;
                         may_list = wl.after > 0;
@@ -653,7 +653,7 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
     v3 o, d;
     load_ray(A.rays, ri, o, d);
     WideRay r;
-    const RayKind kind = wide_ray(o, d, r);
+    const RayKind kind = wide_ray(o, d, A.w.far_origin, A.w.rcp_max, r);
     bool failed = kind == kRayOdd;
     bool bad = false;  // a walk up the reference's tree did not end
     const bool root_hit = slab(A.root[0], A.root[1], A.root[2], A.root[3], A.root[4], A.root[5], o,
@@ -813,7 +813,7 @@ __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const 
     v3 o, d;
     load_ray(A.rays, ri, o, d);
     WideRay r;
-    const RayKind kind = wide_ray(o, d, r);
+    const RayKind kind = wide_ray(o, d, A.w.far_origin, A.w.rcp_max, r);
     bool failed = kind == kRayOdd;
     const float lim = limit[ri];
     const bool use = !(lim == INFINITY);
@@ -943,7 +943,7 @@ void wide_closest(const TraceBvh& bvh, const float* rays, int64_t nrays, const u
     launch_wide_block<false>(L, nrays, ls, bvh.wide.nodes, bvh.wide.tris, rays, nrays, nrays_dev, prim, t, u, v,
                              (const float*)nullptr, (const int32_t*)nullptr, (const int32_t*)nullptr,
                              (uint8_t*)nullptr, counters, reinterpret_cast<unsigned long long*>(counters + 2),
-                             fetch_word(counters, true), wl);
+                             fetch_word(counters, true), wl, bvh.wide.far_origin, bvh.wide.rcp_max);
     const FinishArgs A{bvh.wide, bvh.rec, bvh.root, rays, nrays, nrays_dev, coop.longs, counters + 26,
                        coop.long_cap, counters + 30, counters, fetch_word(counters, true), bvh.ntris};
     const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks, nrays);
@@ -960,7 +960,7 @@ void wide_occluded(const TraceBvh& bvh, const float* rays, int64_t nrays, const 
     launch_wide_block<true>(L, nrays, ls, bvh.wide.nodes, bvh.wide.tris, rays, nrays, nrays_dev, (int32_t*)nullptr,
                             (float*)nullptr, (float*)nullptr, (float*)nullptr, limit, src, dst, visible,
                             counters + 1, reinterpret_cast<unsigned long long*>(counters + 4),
-                            fetch_word(counters, false), wl);
+                            fetch_word(counters, false), wl, bvh.wide.far_origin, bvh.wide.rcp_max);
     const FinishArgs A{bvh.wide, bvh.rec, bvh.root, rays, nrays, nrays_dev, ids, counters + 20,
                        coop.spill_cap, counters + 22, counters + 1, fetch_word(counters, false), bvh.ntris};
     const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks, nrays);

@@ -395,7 +395,9 @@ int cav_scene_create_from_pbrt(cav_ctx* ctx, const char* path, const cav_pbrt_ov
  * they walk the reference's own tree in its visiting order when the hand-off
  * is 1<<30 (closest-hit, any-hit), any_hit_step is CAV_ANY_STEP_PAIR or
  * any_hit_whole_line is 1 (any-hit), when that tree is more than 64 levels
- * deep, a coordinate is beyond 2^40, or there was no memory for the wide tree.
+ * deep, a coordinate is beyond 2^40, or there was no memory for the wide tree;
+ * so do single rays that start more than 2^20 times the scene's largest
+ * coordinate from 0 or whose direction is close to the limits of a float.
  * Workgroups per CU (0: as many as fit; reference's tree only), rays a wave takes from the dispenser at a time
  * (64..65536), traversal-stack entries kept in LDS (32 or 48; the rest of
  * the reference's 64 in scratch) and threads per traversal workgroup (64,

@@ -156,3 +156,45 @@ def test_rebuild_reuses_the_tree(ctx):
         rays = scenes.random_rays(20000, seed=50 + k, lo=0.0, hi=1.0)
         lim = scenes.shadow_limits(len(rays), seed=60 + k)
         _check(bvh, nd, tris, rays, lim, f"rebuild {k}")
+
+
+def _floor(k, size, axis=2, noise=0.0, seed=0):
+    """k x k cells of two triangles each, side `size`, flat on `axis` but for
+    noise of that size in its coordinate."""
+    rng = np.random.default_rng(seed)
+    g = np.linspace(0, size, k + 1)
+    x, y = np.meshgrid(g, g, indexing="ij")
+    p = np.stack([x, y, noise * rng.uniform(-1, 1, x.shape)], -1)
+    a, b, c, d = p[:-1, :-1], p[1:, :-1], p[1:, 1:], p[:-1, 1:]
+    t = np.concatenate([np.stack(q, 2).reshape(-1, 3, 3) for q in ((a, b, c), (a, c, d))])
+    return np.roll(t, axis - 2, axis=2)
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("size", [2e-3, 1.0, 4000.0])
+@pytest.mark.parametrize("noise", [0.0, 1e-17])
+def test_rays_almost_along_flat_boxes(ctx, axis, size, noise):
+    """Rays 1e-22 to 1e-9 of a floor's size above (below) it that sink to it
+    (rise to it) over distances of its size: directions whose one component is
+    far below the others, along boxes without extent on that axis. With noise,
+    rays between the floor's lowest and highest vertex that do not move along
+    its axis at all too."""
+    rng = np.random.default_rng(int(axis + size) + (noise > 0))
+    tris = np.ascontiguousarray(_floor(12, size, axis, noise * size).reshape(-1, 9), np.float32)
+    n = 6000
+    ang = rng.uniform(0, 2 * np.pi, n)
+    h = size * 10.0 ** rng.uniform(-22, -9, n) * rng.choice([-1, 1], n)
+    far = size * rng.uniform(0.05, 0.9, n)
+    o = np.stack([*(rng.uniform(0, size, (2, n))), h], -1)
+    d = np.stack([np.cos(ang), np.sin(ang), -h / far], -1)
+    d[::3, 0] = 0.0
+    if noise:
+        o[::2, 2] = size * noise * rng.uniform(-0.9, 0.9, len(o[::2]))
+        d[::2, 2] = rng.choice([0.0, -0.0], len(o[::2]))
+    o, d = np.roll(o, axis - 2, 1), np.roll(d, axis - 2, 1)
+    rays = np.ascontiguousarray(np.concatenate([o, d], 1), np.float32)
+    lim = (size * rng.uniform(0, 2, n)).astype(np.float32)
+    lim[::4] = np.inf
+    bvh, nd = _tree(ctx, tris, 30, 0)
+    ref = _check(bvh, nd, tris, rays, lim, f"axis {axis}, size {size}, noise {noise}")
+    assert (ref["prim"] >= 0).sum() > 200
