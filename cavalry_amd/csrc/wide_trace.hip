@@ -321,7 +321,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                     bool touch;
                     const float e = leaf_entry(a, b, c, r.o, d, touch);
                     ask = ask || touch || !(e >= 0.f);
-                    if (!kAny) ask = ask || rival <= fmx(best, e) || e > best * kOwnBox;
+                    if (!kAny) ask = ask || rival <= fmx(best, e) || e > best * kOwnBox || !(best < FLT_MAX);
                 }
                 if (kAny) {
                     ovis[ri] = prim >= 0 ? 0 : 1;
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                 }
             } else if (wide_tri_hit(a, b, c, r.o, d, t, u, v)) {
                 rival = fmn(rival, fmx(t, best));
-                if (t < best) {
+                if (bt < 0 || t < best) {  // (the first hit counts at any distance, infinity included)
                     best = t; bu = u; bv = v; bt = (int)(tbase + k);
                     cut = t * kReach * r.scale;
                 }
@@ -655,7 +655,8 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
     WideRay r;
     const RayKind kind = wide_ray(o, d, A.w.far_origin, A.w.rcp_max, r);
     bool failed = kind == kRayOdd;
-    bool bad = false;  // a walk up the reference's tree did not end
+    bool bad = false;      // a walk up the reference's tree did not end
+    bool endless = false;  // a hit at a distance that overflowed (counts where there is no other)
     const bool root_hit = slab(A.root[0], A.root[1], A.root[2], A.root[3], A.root[4], A.root[5], o,
                                div3(mk3(1.f, 1.f, 1.f), d)) >= 0.f;
     float best = FLT_MAX;
@@ -687,9 +688,11 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
                 if (wide_tri_hit(a, b, c, o, d, t, u, v)) {
                     bool touch;
                     e = leaf_entry(a, b, c, o, d, touch);
-                    hit = e >= 0.f && t < FLT_MAX && e < FLT_MAX;
+                    hit = e >= 0.f && e < FLT_MAX;
                     p = __float_as_int(a.w);
                     if (hit && touch) hit = root_hit && reached(A.w, p, o, d, bad);
+                    endless = endless || (hit && !(t < FLT_MAX));
+                    hit = hit && t < FLT_MAX;
                 }
             }
             float m = hit ? t : FLT_MAX;
@@ -733,7 +736,7 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
         wave_fence();
     }
     wave_fence();
-    if (__ballot(bad)) failed = true;
+    if (__ballot(bad) || (nc == 0 && __ballot(endless))) failed = true;
     int win = -1;
     if (!failed && nc > 0) {
         // the hits whose order could matter: at or before the farthest of

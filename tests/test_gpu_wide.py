@@ -198,3 +198,18 @@ def test_rays_almost_along_flat_boxes(ctx, axis, size, noise):
     bvh, nd = _tree(ctx, tris, 30, 0)
     ref = _check(bvh, nd, tris, rays, lim, f"axis {axis}, size {size}, noise {noise}")
     assert (ref["prim"] >= 0).sum() > 200
+
+
+@pytest.mark.parametrize("size,length", [(1.0, 1e-38), (1.0, 2.4e-38), (1.0, 1e-36), (1e12, 1e-27), (1e10, 1e-30)])
+def test_distances_near_the_limits_of_a_float(ctx, size, length):
+    """Scenes and directions whose hits lie at distances up to infinity (the
+    reference takes the first hit whatever its distance)."""
+    tris = (scenes.gmm_triangles(700, seed=13, edge=0.4) * np.float32(size)).astype(np.float32)
+    rays = scenes.random_rays(6000, seed=14, lo=0.2, hi=0.8)
+    rays[:, :3] *= np.float32(size)
+    rays[:, 3:] = (rays[:, 3:] * length).astype(np.float32)
+    rays[::2, 4:] = 0.0
+    lim = np.full(len(rays), np.inf, np.float32)
+    lim[::3] = np.float32(size / length * 0.3) if size / length < 1e38 else np.float32(3e38)
+    bvh, nd = _tree(ctx, tris, 30, 0)
+    _check(bvh, nd, tris, rays, lim, f"size {size}, directions of {length}")
