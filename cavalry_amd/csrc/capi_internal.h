@@ -53,7 +53,7 @@ inline TraceBvh bvh_trace(const cav_bvh* h) {
     TraceBvh t{h->rec, h->n, h->root, WideDev{}};
     if (h->wide_ok)
         t.wide = WideDev{h->wide.nodes, h->wide.tris, h->b.nbox, h->b.topo, h->wide.leaf_of, h->wide_scale.far_origin,
-                         h->wide_scale.rcp_max};
+                         h->wide_scale.rcp_max, h->wide_scale.near_slack};
     return t;
 }
 // frees context-owned state of other subsystems before the stream goes away

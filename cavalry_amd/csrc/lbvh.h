@@ -183,6 +183,7 @@ struct WideDev {
     const int32_t* leaf_of = nullptr;
     float far_origin = 0.f;  // WideScale of the scene
     float rcp_max = 0.f;
+    float near_slack = 0.f;
 };
 // A flattened BVH of ntris triangles with its wide tree, if it has one.
 struct TraceBvh {

@@ -41,6 +41,7 @@ inline int64_t wide_node_capacity(int64_t n) { return 2 * n / 7 + 16; }
 struct WideScale {
     float far_origin;   // rays from beyond go to the reference's traversal
     float rcp_max;
+    float near_slack;   // 2^(k - 16): how far beyond the nearest hit boxes are always visited (scaled directions)
     uint32_t min_unit;  // exponent (biased by 127) of the smallest unit, 2^(2k - 67)
 };
 __host__ __device__ inline WideScale wide_scale(const float* box6) {
@@ -50,7 +51,7 @@ __host__ __device__ inline WideScale wide_scale(const float* box6) {
     k = k < -20 ? -20 : (k > 40 ? 40 : k);
     const auto pow2 = [](int e) { return __builtin_bit_cast(float, (uint32_t)(e + 127) << 23); };
     const int e = 60 + 2 * k;
-    return WideScale{pow2(k + 20), pow2(104 - k), (uint32_t)(e < 40 ? 40 : e)};
+    return WideScale{pow2(k + 20), pow2(104 - k), pow2(k - 16), (uint32_t)(e < 40 ? 40 : e)};
 }
 
 // Scratch and results of one build (library-owned, sized for n triangles).

@@ -31,11 +31,21 @@
 // The wide boxes only have to contain the exact ones. They are rounded
 // outwards, their planes' distances carry a slack of 2^-20 of their terms
 // (the two roundings are 2^-23 each), and boxes are skipped only beyond
-// kReach = 1 + 2^-5 times the nearest hit (any-hit: times the limit). A
-// triangle beyond that could matter only if Moller-Trumbore put its t more
-// than 2^-6 (relative) short of the start of its own box: the same
-// assumption, with a margin 16 times wider, that the cooperative passes over
-// the reference's tree make (traverse.hip).
+// kReach = 1 + 2^-5 times the nearest hit (any-hit: times the limit) and a
+// slack of 2^-16 of the scene's largest coordinate. A triangle beyond that
+// could matter only if Moller-Trumbore put its t about as far short of the
+// start of its own box (the assumption, with a margin 16 times wider, that
+// the cooperative passes over the reference's tree make, traverse.hip). It does where its determinant is
+// little more than rounding: a triangle met edge on, a needle, products near
+// the smallest floats. Such a triangle rarely comes alone -- a ray in the
+// plane of a tessellated floor meets dozens -- so a closest-hit ray that
+// tests one (thin_test), or whose nearest hit is one (thin_hit), goes to the
+// finishing pass, which then walks the ray's whole line without skipping any
+// box: its answer assumes nothing about distances. On a model of rays in the
+// plane of turned floors with walls (460,000 rays, 50 seeds), no answer was
+// wrong down to an eighth of thin_test's limit; what remains open is a ray
+// whose only thin triangles all lie behind its nearest hit. Random rays go
+// that way once in 10,000 (interiors, soups of 20,000 triangles).
 //
 // Per node and lane: five 16-byte loads from one line and about 190 VALU
 // instructions for eight children, against four loads and 90 instructions
@@ -66,6 +76,10 @@ namespace {
 constexpr float kReach = 1.0f + 1.0f / 32.0f;
 constexpr float kOwnBox = 1.0f + 1.0f / 64.0f;  // a box starting further beyond its hit: the reference decides
 constexpr float kSlack = 1.0f / 1048576.0f;     // 2^-20
+// Limits of a determinant against the sizes of its factors:
+constexpr float kThinTest = 0x1p-16f;  // of a tested triangle (largest components)
+constexpr float kThinHit = 0x1p-20f;   // of a hit: the error of its t against what boxes are visited beyond it
+constexpr float kTiny = 0x1p-100f;     // below: products in the triangle test may have lost bits to underflow
 constexpr int kWideStack = 12;                  // stack entries in LDS
 constexpr int kWideDeep = 68;                   // entries in all: more than a tree over 32-bit codes has levels
 // Idle lanes a wave collects before it hands out rays: setting a ray up costs
@@ -196,13 +210,40 @@ __device__ __forceinline__ float leaf_entry(const float4& a, const float4& b, co
     touch = grazes(inv.x, o.x, lo.x, hi.x) || grazes(inv.y, o.y, lo.y, hi.y) || grazes(inv.z, o.z, lo.z, hi.z);
     return slab(lo.x, lo.y, lo.z, hi.x, hi.y, hi.z, o, inv);
 }
+__device__ __forceinline__ TTri edges(const float4& a, const float4& b, const float4& c) {
+    return TTri{a, make_float4(b.x - a.x, b.y - a.y, b.z - a.z, 0.f), make_float4(c.x - a.x, c.y - a.y, c.z - a.z, 0.f)};
+}
 __device__ __forceinline__ bool wide_tri_hit(const float4& a, const float4& b, const float4& c, v3 o, v3 d, float& t,
                                              float& u, float& v) {
-    TTri tr;
-    tr.a = a;
-    tr.b = make_float4(b.x - a.x, b.y - a.y, b.z - a.z, 0.f);
-    tr.c = make_float4(c.x - a.x, c.y - a.y, c.z - a.z, 0.f);
-    return tri_hit(tr, o, d, t, u, v);
+    return tri_hit(edges(a, b, c), o, d, t, u, v);
+}
+__device__ __forceinline__ float det_of(const TTri& tr, v3 d) {
+    return dot3(mk3(tr.b.x, tr.b.y, tr.b.z), cross3(d, mk3(tr.c.x, tr.c.y, tr.c.z)));
+}
+__device__ __forceinline__ float size_of(v3 v) { return fabsf(v.x) + fabsf(v.y) + fabsf(v.z); }
+__device__ __forceinline__ float sizes_of(const TTri& tr) {
+    return size_of(mk3(tr.b.x, tr.b.y, tr.b.z)) * size_of(mk3(tr.c.x, tr.c.y, tr.c.z));
+}
+// Whether a triangle's determinant is too small to trust its t (0: never a hit).
+__device__ __forceinline__ bool thin_test(const float4& a, const float4& b, const float4& c, v3 d, float scale) {
+    const TTri tr = edges(a, b, c);
+    const float det = det_of(tr, d);
+    const float m1 = fmx(fabsf(tr.b.x), fmx(fabsf(tr.b.y), fabsf(tr.b.z)));
+    const float m2 = fmx(fabsf(tr.c.x), fmx(fabsf(tr.c.y), fabsf(tr.c.z)));
+    return det != 0.f && fabsf(det) < fmx(m1 * m2 * (scale * kThinTest), kTiny);
+}
+// The same for a hit at t, its numerator looked at too: whether t is off by
+// more than a good part of `past`, the distance beyond it that boxes are visited to.
+__device__ __forceinline__ bool thin_hit(const float4& a, const float4& b, const float4& c, v3 o, v3 d, float t,
+                                         float past) {
+    const TTri tr = edges(a, b, c);
+    const float num = fabsf(det_of(tr, d)) * past;
+    const float err = sizes_of(tr) * (size_of(d) * t + size_of(sub3(o, mk3(a.x, a.y, a.z)))) * kThinHit;
+    return !(err <= num) || num < kTiny;
+}
+// 1 / r.scale, the distance in true units of one in scaled ones
+__device__ __forceinline__ float unscale(const WideRay& r) {
+    return __uint_as_float((254u - (__float_as_uint(r.scale) >> 23)) << 23);
 }
 
 // A wave's next rays for the lanes that need one (wave-uniform control flow).
@@ -287,7 +328,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                                                   uint32_t* __restrict__ overflow,
                                                   unsigned long long* __restrict__ next_ray,
                                                   unsigned long long* __restrict__ fetched, WideList wl,
-                                                  float farthest, float rcp_max, int most) {
+                                                  float farthest, float rcp_max, float slack, int most) {
     __shared__ WideStackLds<B> lds;
     const int lane = threadIdx.x & 63;
     const int64_t nrays = nrays_dev ? (int64_t)*nrays_dev : nrays_arg;
@@ -301,6 +342,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
     float best = FLT_MAX, rival = FLT_MAX, bu = 0.f, bv = 0.f, cut = 0.f;  // rival: the second nearest hit
     int bt = -1, sm = -1, dm = -1, steps = 0;  // bt: the nearest hit's triangle record
     bool odd = false, over = false, may_list = false, drained = false;  // over: traversed, result still to be written
+    bool thin = false;  // has tested a triangle whose t is not to be trusted
     uint32_t cbase = 0, group = 0;  // the current node's inner children: first one, slot mask << 8 | bits to visit
     uint32_t tbase = 0, tbits = 0;  // triangles to test
     int sp = 0, maxsp = 0;
@@ -321,7 +363,11 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                     bool touch;
                     const float e = leaf_entry(a, b, c, r.o, d, touch);
                     ask = ask || touch || !(e >= 0.f);
-                    if (!kAny) ask = ask || rival <= fmx(best, e) || e > best * kOwnBox || !(best < FLT_MAX);
+                    if (!kAny) {
+                        const float near = slack * unscale(r);
+                        ask = ask || rival <= fmx(best, e) || e > best * kOwnBox + 0.5f * near || !(best < FLT_MAX) ||
+                              thin || thin_hit(a, b, c, r.o, d, best, best * (kReach - 1.f) + near);
+                    }
                 }
                 if (kAny) {
                     ovis[ri] = prim >= 0 ? 0 : 1;
@@ -351,6 +397,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                         const RayKind kind = wide_ray(o, d, farthest, rcp_max, r);
                         best = rival = FLT_MAX; bt = -1; bu = 0.f; bv = 0.f;
                         odd = kind == kRayOdd;
+                        thin = false;
                         may_list = wl.after > 0;
                         steps = 0; sp = 0; tbits = 0;
                         cbase = 0;
@@ -359,7 +406,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                         if (kAny) {
                             best = limit[ri];
                             const bool use = !(best == INFINITY);
-                            if (use) cut = best * kReach * r.scale;
+                            if (use) cut = __builtin_fmaf(best * r.scale, kReach, slack);
                             if (use && !(best > 0.f)) group = 0;  // nothing lies before it
                             sm = src ? src[ri] : -1;
                             dm = dst ? dst[ri] : -1;
@@ -442,11 +489,14 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                     bt = (int)(tbase + k);
                     done = true;
                 }
-            } else if (wide_tri_hit(a, b, c, r.o, d, t, u, v)) {
-                rival = fmn(rival, fmx(t, best));
-                if (bt < 0 || t < best) {  // (the first hit counts at any distance, infinity included)
-                    best = t; bu = u; bv = v; bt = (int)(tbase + k);
-                    cut = t * kReach * r.scale;
+            } else {
+                thin = thin || thin_test(a, b, c, d, r.scale);
+                if (wide_tri_hit(a, b, c, r.o, d, t, u, v)) {
+                    rival = fmn(rival, fmx(t, best));
+                    if (bt < 0 || t < best) {  // (the first hit counts at any distance, infinity included)
+                        best = t; bu = u; bv = v; bt = (int)(tbase + k);
+                        cut = __builtin_fmaf(t * r.scale, kReach, slack);
+                    }
                 }
             }
         }
@@ -468,12 +518,21 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
 // ------------------------------------------------------------- finishing pass
 // One wave per listed ray, from the wide tree's root: pending nodes in LDS,
 // eight at a time, one child per lane. Closest-hit collects every hit within
-// kReach of the nearest (64 at most) and, when several lie close enough for
+// reach of the nearest (64 at most) and, when several lie close enough for
 // the reference's order to decide, replays that order; any-hit stops at the
-// first blocker. A ray that does not fit goes through the reference's tree on
-// one lane of the wave.
+// first blocker. A closest-hit ray that meets a thin triangle is left to the
+// whole workgroup, which collects every hit on its line. A ray that does not
+// fit goes through the reference's tree on one lane of the wave.
+//
+// Few rays go over their whole line (5 of 2M camera rays, 86 of 1M random
+// ones), but one holds up the launch: by one wave it took 130 us in an
+// interior and 190 in a soup of 0.5M triangles, a microsecond for each eight
+// nodes.
 constexpr int kPend = 1024;
 constexpr int kCands = 64;
+constexpr int kFinishWaves = 8;       // closest-hit: waves of a workgroup
+constexpr int kFinishTurn = 16;       // rays a wave takes before the workgroup's whole lines
+constexpr int kWholePend = 4096, kWholeCands = 512;
 constexpr int kRefStack = 64;  // BVH/BVH.h:41,122
 
 __device__ __forceinline__ void wave_fence() {
@@ -596,6 +655,13 @@ struct FinishLds {
     int32_t p[kCands];
     int stack[kRefStack];
 };
+struct WholeLds {
+    uint32_t pend[kWholePend];
+    float t[kWholeCands], u[kWholeCands], v[kWholeCands], e[kWholeCands];
+    int32_t p[kWholeCands];
+    int stack[kRefStack];
+    uint32_t npend, ncands, bad, endless;
+};
 
 // A lane's child of a pending node: its wide box against the ray. Returns the
 // slot byte's meaning: inner child index (inner set) or first triangle and
@@ -605,6 +671,12 @@ __device__ __forceinline__ void lane_child(const uint4* nd, int slot, const Wide
     const uint4 w0 = nd[0], w1 = nd[1];
     const uint8_t* by = reinterpret_cast<const uint8_t*>(nd);
     const uint32_t m = by[24 + slot];
+    uint32_t plane[6];  // (all loads before the first branch)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        plane[2 * k] = by[wide_plane(k, slot)];
+        plane[2 * k + 1] = by[wide_plane(k, slot) + 2];
+    }
     inner = false;
     at = 0;
     count = 0;
@@ -616,7 +688,7 @@ __device__ __forceinline__ void lane_child(const uint4* nd, int slot, const Wide
     for (int k = 0; k < 3; ++k) {
         const AxisPlanes ap = axis_planes(org[k], (w0.w >> (8 * k)) & 255u, ro[k], ri[k]);
         constexpr float kByte = 1.f / (float)(1 << kPlaneBits);
-        const float lo = (float)by[wide_plane(k, slot)] * kByte, hi = (float)by[wide_plane(k, slot) + 2] * kByte;
+        const float lo = (float)plane[2 * k] * kByte, hi = (float)plane[2 * k + 1] * kByte;
         tn = fmx(tn, __builtin_fmaf(ri[k] < 0.f ? hi : lo, ap.an, ap.bn));
         tf = fmn(tf, __builtin_fmaf(ri[k] < 0.f ? lo : hi, ap.af, ap.bf));
     }
@@ -647,9 +719,81 @@ struct FinishArgs {
     int ntris;
 };
 
-__device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, int32_t* oprim, float* ot, float* ou,
-                               float* ov, uint64_t& nfetch) {
-    const int lane = threadIdx.x;
+// Which of the hits of a wave's lanes (rival, two or more) the reference's
+// traversal ends with: its order among them, one lane each. A hit is skipped
+// when its path, below the box that was pending before an earlier hit was
+// met, starts at or beyond that hit. -1: a walk up the tree did not end.
+__device__ int replay(const WideDev& w, v3 o, v3 d, bool rival, float ct, float ce, int prim) {
+    const int lane = threadIdx.x & 63;
+    const v3 inv = div3(mk3(1.f, 1.f, 1.f), d);
+    uint64_t path = ~0ull;
+    int depth = 0;
+    bool reach;
+    const bool ok = !rival || leaf_path(w, w.leaf_of[prim], o, inv, path, depth, reach);
+    if (__ballot(!ok)) return -1;
+    float near = FLT_MAX;
+    bool visited = false;
+    int win = -1;
+    for (uint64_t left = __ballot(rival); left != 0ull;) {
+        uint64_t first = (left >> lane) & 1ull ? path : ~0ull;
+#pragma unroll
+        for (int dd = 32; dd >= 1; dd >>= 1) {
+            const uint64_t other = (uint64_t)__shfl_xor((unsigned long long)first, dd, 64);
+            first = other < first ? other : first;
+        }
+        const uint64_t at = __ballot(((left >> lane) & 1ull) && path == first);
+        const int c = __ffsll((long long)at) - 1;
+        left &= ~(1ull << c);
+        const float ec = __shfl(ce, c, 64), tc = __shfl(ct, c, 64);
+        const int dc = __shfl(depth, c, 64);
+        const bool skips = visited && ec >= ct && dc > __clzll((long long)(path ^ first)) + 1;
+        if (__ballot(skips)) continue;
+        if (lane == c) visited = true;
+        if (tc < near) {
+            near = tc;
+            win = c;
+        }
+    }
+    return win;
+}
+__device__ __forceinline__ float wave_min(float v) {
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) v = fmn(v, __shfl_xor(v, dd, 64));
+    return v;
+}
+__device__ __forceinline__ float wave_max(float v) {
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) v = fmx(v, __shfl_xor(v, dd, 64));
+    return v;
+}
+
+struct ClosestOut {
+    int32_t* prim;
+    float *t, *u, *v;
+};
+__device__ void write_hit(const ClosestOut& out, int64_t ri, int prim, float t, float u, float v) {
+    out.prim[ri] = prim;
+    out.t[ri] = t;
+    if (out.u) out.u[ri] = u;
+    if (out.v) out.v[ri] = v;
+}
+// One lane: the ray over the reference's tree.
+__device__ void reference_ray(const FinishArgs& A, int64_t ri, v3 o, v3 d, int* stack, const ClosestOut& out) {
+    uint32_t ovf = 0;
+    int prim;
+    float t, u, v;
+    reference_closest(A.recs, A.root, o, d, 2 * A.ntris - 1, stack, prim, t, u, v, ovf);
+    if (ovf) atomicAdd(A.overflow, ovf);
+    atomicAdd(A.fails, 1u);
+    write_hit(out, ri, prim, t, u, v);
+}
+__device__ __forceinline__ bool root_hit(const FinishArgs& A, v3 o, v3 d) {
+    return slab(A.root[0], A.root[1], A.root[2], A.root[3], A.root[4], A.root[5], o, div3(mk3(1.f, 1.f, 1.f), d)) >= 0.f;
+}
+
+// A ray by a wave. false: it has to be taken over its whole line.
+__device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, const ClosestOut& out, uint64_t& nfetch) {
+    const int lane = threadIdx.x & 63;
     v3 o, d;
     load_ray(A.rays, ri, o, d);
     WideRay r;
@@ -657,8 +801,9 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
     bool failed = kind == kRayOdd;
     bool bad = false;      // a walk up the reference's tree did not end
     bool endless = false;  // a hit at a distance that overflowed (counts where there is no other)
-    const bool root_hit = slab(A.root[0], A.root[1], A.root[2], A.root[3], A.root[4], A.root[5], o,
-                               div3(mk3(1.f, 1.f, 1.f), d)) >= 0.f;
+    bool thin = false;
+    const bool in_root = root_hit(A, o, d);
+    const float near = A.w.near_slack * unscale(r);
     float best = FLT_MAX;
     int count = kind == kRayFine ? 1 : 0, nc = 0;
     if (lane == 0) L.pend[0] = 0u;
@@ -671,7 +816,7 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
         int nt = 0;
         if (g < k) {
             const uint32_t node = L.pend[count - 1 - g];
-            const float cut = best == FLT_MAX ? FLT_MAX : best * kReach * r.scale;
+            const float cut = best == FLT_MAX ? FLT_MAX : __builtin_fmaf(best * r.scale, kReach, A.w.near_slack);
             lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, cut, inner, at, nt);
             nfetch += (lane & 7) == 0 ? 1u : 0u;
         }
@@ -685,21 +830,20 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
                 const float4* tp = A.w.tris + (int64_t)(at + (uint32_t)j) * 3;
                 const float4 a = tp[0], b = tp[1], c = tp[2];
                 ++nfetch;
+                thin = thin || thin_test(a, b, c, d, r.scale);
                 if (wide_tri_hit(a, b, c, o, d, t, u, v)) {
+                    thin = thin || thin_hit(a, b, c, o, d, t, t * (kReach - 1.f) + near);
                     bool touch;
                     e = leaf_entry(a, b, c, o, d, touch);
                     hit = e >= 0.f && e < FLT_MAX;
                     p = __float_as_int(a.w);
-                    if (hit && touch) hit = root_hit && reached(A.w, p, o, d, bad);
+                    if (hit && touch) hit = in_root && reached(A.w, p, o, d, bad);
                     endless = endless || (hit && !(t < FLT_MAX));
                     hit = hit && t < FLT_MAX;
                 }
             }
-            float m = hit ? t : FLT_MAX;
-#pragma unroll
-            for (int dd = 32; dd >= 1; dd >>= 1) m = fmn(m, __shfl_xor(m, dd, 64));
-            best = fmn(best, m);
-            const bool add = hit && t <= best * kReach;
+            best = fmn(best, wave_min(hit ? t : FLT_MAX));
+            const bool add = hit && t <= best * kReach + near;
             const uint64_t am = __ballot(add);
             if (am == 0ull) continue;
             const int na = __popcll(am);
@@ -707,7 +851,7 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
             if (nc + na > kCands) {  // keep those still near the nearest
                 const float ct = L.t[lane], cu = L.u[lane], cv = L.v[lane], ce = L.e[lane];
                 const int cp = L.p[lane];
-                const bool keep = lane < nc && ct <= best * kReach;
+                const bool keep = lane < nc && ct <= best * kReach + near;
                 const uint64_t km = __ballot(keep);
                 wave_fence();
                 if (keep) {
@@ -730,12 +874,13 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
         const uint64_t im = __ballot(inner);
         const int ni = __popcll(im);
         if (count + ni > kPend) failed = true;
-        if (failed) break;
+        if (failed || __ballot(thin)) break;
         if (inner) L.pend[count + __popcll(im & ((1ull << lane) - 1ull))] = at;
         count += ni;
         wave_fence();
     }
     wave_fence();
+    if (!failed && __ballot(thin)) return false;
     if (__ballot(bad) || (nc == 0 && __ballot(endless))) failed = true;
     int win = -1;
     if (!failed && nc > 0) {
@@ -743,71 +888,137 @@ __device__ void finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, in
         // their own boxes' starts
         const float ct = lane < nc ? L.t[lane] : FLT_MAX, ce = lane < nc ? L.e[lane] : 0.f;
         float bound = best;
-        bool grew = true;
-        while (grew) {
-            float m = ct <= bound ? fmx(ct, ce) : 0.f;
-#pragma unroll
-            for (int dd = 32; dd >= 1; dd >>= 1) m = fmx(m, __shfl_xor(m, dd, 64));
+        for (bool grew = true; grew;) {
+            const float m = wave_max(ct <= bound ? fmx(ct, ce) : 0.f);
             grew = m > bound;
             if (grew) bound = m;
         }
+        if (bound > best * kOwnBox + 0.5f * near) return false;
         const bool rival = ct <= bound;
         const uint64_t rm = __ballot(rival);
-        if (bound > best * kOwnBox) {
-            failed = true;
-        } else if (__popcll(rm) == 1) {
-            win = __ffsll((long long)rm) - 1;
-        } else {
-            // Replay the reference's order among them, one lane each. A hit is
-            // skipped when its path, below the box that was pending before an
-            // earlier hit was met, starts at or beyond that hit.
-            const v3 inv = div3(mk3(1.f, 1.f, 1.f), d);
-            uint64_t path = ~0ull;
-            int depth = 0;
-            bool reach;
-            const bool ok = !rival || leaf_path(A.w, A.w.leaf_of[L.p[lane]], o, inv, path, depth, reach);
-            if (__ballot(!ok)) failed = true;
-            float near = FLT_MAX;
-            bool visited = false;
-            for (uint64_t left = rm; left != 0ull && !failed;) {
-                uint64_t first = (left >> lane) & 1ull ? path : ~0ull;
-#pragma unroll
-                for (int dd = 32; dd >= 1; dd >>= 1) {
-                    const uint64_t other = (uint64_t)__shfl_xor((unsigned long long)first, dd, 64);
-                    first = other < first ? other : first;
-                }
-                const uint64_t at = __ballot(((left >> lane) & 1ull) && path == first);
-                const int c = __ffsll((long long)at) - 1;
-                left &= ~(1ull << c);
-                const float ec = __shfl(ce, c, 64), tc = __shfl(ct, c, 64);
-                const int dc = __shfl(depth, c, 64);
-                const bool skips = visited && ec >= ct && dc > __clzll((long long)(path ^ first)) + 1;
-                if (__ballot(skips)) continue;
-                if (lane == c) visited = true;
-                if (tc < near) {
-                    near = tc;
-                    win = c;
-                }
-            }
-        }
+        win = __popcll(rm) == 1 ? __ffsll((long long)rm) - 1 : replay(A.w, o, d, rival, ct, ce, rival ? L.p[lane] : 0);
+        if (win < 0) failed = true;
     }
     if (lane == 0) {
-        int prim = -1;
-        float t = 0.f, u = 0.f, v = 0.f;
-        if (failed) {
-            uint32_t ovf = 0;
-            reference_closest(A.recs, A.root, o, d, 2 * A.ntris - 1, L.stack, prim, t, u, v, ovf);
-            if (ovf) atomicAdd(A.overflow, ovf);
-            atomicAdd(A.fails, 1u);
-        } else if (win >= 0) {
-            prim = L.p[win]; t = L.t[win]; u = L.u[win]; v = L.v[win];
-        }
-        oprim[ri] = prim;
-        ot[ri] = t;
-        if (ou) ou[ri] = u;
-        if (ov) ov[ri] = v;
+        if (failed) reference_ray(A, ri, o, d, L.stack, out);
+        else if (win >= 0) write_hit(out, ri, L.p[win], L.t[win], L.u[win], L.v[win]);
+        else write_hit(out, ri, -1, 0.f, 0.f, 0.f);
     }
     wave_fence();
+    return true;
+}
+
+// A ray over its whole line by all waves of the workgroup, 64 nodes at a
+// time: no box of the line is skipped, so that the answer does not rest on
+// where the hits' distances lie.
+__device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const ClosestOut& out, uint64_t& nfetch) {
+    const int lane = threadIdx.x & 63;
+    v3 o, d;
+    load_ray(A.rays, ri, o, d);
+    WideRay r;
+    const RayKind kind = wide_ray(o, d, A.w.far_origin, A.w.rcp_max, r);  // (fine: others are not sent here)
+    const bool in_root = root_hit(A, o, d);
+    if (threadIdx.x == 0) {
+        W.pend[0] = 0u;
+        W.npend = kind == kRayFine ? 1u : 0u;
+        W.ncands = W.bad = W.endless = 0u;
+    }
+    __syncthreads();
+    while (true) {
+        const int count = (int)W.npend;
+        if (count == 0 || W.bad != 0u || W.ncands > (uint32_t)kWholeCands) break;  // (alike in all threads)
+        const int k = count < 8 * kFinishWaves ? count : 8 * kFinishWaves;
+        const int g = (int)(threadIdx.x >> 3);
+        const uint32_t node = g < k ? W.pend[count - 1 - g] : 0u;
+        __syncthreads();
+        if (threadIdx.x == 0) W.npend = (uint32_t)(count - k);
+        __syncthreads();
+        bool inner = false;
+        uint32_t at = 0;
+        int nt = 0;
+        if (g < k) {
+            lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, FLT_MAX, inner, at, nt);
+            nfetch += (lane & 7) == 0 ? 1u : 0u;
+        }
+        const uint64_t im = __ballot(inner);
+        if (im != 0ull) {
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(&W.npend, (uint32_t)__popcll(im));
+            base = (uint32_t)__shfl((int)base, 0, 64) + (uint32_t)__popcll(im & ((1ull << lane) - 1ull));
+            if (inner && base < (uint32_t)kWholePend) W.pend[base] = at;
+            if (inner && base >= (uint32_t)kWholePend) W.bad = 1u;
+        }
+        float4 tri[kWideLeaf * 3];  // (loaded together: a latency each otherwise)
+#pragma unroll
+        for (int j = 0; j < kWideLeaf * 3; ++j)
+            if (j < 3 * nt) tri[j] = A.w.tris[(int64_t)at * 3 + j];
+#pragma unroll
+        for (int j = 0; j < kWideLeaf; ++j) {
+            if (j >= nt) continue;
+            const float4 a = tri[3 * j], b = tri[3 * j + 1], c = tri[3 * j + 2];
+            ++nfetch;
+            float t, u, v;
+            if (!wide_tri_hit(a, b, c, o, d, t, u, v)) continue;
+            bool touch, bad = false;
+            const float e = leaf_entry(a, b, c, o, d, touch);
+            bool hit = e >= 0.f && e < FLT_MAX;
+            const int p = __float_as_int(a.w);
+            if (hit && touch) hit = in_root && reached(A.w, p, o, d, bad);
+            if (bad) W.bad = 1u;
+            if (!hit) continue;
+            if (!(t < FLT_MAX)) {
+                W.endless = 1u;
+                continue;
+            }
+            const uint32_t i = atomicAdd(&W.ncands, 1u);
+            if (i < (uint32_t)kWholeCands) {
+                W.t[i] = t; W.u[i] = u; W.v[i] = v; W.e[i] = e; W.p[i] = p;
+            }
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x < 64) {
+        const int nc = (int)W.ncands;
+        bool failed = W.bad != 0u || nc > kWholeCands || (nc == 0 && W.endless != 0u);
+        int win = -1;
+        if (!failed && nc > 0) {
+            // as in finish_closest, and the hits that could matter in its lanes
+            float best = FLT_MAX;
+            for (int i = lane; i < nc; i += 64) best = fmn(best, W.t[i]);
+            best = wave_min(best);
+            float bound = best;
+            for (bool grew = true; grew;) {
+                float m = 0.f;
+                for (int i = lane; i < nc; i += 64)
+                    if (W.t[i] <= bound) m = fmx(m, fmx(W.t[i], W.e[i]));
+                m = wave_max(m);
+                grew = m > bound;
+                if (grew) bound = m;
+            }
+            int mine = -1, n = 0;
+            for (int b = 0; b < nc && n <= 64; b += 64) {
+                uint64_t m = __ballot(b + lane < nc && W.t[b + lane < nc ? b + lane : 0] <= bound);
+                for (; m != 0ull; m &= m - 1ull, ++n)
+                    if (lane == n) mine = b + __ffsll((long long)m) - 1;
+            }
+            if (n > 64) {
+                failed = true;
+            } else {
+                const bool rival = mine >= 0;
+                const int c = n == 1 ? 0
+                                     : replay(A.w, o, d, rival, rival ? W.t[mine] : FLT_MAX, rival ? W.e[mine] : 0.f,
+                                              rival ? W.p[mine] : 0);
+                if (c < 0) failed = true;
+                else win = __shfl(mine, c, 64);
+            }
+        }
+        if (lane == 0) {
+            if (failed) reference_ray(A, ri, o, d, W.stack, out);
+            else if (win >= 0) write_hit(out, ri, W.p[win], W.t[win], W.u[win], W.v[win]);
+            else write_hit(out, ri, -1, 0.f, 0.f, 0.f);
+        }
+    }
+    __syncthreads();
 }
 
 __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const float* limit, const int32_t* src,
@@ -820,7 +1031,7 @@ __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const 
     bool failed = kind == kRayOdd;
     const float lim = limit[ri];
     const bool use = !(lim == INFINITY);
-    const float cut = use ? lim * kReach * r.scale : FLT_MAX;
+    const float cut = use ? __builtin_fmaf(lim * r.scale, kReach, A.w.near_slack) : FLT_MAX;
     const int sm = src ? src[ri] : -1, dm = dst ? dst[ri] : -1;
     int count = kind != kRayFine || (use && !(lim > 0.f)) ? 0 : 1;
     bool blocked = false, bad = false;
@@ -879,34 +1090,76 @@ __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const 
     wave_fence();
 }
 
-template <bool kAny>
-__global__ __launch_bounds__(64) void k_wide_finish(FinishArgs A, int32_t* oprim, float* ot, float* ou, float* ov,
-                                                    const float* limit, const int32_t* src, const int32_t* dst,
-                                                    uint8_t* ovis) {
+__device__ __forceinline__ void add_fetches(unsigned long long* fetched, uint64_t n) {
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) n += __shfl_xor(n, dd, 64);
+    if ((threadIdx.x & 63) == 0 && n > 0) atomicAdd(fetched, (unsigned long long)n);
+}
+
+__global__ __launch_bounds__(64 * kFinishWaves) void k_wide_finish_closest(FinishArgs A, ClosestOut out) {
+    union Lds {
+        FinishLds wave[kFinishWaves];
+        WholeLds whole;
+    };
+    __shared__ Lds lds;
+    __shared__ uint32_t queue[64 * kFinishWaves];  // rays of this turn to take over their whole lines
+    __shared__ uint32_t queued;
+    const uint32_t all = *A.n;
+    const uint32_t total = min(all, A.cap);
+    if (blockIdx.x >= total) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint64_t nfetch = 0;
+    const auto take = [&](int64_t ri) {
+        if (!finish_closest(A, ri, lds.wave[wave], out, nfetch) && lane == 0) queue[atomicAdd(&queued, 1u)] = (uint32_t)ri;
+    };
+    const auto wholes = [&]() {  // all threads
+        __syncthreads();
+        const uint32_t n = queued;
+        for (uint32_t i = 0; i < n; ++i) finish_whole(A, queue[i], lds.whole, out, nfetch);
+        __syncthreads();
+        if (threadIdx.x == 0) queued = 0u;
+        __syncthreads();
+    };
+    if (threadIdx.x == 0) queued = 0u;
+    __syncthreads();
+    // kFinishTurn rays a wave and turn; the first gridDim.x rays go to as many workgroups
+    const int64_t lanes = (int64_t)gridDim.x * kFinishWaves;
+    for (int64_t base = 0; base < (int64_t)total; base += lanes * kFinishTurn) {
+        for (int j = 0; j < kFinishTurn; ++j) {
+            const int64_t i = base + j * lanes + (int64_t)wave * gridDim.x + blockIdx.x;
+            if (i < (int64_t)total) take(A.ids[i]);
+        }
+        wholes();
+    }
+    if (all > A.cap) {  // the list ran over: find the marked rays
+        const int64_t nrays = A.nrays_dev ? (int64_t)*A.nrays_dev : A.nrays;
+        for (int64_t b = (int64_t)blockIdx.x * 64 * kFinishWaves; b < nrays; b += lanes * 64) {
+            const int64_t first = b + 64 * wave, i = first + lane;
+            for (uint64_t m = __ballot(i < nrays && out.prim[i] == kUndecided); m; m &= m - 1ull)
+                take(first + __ffsll((long long)m) - 1);
+            wholes();
+        }
+    }
+    add_fetches(A.fetched, nfetch);
+}
+
+__global__ __launch_bounds__(64) void k_wide_finish_any(FinishArgs A, const float* limit, const int32_t* src,
+                                                        const int32_t* dst, uint8_t* ovis) {
     __shared__ FinishLds L;
     const uint32_t all = *A.n;
     const uint32_t total = min(all, A.cap);
     if (blockIdx.x >= total) return;
     uint64_t nfetch = 0;
-    for (uint32_t i = blockIdx.x; i < total; i += gridDim.x) {
-        if (kAny) finish_any(A, A.ids[i], L, limit, src, dst, ovis, nfetch);
-        else finish_closest(A, A.ids[i], L, oprim, ot, ou, ov, nfetch);
-    }
+    for (uint32_t i = blockIdx.x; i < total; i += gridDim.x) finish_any(A, A.ids[i], L, limit, src, dst, ovis, nfetch);
     if (all > A.cap) {  // the list ran over: find the marked rays
         const int64_t nrays = A.nrays_dev ? (int64_t)*A.nrays_dev : A.nrays;
         for (int64_t b = (int64_t)blockIdx.x * 64; b < nrays; b += (int64_t)gridDim.x * 64) {
             const int64_t i = b + threadIdx.x;
-            uint64_t m = __ballot(i < nrays && (kAny ? ovis[i] == 255 : oprim[i] == kUndecided));
-            for (; m; m &= m - 1ull) {
-                const int64_t ri = b + __ffsll((long long)m) - 1;
-                if (kAny) finish_any(A, ri, L, limit, src, dst, ovis, nfetch);
-                else finish_closest(A, ri, L, oprim, ot, ou, ov, nfetch);
-            }
+            for (uint64_t m = __ballot(i < nrays && ovis[i] == 255); m; m &= m - 1ull)
+                finish_any(A, b + __ffsll((long long)m) - 1, L, limit, src, dst, ovis, nfetch);
         }
     }
-#pragma unroll
-    for (int dd = 32; dd >= 1; dd >>= 1) nfetch += __shfl_xor(nfetch, dd, 64);
-    if (threadIdx.x == 0 && nfetch > 0) atomicAdd(A.fetched, (unsigned long long)nfetch);
+    add_fetches(A.fetched, nfetch);
 }
 
 constexpr int kFinishBlocks = 4096;
@@ -946,12 +1199,12 @@ void wide_closest(const TraceBvh& bvh, const float* rays, int64_t nrays, const u
     launch_wide_block<false>(L, nrays, ls, bvh.wide.nodes, bvh.wide.tris, rays, nrays, nrays_dev, prim, t, u, v,
                              (const float*)nullptr, (const int32_t*)nullptr, (const int32_t*)nullptr,
                              (uint8_t*)nullptr, counters, reinterpret_cast<unsigned long long*>(counters + 2),
-                             fetch_word(counters, true), wl, bvh.wide.far_origin, bvh.wide.rcp_max);
+                             fetch_word(counters, true), wl, bvh.wide.far_origin, bvh.wide.rcp_max, bvh.wide.near_slack);
     const FinishArgs A{bvh.wide, bvh.rec, bvh.root, rays, nrays, nrays_dev, coop.longs, counters + 26,
                        coop.long_cap, counters + 30, counters, fetch_word(counters, true), bvh.ntris};
-    const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks, nrays);
-    ls.launch("k_wide_finish<closest>", &k_wide_finish<false>, dim3(blocks), dim3(64), A, prim, t, u, v,
-              (const float*)nullptr, (const int32_t*)nullptr, (const int32_t*)nullptr, (uint8_t*)nullptr);
+    const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks / kFinishWaves, nrays);
+    ls.launch("k_wide_finish_closest", &k_wide_finish_closest, dim3(blocks), dim3(64 * kFinishWaves), A,
+              ClosestOut{prim, t, u, v});
 }
 
 // Words 20 and 22 likewise; the list is the failure list behind the spill records.
@@ -963,12 +1216,11 @@ void wide_occluded(const TraceBvh& bvh, const float* rays, int64_t nrays, const 
     launch_wide_block<true>(L, nrays, ls, bvh.wide.nodes, bvh.wide.tris, rays, nrays, nrays_dev, (int32_t*)nullptr,
                             (float*)nullptr, (float*)nullptr, (float*)nullptr, limit, src, dst, visible,
                             counters + 1, reinterpret_cast<unsigned long long*>(counters + 4),
-                            fetch_word(counters, false), wl, bvh.wide.far_origin, bvh.wide.rcp_max);
+                            fetch_word(counters, false), wl, bvh.wide.far_origin, bvh.wide.rcp_max, bvh.wide.near_slack);
     const FinishArgs A{bvh.wide, bvh.rec, bvh.root, rays, nrays, nrays_dev, ids, counters + 20,
                        coop.spill_cap, counters + 22, counters + 1, fetch_word(counters, false), bvh.ntris};
     const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks, nrays);
-    ls.launch("k_wide_finish<any>", &k_wide_finish<true>, dim3(blocks), dim3(64), A, (int32_t*)nullptr,
-              (float*)nullptr, (float*)nullptr, (float*)nullptr, limit, src, dst, visible);
+    ls.launch("k_wide_finish_any", &k_wide_finish_any, dim3(blocks), dim3(64), A, limit, src, dst, visible);
 }
 
 }  // namespace cav

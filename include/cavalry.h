@@ -398,6 +398,12 @@ int cav_scene_create_from_pbrt(cav_ctx* ctx, const char* path, const cav_pbrt_ov
  * deep, a coordinate is beyond 2^40, or there was no memory for the wide tree;
  * so do single rays that start more than 2^20 times the scene's largest
  * coordinate from 0 or whose direction is close to the limits of a float.
+ * Over the wide tree a closest hit is the reference's but for one assumption:
+ * boxes more than 2^-5 (relative) and 2^-16 of the scene's largest coordinate
+ * beyond the nearest hit are skipped, and a triangle in one can only matter
+ * where Moller-Trumbore's t is that far off, in a triangle met edge on or a
+ * needle. Rays that test such a triangle are walked along their whole line, so
+ * an answer can differ only where all of them lie behind the nearest hit.
  * Workgroups per CU (0: as many as fit; reference's tree only), rays a wave takes from the dispenser at a time
  * (64..65536), traversal-stack entries kept in LDS (32 or 48; the rest of
  * the reference's 64 in scratch) and threads per traversal workgroup (64,
@@ -411,9 +417,10 @@ int cav_scene_create_from_pbrt(cav_ctx* ctx, const char* path, const cav_pbrt_ov
  * nodes sharing a 128-byte line, both tested), and whether any-hit rays
  * visit boxes that start beyond their limit (1: every box the ray's line
  * crosses, the reference's visiting order; 0, the default: a box starting
- * more than 2^-10 (relative) beyond the limit is skipped, since no triangle
- * in it can block the ray unless Moller-Trumbore's t is off by more than
- * that, which takes a ray within about 1e-4 rad of a sliver's plane).
+ * more than 2^-5 (the wide tree) or 2^-10 (the reference's; relative) beyond
+ * the limit is skipped, since no triangle in it can block the ray unless
+ * Moller-Trumbore's t is off by more than that, which takes a ray within
+ * about 1e-5 or 1e-4 rad of a sliver's plane).
  * Each ray's closest-hit node order is the reference's, the any-hit answer
  * does not depend on the order the reachable leaves are tested in, and each
  * sample's shading is its own, so results do not depend on the shape. STANDALONE applies to cav_trace_*, WAVEFRONT to

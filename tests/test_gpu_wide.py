@@ -200,10 +200,12 @@ def test_rays_almost_along_flat_boxes(ctx, axis, size, noise):
     assert (ref["prim"] >= 0).sum() > 200
 
 
-@pytest.mark.parametrize("size,length", [(1.0, 1e-38), (1.0, 2.4e-38), (1.0, 1e-36), (1e12, 1e-27), (1e10, 1e-30)])
+@pytest.mark.parametrize("size,length", [(1.0, 1e-38), (1.0, 2.4e-38), (1.0, 1e-36), (1e12, 1e-27), (1e10, 1e-30),
+                                         (1e-13, 1.0), (1e-15, 1.0), (1e-7, 1e-14)])
 def test_distances_near_the_limits_of_a_float(ctx, size, length):
     """Scenes and directions whose hits lie at distances up to infinity (the
-    reference takes the first hit whatever its distance)."""
+    reference takes the first hit whatever its distance), and whose products
+    in the triangle test lose bits to underflow."""
     tris = (scenes.gmm_triangles(700, seed=13, edge=0.4) * np.float32(size)).astype(np.float32)
     rays = scenes.random_rays(6000, seed=14, lo=0.2, hi=0.8)
     rays[:, :3] *= np.float32(size)
@@ -213,3 +215,59 @@ def test_distances_near_the_limits_of_a_float(ctx, size, length):
     lim[::3] = np.float32(size / length * 0.3) if size / length < 1e38 else np.float32(3e38)
     bvh, nd = _tree(ctx, tris, 30, 0)
     _check(bvh, nd, tris, rays, lim, f"size {size}, directions of {length}")
+
+
+def _turned(tris, seed, size):
+    q, _ = np.linalg.qr(np.random.default_rng(seed).normal(size=(3, 3)))
+    return np.ascontiguousarray((tris @ q.T * size).reshape(-1, 9), np.float32), q
+
+
+@pytest.mark.parametrize("size", [1.0, 10.0, 1e-3])
+@pytest.mark.parametrize("walls", [False, True])
+def test_rays_in_the_plane_of_a_turned_floor(ctx, size, walls):
+    """Rays in the plane of a turned, tessellated floor meet its triangles edge
+    on, where Moller-Trumbore's t is rounding noise that may lie far from the
+    triangle's box; walls across the floor stop them at exact distances."""
+    tris = _floor(40, 1.0)
+    tris[..., :2] -= 0.5
+    for x in (-0.2, 0.05, 0.3) if walls else ():
+        w = tris[::7, :, [2, 1, 0]].copy()
+        w[..., 0] = x
+        tris = np.concatenate([tris, w])
+    for seed in range(6):
+        rng = np.random.default_rng(seed)
+        tt, q = _turned(tris, seed, size)
+        n = 8000
+        o = np.stack([rng.uniform(-0.8, 0.8, n), rng.uniform(-0.8, 0.8, n), np.zeros(n)], -1)
+        a = rng.uniform(0, 2 * np.pi, n)
+        d = np.stack([np.cos(a), np.sin(a), rng.normal(size=n) * (0.0, 1e-8, 1e-7)[seed % 3]], -1)
+        rays = np.ascontiguousarray(np.concatenate([o @ q.T * size, d @ q.T], 1), np.float32)
+        bvh, nd = _tree(ctx, tt, 30, 3 * (seed % 2))
+        ref, got = oracle.trace_closest(nd, tt, rays), bvh.intersect(rays)
+        print(f"[wide] turned floor, size {size}, walls {walls}, seed {seed}: "
+              f"{(ref['prim'] != got['prim']).sum()} of {n} differ; {bvh.trace_fetches()}", flush=True)
+        np.testing.assert_array_equal(got["prim"], ref["prim"])
+        for k in ("t", "u", "v"):
+            np.testing.assert_array_equal(bits(got[k]), bits(ref[k]), err_msg=k)
+
+
+@pytest.mark.parametrize("ratio", [300, 30000, 3000000])
+def test_needles(ctx, ratio):
+    """Triangles `ratio` times longer than wide among ordinary ones, and rays
+    aimed at them: edge on or not, their determinants are small."""
+    rng = np.random.default_rng(ratio)
+    base = scenes.gmm_triangles(3000, seed=15, edge=0.1)
+    thin = scenes.gmm_triangles(3000, seed=16, edge=0.3).reshape(-1, 3, 3)
+    thin[:, 2] = thin[:, 1] + (thin[:, 2] - thin[:, 1]) / np.float32(ratio)
+    tris = np.ascontiguousarray(np.concatenate([base, thin.reshape(-1, 9)]), np.float32)
+    n = 30000
+    k, w = rng.integers(0, 3000, n), rng.random((n, 1))
+    at = thin[k, 0] * (1 - w) + (thin[k, 1] + thin[k, 2]) / 2 * w
+    o = rng.random((n, 3))
+    d = at - o
+    rays = np.ascontiguousarray(np.concatenate([o, d / np.linalg.norm(d, axis=1, keepdims=True)], 1), np.float32)
+    # (with a limit, any-hit rays may skip a needle whose t lies far from its box: see cav_trace_launch)
+    lim = np.full(n, np.inf, np.float32)
+    bvh, nd = _tree(ctx, tris, 30, 0)
+    _check(bvh, nd, tris, rays, lim, f"needles {ratio}")
+    print(f"[wide] needles {ratio}: {bvh.trace_fetches()}", flush=True)
