@@ -57,7 +57,12 @@ ALG_BYTES_LAUNCH_30 = {
     "refit_bottom_up": lambda n: (4 + 36 + 4 + 32 + 12 + 4) * n + (n - 1) * (32 + 12 + 4 + 4),
 }
 ALG_BYTES_PER_TRI_30 = 248  # whole build, canonical model: S1 68 + S2 68 + S3 20 + S4 92
-TRACE_RECORD_BYTES = 64  # one traversal record (node or triangle) per step
+TRACE_RECORD_BYTES = 64  # one traversal record (node or triangle) of the reference's tree
+# the wide tree's: bytes fetched, and VALU instructions of the compiled tests
+# (a node's eight children; a triangle up to the test's first exit)
+WIDE_NODE_BYTES, WIDE_TRI_BYTES = 80, 48
+WIDE_NODE_OPS, WIDE_TRI_OPS = 198, 45
+VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12  # FP32 instructions, one per lane and clock: 256 CUs of 64 lanes at 2.4 GHz
 
 
 def log(msg: str) -> None:
@@ -576,6 +581,7 @@ def main() -> int:
     ctx.synchronize()
     bvh.trace_counters(reset=True)  # count stack overflows of the timed traces only
     bvh.trace_fetches(reset=True)
+    bvh.trace_wide(reset=True)
     recs = []
     t0 = time.perf_counter()
     for i in range(args.steps):
@@ -588,6 +594,7 @@ def main() -> int:
     # results are partial and the run fails
     trav = bvh.trace_counters()
     fetches = bvh.trace_fetches()
+    walked = bvh.trace_wide()
     trav["max_leaf_depth"] = bvh.max_depth()
     trav["stack_entries"] = 64
     # the timed traces' answers (cooperative passes, limit cull) against the
@@ -604,6 +611,7 @@ def main() -> int:
     stages = {}
     for k in ("ms_bounds", "ms_morton", "ms_sort", "ms_karras", "ms_refit", "ms_treelet", "ms_flatten"):
         stages[k[3:]] = round(float(np.mean([rec[0][k] for rec in recs])), 4)
+    stages["wide_tree"] = round(float(np.mean([rec[0]["ms_wide"] for rec in recs])), 4)
     stages["trace_closest"] = round(float(np.mean([rec[2] for rec in recs])), 4)
     stages["trace_shadow"] = round(float(np.mean([rec[3] for rec in recs])), 4)
     # (the radix tree is emitted by the refit's climb: karras is 0)
@@ -637,33 +645,41 @@ def main() -> int:
         "build_frac": round(ALG_BYTES_PER_TRI_30 * n / (lbvh_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
         "build_alg_bytes_per_tri": ALG_BYTES_PER_TRI_30,
     }
-    # roofline of the step's dominant kernel, the traversal: the records its
-    # timed launches fetched (64 bytes each: a wide node is 80, a wide triangle
-    # 48, a record of the reference's tree 64) + the rays read and the hits
-    # written; launches that walk the reference's tree count the records of its
-    # visiting order instead, which are fewer than the wave passes fetch
+    # roofline of the step's dominant kernel, the traversal: the bytes of the
+    # records it fetched (whether the caches or HBM serve them), the rays and the
+    # hits against HBM, and over the wide tree the VALU instructions of the tests
+    # it made against the chip's issue rate; the nearer one bounds it. Over the
+    # reference's tree the records are those of its visiting order, which are
+    # fewer than the wave passes fetch.
     fetch = {k: v / args.steps for k, v in fetches.items()}
-    wide = {k: fetch[k] < ref_fetch[k] for k in fetch}
-    counted = {k: fetch[k] if wide[k] else ref_fetch[k] for k in fetch}
-    trav_bytes = {
-        "closest": counted["closest"] * TRACE_RECORD_BYTES + r * (24 + 8),
-        "occluded": counted["occluded"] * TRACE_RECORD_BYTES + r * (24 + 4 + 1),
-    }
+    tri_fetch = {k: walked[k + "_triangles"] / args.steps for k in ("closest", "occluded")}
     trav_ms = {"closest": stages["trace_closest"], "occluded": stages["trace_shadow"]}
     tdom = max(trav_ms, key=lambda k: trav_ms[k])
-    t_ach = trav_bytes[tdom] / (trav_ms[tdom] * 1e-3) / 1e9
+    alg = r * {"closest": 24 + 8, "occluded": 24 + 4 + 1}[tdom]
+    tops = 0.0
+    if walked[tdom]:
+        nodes = fetch[tdom] - tri_fetch[tdom]
+        alg += nodes * WIDE_NODE_BYTES + tri_fetch[tdom] * WIDE_TRI_BYTES
+        tops = (nodes * WIDE_NODE_OPS + tri_fetch[tdom] * WIDE_TRI_OPS) / (trav_ms[tdom] * 1e-3) / 1e12
+    else:
+        alg += ref_fetch[tdom] * TRACE_RECORD_BYTES
+    gbs = alg / (trav_ms[tdom] * 1e-3) / 1e9
+    valu = tops / VALU_PEAK_TOPS > gbs / HBM_PEAK_GBS
+    ach, peak = (tops, VALU_PEAK_TOPS) if valu else (gbs, HBM_PEAK_GBS)
     roofline = {
-        "bound": "hbm",
-        "kernel": f"{'k_wide_trace' if wide[tdom] else 'k_trace'}<{'closest' if tdom == 'closest' else 'any'}>",
-        "achieved": round(t_ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-        "frac": round(t_ach / HBM_PEAK_GBS, 4), "traffic": None,
-        "avg_launch_ms": round(trav_ms[tdom], 4), "alg_bytes_per_launch": int(trav_bytes[tdom]),
+        "bound": "valu" if valu else "hbm",
+        "kernel": f"{'k_wide_trace' if walked[tdom] else 'k_trace'}<{'closest' if tdom == 'closest' else 'any'}>",
+        "achieved": round(ach, 2), "peak": round(peak, 1), "unit": "Tinstr/s" if valu else "GB/s",
+        "frac": round(ach / peak, 4), "traffic": None,
+        "avg_launch_ms": round(trav_ms[tdom], 4), "alg_bytes_per_launch": int(alg),
+        "fetched_gb_s": round(gbs, 1), "valu_tinstr_s": round(tops, 2), "valu_frac": round(tops / VALU_PEAK_TOPS, 4),
         "records_per_ray": round(ref_fetch[tdom] / r, 1),
         "records_fetched_per_ray": round(fetch[tdom] / r, 1),
-        "note": "algorithmic bytes count every record the timed traces of the wide tree fetched, whether "
-                "L2 or HBM serves it (records_fetched_per_ray); records_per_ray is what the reference's "
-                "visiting order fetches (closest-hit; any-hit up to the ray's limit), counted on an untimed "
-                "trace without the cooperative passes",
+        "triangles_fetched_per_ray": round(tri_fetch[tdom] / r, 1),
+        "note": "algorithmic bytes count every record fetched (wide tree: 80-byte nodes, 48-byte triangles), whether the "
+                "caches or HBM serve it, and the rays and hits; valu: FP32 lane instructions of the wide tree's node and "
+                "triangle tests; records_per_ray is what the reference's visiting order fetches (any-hit up to the ray's "
+                "limit), counted on an untimed trace without the cooperative passes",
         "lbvh_build_frac": lbvh_roofline["build_frac"],
     }
     traffic_file = os.path.join(ROOT, "profiles", "traffic.json")
@@ -710,6 +726,9 @@ def main() -> int:
         },
         "lbvh_build_mtris_s": round(n / (lbvh_ms * 1e-3) / 1e6, 2),
         "lbvh_build_ms": round(lbvh_ms, 4),
+        # with the flattened records and the wide tree that the traces walk
+        "bvh_build_ms": round(lbvh_ms + stages["flatten"] + stages["wide_tree"], 4),
+        "bvh_build_mtris_s": round(n / ((lbvh_ms + stages["flatten"] + stages["wide_tree"]) * 1e-3) / 1e6, 2),
         "treelet_ms_per_round": round(stages["treelet"] / max(args.rounds, 1), 4),
         "trace_closest_mrays_s": round(r / (stages["trace_closest"] * 1e-3) / 1e6, 2),
         "trace_shadow_mrays_s": round(r / (stages["trace_shadow"] * 1e-3) / 1e6, 2),

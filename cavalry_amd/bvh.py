@@ -119,7 +119,10 @@ class BVH:
     def stats(self) -> dict:
         s = _lib.BvhStats()
         check(self.ctx.handle, lib().cav_bvh_stats_get(self.handle, ctypes.byref(s)))
-        return {k: getattr(s, k) for k, _ in s._fields_}
+        out = {k: getattr(s, k) for k, _ in s._fields_}
+        # the tree the traces walk, built beside the reference's (in ms_total)
+        out["ms_wide"] = sum(ms for name, ms in self.kernel_times() if name.startswith("wide"))
+        return out
 
     def kernel_times(self) -> list:
         """[(kernel name, ms)] of the last build, in launch order."""
@@ -185,6 +188,15 @@ class BVH:
         return {"closest": int(out[0]), "occluded": int(out[1]), "spilled_rays": int(out[2]),
                 "respilled_rays": int(out[3]), "long_closest_rays": int(out[4]),
                 "long_closest_retraced": int(out[5])}
+
+    def trace_wide(self, which: int = 0, reset: bool = False) -> dict:
+        """Whether closest-hit / any-hit traces of a launch shape (0: standalone,
+        1: render loops) walk the wide tree instead of the reference's, and how
+        many of trace_fetches' records were triangles of the wide tree."""
+        out = np.zeros(4, np.uint64)
+        check(self.ctx.handle, lib().cav_trace_wide(self.ctx.handle, self.handle, int(which), _ptr(out), 1 if reset else 0))
+        return {"closest": bool(out[0]), "occluded": bool(out[1]), "closest_triangles": int(out[2]),
+                "occluded_triangles": int(out[3])}
 
     def max_depth(self) -> int:
         """Deepest leaf, in edges from the root."""

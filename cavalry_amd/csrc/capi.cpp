@@ -82,7 +82,7 @@ static int bvh_alloc(cav_ctx* ctx, cav_bvh* h, int n) {
         {(void**)&h->b.gate64, sizeof(uint64_t) * bottom_up_gate_words(n), "split gates"},
         {(void**)&h->b.ref, sizeof(int32_t) * m, "ref"},
         {(void**)&h->b.partial, sizeof(uint32_t) * (lbvh_partials(m) + 1), "partial"},
-        {(void**)&h->b.counters, 256, "counters"},
+        {(void**)&h->b.counters, kTraceCounterBytes, "counters"},
         {(void**)&h->rec, sizeof(TRec) * 2 * (size_t)n, "traversal records"},
         {(void**)&h->root, 64, "root"},
         {(void**)&h->b.lvl_list, sizeof(uint32_t) * m, "level list"},
@@ -97,7 +97,7 @@ static int bvh_alloc(cav_ctx* ctx, cav_bvh* h, int n) {
     // the bottom-up build leaves every split gate at zero for the next build;
     // the traversal counters only ever add to (or max into) their words
     HIPCHK(ctx, hipMemsetAsync(h->b.gate64, 0, sizeof(uint64_t) * bottom_up_gate_words(n), ctx->stream));
-    HIPCHK(ctx, hipMemsetAsync(h->b.counters, 0, 256, ctx->stream));
+    HIPCHK(ctx, hipMemsetAsync(h->b.counters, 0, kTraceCounterBytes, ctx->stream));
     // the wide tree is left out where memory is short: the traces then walk
     // the reference's tree
     void* wide = nullptr;
@@ -495,10 +495,24 @@ int cav_trace_fetches(cav_ctx* ctx, const cav_bvh* h, uint64_t* out6, int32_t re
     return CAV_OK;
 }
 
+int cav_trace_wide(cav_ctx* ctx, const cav_bvh* h, int32_t which, uint64_t* out4, int32_t reset) {
+    if (!ctx || !h || !out4) return CAV_ERR_INVALID;
+    if (which != CAV_TRACE_STANDALONE && which != CAV_TRACE_WAVEFRONT)
+        return fail(ctx, CAV_ERR_INVALID, "which must be CAV_TRACE_STANDALONE or CAV_TRACE_WAVEFRONT");
+    HIPCHK(ctx, hipSetDevice(ctx->device));
+    const TraceBvh t = bvh_trace(h);
+    out4[0] = closest_walks_wide(t, ctx->launch[which]) ? 1u : 0u;
+    out4[1] = any_walks_wide(t, ctx->launch[which]) ? 1u : 0u;
+    HIPCHK(ctx, hipMemcpyAsync(out4 + 2, h->b.counters + 32, 16, hipMemcpyDeviceToHost, ctx->stream));
+    if (reset) HIPCHK(ctx, hipMemsetAsync(h->b.counters + 32, 0, 16, ctx->stream));
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    return CAV_OK;
+}
+
 int cav_bvh_max_depth(cav_ctx* ctx, const cav_bvh* h, int32_t* depth) {
     if (!ctx || !h || !depth) return CAV_ERR_INVALID;
     HIPCHK(ctx, hipSetDevice(ctx->device));
-    // counters[8] is free scratch (the traversal uses words 0..7 and 16..30)
+    // counters[8] is free scratch (the traversal uses words 0..7, 16..30 and 32..35)
     uint32_t* word = h->b.counters + 8;
     HIPCHK(ctx, levels_max_depth(h->b, h->n, word, ctx->stream));
     uint32_t d = 0;

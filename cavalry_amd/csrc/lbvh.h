@@ -101,12 +101,14 @@ hipError_t treelet_round_impl(LbvhBuffers& b, int n, hipStream_t s, Marker* mk);
 // means the results are partial); counters[2..5] hold the ray dispensers;
 // counters[6] (closest) and counters[7] (occluded) keep the deepest stack any
 // ray reached (atomic max, never reset by a launch); the 64-bit words at
-// counters[16] (closest) and counters[18] (occluded) add up the 64-byte
-// records every launch fetched (never reset by a launch); counters[20..25]
+// counters[16] (closest) and counters[18] (occluded) add up the records
+// every launch fetched, those at counters[32] and counters[34] the wide
+// tree's triangles among them (never reset by a launch); counters[20..25]
 // are the cooperative any-hit pass's spill count, spill cursor, failure
 // count and ray dispenser, counters[26..30] the cooperative closest-hit
 // pass's long-ray count, cursor, phase-3 ray dispenser (64-bit, 28-29) and
 // phase-3 count (all cleared by each launch).
+constexpr size_t kTraceCounterBytes = 256;
 // Launch shape of the persistent traversal kernels (and, for the render
 // loops, of the per-sample shading kernels). Each ray's node order is fixed
 // and each sample's shading is independent of where it runs, so results do
@@ -192,6 +194,14 @@ struct TraceBvh {
     const float* root = nullptr;
     WideDev wide;
 };
+// From this hand-off on no ray goes to a whole wave: one lane per ray in the
+// reference's order.
+constexpr int kNoHandoff = 1 << 30;
+// Whether traces of such a shape walk the wide tree.
+inline bool closest_walks_wide(const TraceBvh& b, const TraceLaunch& L) { return b.wide.nodes && L.handoff < kNoHandoff; }
+inline bool any_walks_wide(const TraceBvh& b, const TraceLaunch& L) {
+    return b.wide.nodes && L.handoff < kNoHandoff && !L.any_full && !any_step_pairs(L);
+}
 
 // coop: null (every ray traced by one lane in the reference's order) or the
 // cooperative passes' buffers

@@ -263,7 +263,7 @@ int make_pool(cav_server* sv, cav_scene* sc, Pool*& out) {
     A(d.sh.ray, 24 * C); A(d.sh.limit, 4 * C); A(d.sh.src, 4 * C); A(d.sh.dst, 4 * C); A(d.sh.sid, 4 * C);
     A(d.sh.contrib, 12 * C); A(d.sh_rid, 4 * C); A(d.vis, C); A(d.hit_prim, 4 * C); A(d.hit_t, 4 * C);
     A(d.hit_u, 4 * C); A(d.hit_v, 4 * C);
-    A(d.counts, 64); A(d.rays, 64); A(d.trace_counters, 128);
+    A(d.counts, 64); A(d.rays, 64); A(d.trace_counters, kTraceCounterBytes);
     unsigned char* coop = nullptr;
     const uint32_t cc = any_spill_capacity((int64_t)C);
     A(coop, trace_coop_bytes(cc, cc));
@@ -297,7 +297,7 @@ int make_pool(cav_server* sv, cav_scene* sc, Pool*& out) {
     for (auto& e : p->ring) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     ok = ok && hipMemsetAsync(d.counts, 0, 64, p->stream) == hipSuccess &&
          hipMemsetAsync(d.rays, 0, 64, p->stream) == hipSuccess &&
-         hipMemsetAsync(d.trace_counters, 0, 128, p->stream) == hipSuccess &&
+         hipMemsetAsync(d.trace_counters, 0, kTraceCounterBytes, p->stream) == hipSuccess &&
          hipMemsetAsync(R.req, 0, sizeof(RlReqState) * kSlots, p->stream) == hipSuccess &&
          hipMemsetAsync(R.live, 0, kSlots, p->stream) == hipSuccess &&
          hipStreamSynchronize(p->stream) == hipSuccess;

@@ -46,7 +46,9 @@ __device__ __forceinline__ void load_ray(const float* __restrict__ rays, int64_t
 }
 
 // 64-bit count of records fetched by closest-hit (words 16-17) or any-hit
-// (words 18-19) launches
+// (words 18-19) launches; kFetchTris 64-bit words on, how many of them were
+// triangles of the wide tree
+constexpr int kFetchTris = 8;
 __host__ __device__ inline unsigned long long* fetch_word(uint32_t* counters, bool closest) {
     return reinterpret_cast<unsigned long long*>(counters + (closest ? 16 : 18));
 }

@@ -1113,7 +1113,6 @@ void launch_any(const TraceLaunch& L, int64_t work, LaunchSink& ls, A... args) {
 // steps are dropped: its cooperative pass starts again from the root. From
 // kNoHandoff on, no ray goes and the passes are not launched (small scenes,
 // whose rays are all short, save the launches).
-constexpr int kNoHandoff = 1 << 30;
 // lanes of a phase-3 launch (the rays the cooperative passes send back)
 constexpr int64_t kPhase3Lanes = 16384;
 
@@ -1138,7 +1137,7 @@ void trace_any(const TraceBvh& bvh, const float* rays, int64_t nrays, const uint
     AnySpill* spill = tc ? tc->spill : nullptr;
     const uint32_t spill_cap = tc ? tc->spill_cap : 0u;
     const bool coop = spill && spill_cap > 0 && nrays < (int64_t(1) << 32) && L.handoff < kNoHandoff;
-    if (coop && bvh.wide.nodes && !L.any_full && !any_step_pairs(L)) {
+    if (coop && any_walks_wide(bvh, L)) {
         wide_occluded(bvh, rays, nrays, nrays_dev, limit, src, dst, visible, counters, L, *tc, ls);
         return;
     }
@@ -1175,7 +1174,7 @@ void trace_near(const TraceBvh& bvh, const float* rays, int64_t nrays,
                 const uint32_t* nrays_dev, int32_t* prim, float* t, float* u, float* v, uint32_t* counters,
                 const TraceLaunch& L, const TraceCoop* coop, LaunchSink& ls) {
     const bool on = coop && coop->longs && coop->long_cap > 0 && nrays < (int64_t(1) << 32) && L.handoff < kNoHandoff;
-    if (on && bvh.wide.nodes) {
+    if (on && closest_walks_wide(bvh, L)) {
         wide_closest(bvh, rays, nrays, nrays_dev, prim, t, u, v, counters, L, *coop, ls);
         return;
     }

@@ -309,6 +309,19 @@ struct WideStackLds {
     uint16_t bits[kWideStack][B];
 };
 
+// A wave's nodes and triangles fetched into the launch's words (fetch_word).
+__device__ __forceinline__ void add_fetches(unsigned long long* fetched, uint64_t nodes, uint64_t tris) {
+#pragma unroll
+    for (int dd = 32; dd >= 1; dd >>= 1) {
+        nodes += __shfl_xor(nodes, dd, 64);
+        tris += __shfl_xor(tris, dd, 64);
+    }
+    if ((threadIdx.x & 63) == 0 && nodes + tris > 0) {
+        atomicAdd(fetched, (unsigned long long)(nodes + tris));
+        atomicAdd(fetched + kFetchTris, (unsigned long long)tris);
+    }
+}
+
 struct WideList {           // rays left to the finishing pass
     uint32_t* ids = nullptr;
     uint32_t* n = nullptr;  // rays listed (past cap: the rest are marked in the hit ids)
@@ -347,7 +360,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
     uint32_t tbase = 0, tbits = 0;  // triangles to test
     int sp = 0, maxsp = 0;
     uint32_t deep[2 * (kWideDeep - kWideStack)];
-    uint32_t nfetch = 0;
+    uint32_t nnodes = 0, ntris = 0;  // fetched
     Dispenser disp(nrays, most);
 
     while (true) {
@@ -467,7 +480,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                 }
                 const uint4* nd = nodes + (int64_t)child * kWideWords;
                 const uint4 w0 = nd[0], w1 = nd[1], w2 = nd[2], w3 = nd[3], w4 = nd[4];
-                ++nfetch;
+                ++nnodes;
                 const uint32_t mask = test_children(w0, w1, w2, w3, w4, r, cut);
                 cbase = w1.x;
                 tbase = w1.y;
@@ -480,7 +493,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
             tbits &= tbits - 1u;
             const float4* tp = tris + (int64_t)(tbase + k) * 3;
             const float4 a = tp[0], b = tp[1], c = tp[2];
-            ++nfetch;
+            ++ntris;
             float t, u, v;
             if (kAny) {
                 const int mesh = __float_as_int(b.w);
@@ -505,14 +518,10 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
             else over = true;
         }
     }
-    uint64_t fetches = nfetch;
 #pragma unroll
-    for (int dd = 32; dd >= 1; dd >>= 1) {
-        maxsp = max(maxsp, __shfl_xor(maxsp, dd, 64));
-        fetches += __shfl_xor(fetches, dd, 64);
-    }
+    for (int dd = 32; dd >= 1; dd >>= 1) maxsp = max(maxsp, __shfl_xor(maxsp, dd, 64));
     if (lane == 0 && maxsp > 0) atomicMax(overflow + 6, (uint32_t)maxsp);
-    if (lane == 0 && fetches > 0) atomicAdd(fetched, (unsigned long long)fetches);
+    add_fetches(fetched, nnodes, ntris);
 }
 
 // ------------------------------------------------------------- finishing pass
@@ -649,6 +658,9 @@ __device__ bool reference_blocked(const TRec* recs, v3 o, v3 d, float lim, int s
     }
 }
 
+struct Fetches {
+    uint64_t nodes = 0, tris = 0;
+};
 struct FinishLds {
     uint32_t pend[kPend];
     float t[kCands], u[kCands], v[kCands], e[kCands];
@@ -792,7 +804,7 @@ __device__ __forceinline__ bool root_hit(const FinishArgs& A, v3 o, v3 d) {
 }
 
 // A ray by a wave. false: it has to be taken over its whole line.
-__device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, const ClosestOut& out, uint64_t& nfetch) {
+__device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, const ClosestOut& out, Fetches& nfetch) {
     const int lane = threadIdx.x & 63;
     v3 o, d;
     load_ray(A.rays, ri, o, d);
@@ -818,7 +830,7 @@ __device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, co
             const uint32_t node = L.pend[count - 1 - g];
             const float cut = best == FLT_MAX ? FLT_MAX : __builtin_fmaf(best * r.scale, kReach, A.w.near_slack);
             lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, cut, inner, at, nt);
-            nfetch += (lane & 7) == 0 ? 1u : 0u;
+            nfetch.nodes += (lane & 7) == 0 ? 1u : 0u;
         }
         count -= k;
         wave_fence();
@@ -829,7 +841,7 @@ __device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, co
             if (j < nt) {
                 const float4* tp = A.w.tris + (int64_t)(at + (uint32_t)j) * 3;
                 const float4 a = tp[0], b = tp[1], c = tp[2];
-                ++nfetch;
+                ++nfetch.tris;
                 thin = thin || thin_test(a, b, c, d, r.scale);
                 if (wide_tri_hit(a, b, c, o, d, t, u, v)) {
                     thin = thin || thin_hit(a, b, c, o, d, t, t * (kReach - 1.f) + near);
@@ -911,7 +923,7 @@ __device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, co
 // A ray over its whole line by all waves of the workgroup, 64 nodes at a
 // time: no box of the line is skipped, so that the answer does not rest on
 // where the hits' distances lie.
-__device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const ClosestOut& out, uint64_t& nfetch) {
+__device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const ClosestOut& out, Fetches& nfetch) {
     const int lane = threadIdx.x & 63;
     v3 o, d;
     load_ray(A.rays, ri, o, d);
@@ -938,7 +950,7 @@ __device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const
         int nt = 0;
         if (g < k) {
             lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, FLT_MAX, inner, at, nt);
-            nfetch += (lane & 7) == 0 ? 1u : 0u;
+            nfetch.nodes += (lane & 7) == 0 ? 1u : 0u;
         }
         const uint64_t im = __ballot(inner);
         if (im != 0ull) {
@@ -956,7 +968,7 @@ __device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const
         for (int j = 0; j < kWideLeaf; ++j) {
             if (j >= nt) continue;
             const float4 a = tri[3 * j], b = tri[3 * j + 1], c = tri[3 * j + 2];
-            ++nfetch;
+            ++nfetch.tris;
             float t, u, v;
             if (!wide_tri_hit(a, b, c, o, d, t, u, v)) continue;
             bool touch, bad = false;
@@ -1022,7 +1034,7 @@ __device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const
 }
 
 __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const float* limit, const int32_t* src,
-                           const int32_t* dst, uint8_t* ovis, uint64_t& nfetch) {
+                           const int32_t* dst, uint8_t* ovis, Fetches& nfetch) {
     const int lane = threadIdx.x;
     v3 o, d;
     load_ray(A.rays, ri, o, d);
@@ -1046,14 +1058,14 @@ __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const 
         if (g < k) {
             const uint32_t node = L.pend[count - 1 - g];
             lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, cut, inner, at, nt);
-            nfetch += (lane & 7) == 0 ? 1u : 0u;
+            nfetch.nodes += (lane & 7) == 0 ? 1u : 0u;
         }
         count -= k;
         wave_fence();
         for (int j = 0; j < nt && !hit; ++j) {
             const float4* tp = A.w.tris + (int64_t)(at + (uint32_t)j) * 3;
             const float4 a = tp[0], b = tp[1], c = tp[2];
-            ++nfetch;
+            ++nfetch.tris;
             const int mesh = __float_as_int(b.w);
             float t, u, v;
             if (mesh != sm && mesh != dm && wide_tri_hit(a, b, c, o, d, t, u, v) && (!use || t < lim)) {
@@ -1090,12 +1102,6 @@ __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const 
     wave_fence();
 }
 
-__device__ __forceinline__ void add_fetches(unsigned long long* fetched, uint64_t n) {
-#pragma unroll
-    for (int dd = 32; dd >= 1; dd >>= 1) n += __shfl_xor(n, dd, 64);
-    if ((threadIdx.x & 63) == 0 && n > 0) atomicAdd(fetched, (unsigned long long)n);
-}
-
 __global__ __launch_bounds__(64 * kFinishWaves) void k_wide_finish_closest(FinishArgs A, ClosestOut out) {
     union Lds {
         FinishLds wave[kFinishWaves];
@@ -1108,7 +1114,7 @@ __global__ __launch_bounds__(64 * kFinishWaves) void k_wide_finish_closest(Finis
     const uint32_t total = min(all, A.cap);
     if (blockIdx.x >= total) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint64_t nfetch = 0;
+    Fetches nfetch;
     const auto take = [&](int64_t ri) {
         if (!finish_closest(A, ri, lds.wave[wave], out, nfetch) && lane == 0) queue[atomicAdd(&queued, 1u)] = (uint32_t)ri;
     };
@@ -1140,7 +1146,7 @@ __global__ __launch_bounds__(64 * kFinishWaves) void k_wide_finish_closest(Finis
             wholes();
         }
     }
-    add_fetches(A.fetched, nfetch);
+    add_fetches(A.fetched, nfetch.nodes, nfetch.tris);
 }
 
 __global__ __launch_bounds__(64) void k_wide_finish_any(FinishArgs A, const float* limit, const int32_t* src,
@@ -1149,7 +1155,7 @@ __global__ __launch_bounds__(64) void k_wide_finish_any(FinishArgs A, const floa
     const uint32_t all = *A.n;
     const uint32_t total = min(all, A.cap);
     if (blockIdx.x >= total) return;
-    uint64_t nfetch = 0;
+    Fetches nfetch;
     for (uint32_t i = blockIdx.x; i < total; i += gridDim.x) finish_any(A, A.ids[i], L, limit, src, dst, ovis, nfetch);
     if (all > A.cap) {  // the list ran over: find the marked rays
         const int64_t nrays = A.nrays_dev ? (int64_t)*A.nrays_dev : A.nrays;
@@ -1159,7 +1165,7 @@ __global__ __launch_bounds__(64) void k_wide_finish_any(FinishArgs A, const floa
                 finish_any(A, b + __ffsll((long long)m) - 1, L, limit, src, dst, ovis, nfetch);
         }
     }
-    add_fetches(A.fetched, nfetch);
+    add_fetches(A.fetched, nfetch.nodes, nfetch.tris);
 }
 
 constexpr int kFinishBlocks = 4096;

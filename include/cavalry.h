@@ -51,6 +51,8 @@ const char* cav_version(void);
 /* Per-stage device time of the last build (HIP events on the context stream)
  * and the SAH cost of the root before and after treelet restructuring. */
 typedef struct {
+    /* ms_total also holds the wide tree that the traces walk (cav_trace_launch);
+     * its stages are cav_bvh_kernel_times' entries named wide_*. */
     float ms_bounds, ms_morton, ms_sort, ms_karras, ms_refit, ms_treelet, ms_flatten, ms_total;
     float root_cost_lbvh, root_cost_final;
     int n, morton_bits, opt_rounds;
@@ -151,6 +153,12 @@ int cav_trace_counters(cav_ctx* ctx, const cav_bvh* bvh, uint32_t* out, int32_t 
  * in the reference; it measures the algorithmic traffic of BVH::intersect /
  * testVisibility (BVH/BVH.h:23-189). */
 int cav_trace_fetches(cav_ctx* ctx, const cav_bvh* bvh, uint64_t* out, int32_t reset);
+/* Which tree a BVH's traces walk (out holds 4 words): out[0] / out[1] = 1 when
+ * closest-hit / any-hit traces of the launch shape `which` (CAV_TRACE_*) walk
+ * the wide tree (see cav_trace_launch), 0 the reference's; out[2] / out[3] =
+ * how many of cav_trace_fetches' records were triangles of the wide tree
+ * (closest-hit / any-hit). reset != 0 clears out[2..3] after reading. */
+int cav_trace_wide(cav_ctx* ctx, const cav_bvh* bvh, int32_t which, uint64_t* out, int32_t reset);
 /* The deepest leaf of the BVH, in edges from the root: no traversal can push
  * more stack entries than this, so a depth of at most 64 rules out overflow
  * (BVH/BVH.h:41,122). Computed on the device on each call. */

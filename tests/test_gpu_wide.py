@@ -271,3 +271,32 @@ def test_needles(ctx, ratio):
     bvh, nd = _tree(ctx, tris, 30, 0)
     _check(bvh, nd, tris, rays, lim, f"needles {ratio}")
     print(f"[wide] needles {ratio}: {bvh.trace_fetches()}", flush=True)
+
+
+def test_which_tree_is_walked_and_what_it_cost(ctx):
+    """trace_wide follows the launch shape and counts the triangles among the
+    fetches; the build's stages (ms_wide among them) add up to its total."""
+    tris = scenes.gmm_triangles(50000, seed=17, edge=0.01)
+    bvh = BVH.build(ctx, tris, optimization_rounds=2)
+    rays = scenes.random_rays(20000, seed=18, lo=0.0, hi=1.0)
+    lim = scenes.shadow_limits(len(rays), seed=19)
+    saved = tune.get_launch(ctx, tune.STANDALONE)
+    try:
+        for change, closest, occluded in (({}, True, True), ({"handoff_steps": 1 << 30}, False, False),
+                                          ({"any_hit_step": 2}, True, False), ({"any_hit_whole_line": 1}, True, False)):
+            tune.set_launch(ctx, tune.STANDALONE, dict(saved, **change))
+            bvh.trace_fetches(reset=True)
+            bvh.trace_wide(reset=True)
+            bvh.intersect(rays)
+            bvh.test_visibility(rays, lim)
+            f, w = bvh.trace_fetches(), bvh.trace_wide()
+            assert (w["closest"], w["occluded"]) == (closest, occluded), change
+            for k in ("closest", "occluded"):
+                assert (0 < w[k + "_triangles"] < f[k]) == w[k] and (w[k] or w[k + "_triangles"] == 0)
+    finally:
+        tune.set_launch(ctx, tune.STANDALONE, saved)
+    st = bvh.stats()
+    stages = sum(v for k, v in st.items() if k.startswith("ms_") and k != "ms_total")
+    other = sum(ms for name, ms in bvh.kernel_times() if name in ("readback", "levels"))
+    print(f"[wide] stages {stages:.4f} + {other:.4f} of {st['ms_total']:.4f} ms, wide {st['ms_wide']:.4f}", flush=True)
+    assert st["ms_wide"] > 0 and abs(stages + other - st["ms_total"]) < 0.02 * st["ms_total"]
