@@ -5,22 +5,27 @@ The persistent traversal kernels can run with any workgroup size (64, 128 or
 256 threads), any number of workgroups per CU, any ray-dispenser chunk and
 32 or 48 stack entries in LDS; the per-sample shading kernels of the render
 loops (path shading, the RL integrator's Q-table sampling) with any of the
-same workgroup sizes. Every ray's node order is the reference's
+same workgroup sizes. Every ray's answer is that of the reference's order
 (BVH/BVH.h:23-189) and every sample's shading is its own either way, so the
 choice changes only the speed (the reference fixes 256 threads at compile
-time, Utils/GpuCommons.h:63). Which shape is fastest depends on the batch and
-the tree: big incoherent batches over trees much larger than L2 prefer fewer
-rays in flight (less L2 thrash), small or coherent ones prefer more
-(latency).
+time, Utils/GpuCommons.h:63).
+
+Traces walk a wide tree unless the shape asks for the reference's (no
+hand-off; sibling pairs or whole lines for any-hit; see cav_trace_launch).
+Over the wide tree the grid and the stack are the kernels' own, so the
+workgroups per CU and the LDS stack are searched only for shapes that walk
+the reference's, where the fastest depends on the batch and the tree: big
+incoherent batches over trees much larger than L2 prefer fewer rays in flight
+(less L2 thrash), small or coherent ones prefer more (latency).
 
 `tune_trace` times candidate shapes on the caller's own rays (closest-hit and
 any-hit, best of `reps`), by coordinate descent from the current shape over
-workgroup size (at the same waves per CU), workgroups per CU, chunk, LDS
-depth, the steps after which a ray still in flight at the end of a launch
+workgroup size (at the same waves per CU), chunk, the workgroups per CU and
+LDS depth where they matter, the steps after which a ray still in flight at the end of a launch
 goes to a cooperative pass (a whole wave per ray) and whether an any-hit
 step fetches one node or a pair of siblings, sets the fastest on the
-context and records it in a JSON cache keyed by device, tree size and batch
-size. A later call with the same key reuses
+context and records it in a JSON cache keyed by device, traversal, tree size
+and batch size. A later call with the same key reuses
 the cached shape without timing (`use_cache`). `tune_render` does the same
 for the render loops (WAVEFRONT) on one render, and also descends over the
 shading workgroup size.
@@ -52,6 +57,11 @@ HANDOFFS = (256, 1024, 4096, 1 << 30)  # steps before a ray still in flight at t
 LDS = (32, 48)
 ANY_STEPS = (1, 2)              # any-hit step: one node, or a pair of sibling nodes (0: one node)
 ROUNDS = (0, 1, 2, 3, 4, 6, 8)
+
+
+# In every cache key: what was timed. Shapes (and round counts) chosen for
+# other traversals may be the slowest for this one.
+TRAVERSAL = "wide8"
 
 
 def default_cache_path() -> str:
@@ -113,6 +123,10 @@ def _store(path: str, key: str, entry: dict) -> None:
     os.replace(tmp, path)
 
 
+def _cache_key(*parts: str) -> str:
+    return "|".join((_device_name(), TRAVERSAL) + parts)
+
+
 def _key(shape: dict) -> str:
     return (f"{shape['workgroups_per_cu']}/{shape['ray_chunk']}/{shape['lds_stack']}/"
             f"{shape.get('workgroup_size', 256) or 256}/{shape.get('shade_workgroup_size', 256) or 256}/"
@@ -135,12 +149,21 @@ def _per_cu_for(size: int) -> tuple:
     return tuple(w * 64 // size for w in WAVES)
 
 
-def _descend(ctx, which: int, timer, start: dict, reps: int, shade: bool = False) -> tuple[dict, dict]:
+def _descend(ctx, which: int, timer, start: dict, reps: int, shade: bool = False,
+             wide=None) -> tuple[dict, dict]:
     """Coordinate descent from `start` over the workgroup size (keeping the
     waves per CU), workgroups per CU, chunk, LDS depth, hand-off steps, the
     any-hit step and, with `shade`, the shading workgroup size; returns the best shape and
-    every timing taken (ms)."""
+    every timing taken (ms). wide: tells whether the traces walk the wide tree
+    under the shape that is set (None: never); workgroups per CU and LDS depth
+    are then left as they are."""
     timings = {}
+
+    def walks_wide(shape):
+        if wide is None:
+            return False
+        set_launch(ctx, which, shape)
+        return wide()
 
     def measure(shape):
         k = _key(shape)
@@ -158,15 +181,21 @@ def _descend(ctx, which: int, timer, start: dict, reps: int, shade: bool = False
     for b in SIZES:
         w = waves(best)
         per = max(1, w * 64 // b) if w else 0
-        cand = dict(best, workgroup_size=b, workgroups_per_cu=per)
+        cand = dict(best, workgroup_size=b)
+        if not walks_wide(best):
+            cand["workgroups_per_cu"] = per
         ms = measure(cand)
         if ms < best_ms:
             best, best_ms = cand, ms
     fields = [("workgroups_per_cu", None), ("ray_chunk", CHUNKS), ("lds_stack", LDS), ("handoff_steps", HANDOFFS),
               ("any_hit_step", ANY_STEPS)]
+    if wide is not None:  # what decides the tree first
+        fields = fields[3:] + fields[:3]
     if shade:
         fields.append(("shade_workgroup_size", SIZES))
     for field, values in fields:
+        if field in ("workgroups_per_cu", "lds_stack") and walks_wide(best):
+            continue
         for v in (values if values is not None else _per_cu_for(best["workgroup_size"])):
             cand = dict(best, **{field: v})
             ms = measure(cand)
@@ -185,7 +214,7 @@ def tune_trace(ctx, bvh, rays, nrays: int, shadow_rays=None, limit=None, reps: i
     import torch
 
     path = cache_path or default_cache_path()
-    key = f"{_device_name()}|standalone|tris={_size_class(bvh.n)}|rays={_size_class(nrays)}"
+    key = _cache_key("standalone", f"tris={_size_class(bvh.n)}", f"rays={_size_class(nrays)}")
     if use_cache:
         hit = _load(path).get("entries", {}).get(key)
         if hit:
@@ -209,7 +238,11 @@ def tune_trace(ctx, bvh, rays, nrays: int, shadow_rays=None, limit=None, reps: i
         ctx.synchronize()
         return (time.perf_counter() - t0) * 1e3
 
-    best, timings = _descend(ctx, STANDALONE, timer, get_launch(ctx, STANDALONE), reps)
+    def wide():
+        w = bvh.trace_wide(STANDALONE)
+        return w["closest"] and (w["occluded"] or shadow_rays is None)
+
+    best, timings = _descend(ctx, STANDALONE, timer, get_launch(ctx, STANDALONE), reps, wide=wide)
     entry = {"shape": best, "ms": timings[_key(best)], "timings": timings,
              "when": time.strftime("%Y-%m-%d %H:%M:%S")}
     _store(path, key, entry)
@@ -229,8 +262,8 @@ def tune_render(ctx, scene, spp: int, integrator: str = "path", camera=None, max
     if cam is None:
         cam = for_scene(scene.arrays)
     ntris = len(scene.arrays.tris) if scene.arrays is not None else 0
-    key = (f"{_device_name()}|wavefront|{integrator}|tris={_size_class(ntris)}|"
-           f"samples={_size_class(cam.width * cam.height * spp)}")
+    key = _cache_key("wavefront", integrator, f"tris={_size_class(ntris)}",
+                     f"samples={_size_class(cam.width * cam.height * spp)}")
     if use_cache:
         hit = _load(path).get("entries", {}).get(key)
         if hit:
@@ -242,7 +275,12 @@ def tune_render(ctx, scene, spp: int, integrator: str = "path", camera=None, max
         _, st = render(ctx, scene, spp, integrator=integrator, camera=cam, max_depth=max_depth, **render_kw)
         return float(st["ms_total"])
 
-    best, timings = _descend(ctx, WAVEFRONT, timer, get_launch(ctx, WAVEFRONT), reps, shade=True)
+    def wide():
+        out = (ctypes.c_uint64 * 4)()
+        check(ctx.handle, lib().cav_trace_wide(ctx.handle, lib().cav_scene_bvh(scene.handle), WAVEFRONT, out, 0))
+        return bool(out[0] and out[1])
+
+    best, timings = _descend(ctx, WAVEFRONT, timer, get_launch(ctx, WAVEFRONT), reps, shade=True, wide=wide)
     entry = {"shape": best, "ms": timings[_key(best)], "timings": timings,
              "when": time.strftime("%Y-%m-%d %H:%M:%S")}
     _store(path, key, entry)
@@ -267,8 +305,8 @@ def tune_rounds(ctx, triangles, rays, shadow_rays=None, limit=None, traces: int 
 
     path = cache_path or default_cache_path()
     n, nrays = len(triangles), len(rays)
-    key = (f"{_device_name()}|rounds|tris={_size_class(n)}|rays={_size_class(nrays)}|traces={traces}|"
-           f"any={shadow_rays is not None}|cands={','.join(str(c) for c in candidates)}")
+    key = _cache_key("rounds", f"tris={_size_class(n)}", f"rays={_size_class(nrays)}", f"traces={traces}",
+                     f"any={shadow_rays is not None}", f"cands={','.join(str(c) for c in candidates)}")
     if use_cache:
         hit = _load(path).get("entries", {}).get(key)
         if hit:

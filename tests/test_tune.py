@@ -71,3 +71,56 @@ def test_cache_round_trip(tmp_path):
     assert set(data["entries"]) == {"k1", "k2"}
     assert tune._load(p)["entries"]["k1"]["shape"]["lds_stack"] == 48
     assert tune._load(str(tmp_path / "missing.json")) == {}
+
+
+def test_descent_over_the_wide_tree(monkeypatch):
+    """Where the traces walk the wide tree, workgroups per CU and LDS depth do
+    nothing: they keep their values, whatever noise the timer adds, unless the
+    search ends at a shape that walks the reference's tree."""
+    cur, tried = {}, []
+
+    def setter(ctx, which, shape):
+        cur.clear()
+        cur.update(shape)
+
+    monkeypatch.setattr(tune, "set_launch", setter)
+    start = {"workgroups_per_cu": 5, "ray_chunk": 256, "lds_stack": 32}
+    wide = lambda: cur["handoff_steps"] < 1 << 30 and cur["any_hit_step"] != 2
+
+    def timer(ref):  # the reference's tree takes `ref` times as long; per_cu and lds lure
+        tried.append(dict(cur))
+        return (1.0 if wide() else ref) + 0.01 * cur["workgroups_per_cu"] + (0.1 if cur["lds_stack"] == 32 else 0)
+
+    best, _ = tune._descend(None, tune.STANDALONE, lambda: timer(100.0), start, reps=1, wide=wide)
+    assert (best["workgroups_per_cu"], best["lds_stack"]) == (5, 32) and best["handoff_steps"] < 1 << 30
+    assert {(s["workgroups_per_cu"], s["lds_stack"]) for s in tried} == {(5, 32)}
+    best, _ = tune._descend(None, tune.STANDALONE, lambda: timer(0.1), start, reps=1, wide=wide)
+    assert not wide() and best["lds_stack"] == 48 and best["workgroups_per_cu"] == min(tune._per_cu_for(best["workgroup_size"]))
+
+
+def test_cached_shapes_of_other_traversals_are_not_reused(monkeypatch, tmp_path):
+    """An entry stored when traces walked the reference's tree (its key named no
+    traversal) is not applied: its sibling pairs would switch the wide tree off."""
+    p = str(tmp_path / "t.json")
+    shape = {"workgroups_per_cu": 2, "ray_chunk": 128, "lds_stack": 48, "any_hit_step": 2}
+    for old in ("standalone|tris=2^20|rays=2^20", "rounds|tris=2^20|rays=2^20|traces=1|any=False|cands=0,1"):
+        tune._store(p, f"{tune._device_name()}|{old}", {"shape": shape, "ms": 1.0, "rounds": 1})
+    applied = []
+    monkeypatch.setattr(tune, "set_launch", lambda ctx, which, s: applied.append(s))
+
+    class Bvh:
+        n = 1 << 20
+
+    class Timed(Exception):
+        pass
+
+    def timed(*a, **k):
+        raise Timed
+
+    import torch
+    monkeypatch.setattr(torch, "empty", timed)  # (the first thing it does when it has to time)
+    try:
+        tune.tune_trace(None, Bvh, None, 1 << 20, cache_path=p)
+        assert False
+    except Timed:
+        assert not applied
