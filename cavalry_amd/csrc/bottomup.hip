@@ -167,7 +167,8 @@ __global__ __launch_bounds__(kBlock) void k_bottom_up(const K* __restrict__ code
                                                       const uint32_t* __restrict__ order,
                                                       const float* __restrict__ tris,
                                                       NodeBox* nbox, int4* topo, uint32_t* hw,
-                                                      unsigned long long* gate64) {
+                                                      unsigned long long* gate64, const uint32_t* err) {
+    if (err && *err) return;
     __shared__ K skey[kBlock + 2];        // codes of positions k0-1 .. k0+256
     __shared__ int sdel[kBlock + 1];      // delta of boundaries k0-1 .. k0+255 (-1: none)
     __shared__ int wmin[kBlock / 64];
@@ -301,7 +302,9 @@ __global__ __launch_bounds__(kBlock) void k_bottom_up(const K* __restrict__ code
 // arrival word added to the gate) lets that child's climb continue. The
 // node ids, parents and boxes are those of pass 1's rule.
 __global__ __launch_bounds__(kBlock) void k_climb_crossing(int n, int nedges, NodeBox* nbox, int4* topo,
-                                                           uint32_t* hw, unsigned long long* gate64) {
+                                                           uint32_t* hw, unsigned long long* gate64,
+                                                           const uint32_t* err) {
+    if (err && *err) return;
     const int e = blockIdx.x * kBlock + threadIdx.x + 1;  // the edge between workgroups e-1 and e
     if (e > nedges) return;
     unsigned long long* edge = gate64 + n;  // two arrival words per edge split
@@ -400,16 +403,16 @@ hipError_t bottom_up_tree(const void* codes, int keybits, const float* tris, int
     if (keybits > 32)
         hipLaunchKernelGGL(k_bottom_up<uint64_t>, dim3(nb), dim3(kBlock), 0, s,
                            static_cast<const uint64_t*>(codes), n, keybits, o.order, tris, o.nbox, o.topo,
-                           o.hw, o.gate64);
+                           o.hw, o.gate64, o.err);
     else
         hipLaunchKernelGGL(k_bottom_up<uint32_t>, dim3(nb), dim3(kBlock), 0, s,
                            static_cast<const uint32_t*>(codes), n, keybits, o.order, tris, o.nbox, o.topo,
-                           o.hw, o.gate64);
+                           o.hw, o.gate64, o.err);
     mark(mk, "refit_bottom_up");
     const int nedges = nb - 1;
     if (nedges > 0) {
         hipLaunchKernelGGL(k_climb_crossing, dim3((unsigned)((nedges + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
-                           n, nedges, o.nbox, o.topo, o.hw, o.gate64);
+                           n, nedges, o.nbox, o.topo, o.hw, o.gate64, o.err);
         mark(mk, "refit_crossing");
     }
     return hipGetLastError();
@@ -417,7 +420,8 @@ hipError_t bottom_up_tree(const void* codes, int keybits, const float* tris, int
 
 hipError_t lbvh_bottom_up(LbvhBuffers& b, const void* codes, int keybits, const float* tris, int n,
                           hipStream_t s, Marker* mk) {
-    return bottom_up_tree(codes, keybits, tris, n, BottomUpOut{b.order, b.nbox, b.topo, b.visited, b.gate64}, s, mk);
+    return bottom_up_tree(codes, keybits, tris, n, BottomUpOut{b.order, b.nbox, b.topo, b.visited, b.gate64, nullptr},
+                          s, mk);
 }
 
 }  // namespace cav

@@ -81,6 +81,7 @@ struct BottomUpOut {
     int4* topo;                  // 2n-1
     uint32_t* hw;                // 2n-1 heights of the inner nodes
     unsigned long long* gate64;  // bottom_up_gate_words(n), zero before and after
+    const uint32_t* err;         // set: the order is not one, nothing is built (null: not looked at)
 };
 hipError_t bottom_up_tree(const void* codes, int keybits, const float* tris, int n, const BottomUpOut& o,
                           hipStream_t s, Marker* mk);
@@ -103,12 +104,14 @@ hipError_t treelet_round_impl(LbvhBuffers& b, int n, hipStream_t s, Marker* mk);
 // ray reached (atomic max, never reset by a launch); the 64-bit words at
 // counters[16] (closest) and counters[18] (occluded) add up the records
 // every launch fetched, those at counters[32] and counters[34] the wide
-// tree's triangles among them (never reset by a launch); counters[20..25]
+// tree's triangles among them (never reset by a launch); counters[36] counts
+// look-backs of the render loops' sorts that gave up; counters[20..25]
 // are the cooperative any-hit pass's spill count, spill cursor, failure
 // count and ray dispenser, counters[26..30] the cooperative closest-hit
 // pass's long-ray count, cursor, phase-3 ray dispenser (64-bit, 28-29) and
 // phase-3 count (all cleared by each launch).
 constexpr size_t kTraceCounterBytes = 256;
+constexpr int kSortErrWord = 36;
 // Launch shape of the persistent traversal kernels (and, for the render
 // loops, of the per-sample shading kernels). Each ray's node order is fixed
 // and each sample's shading is independent of where it runs, so results do

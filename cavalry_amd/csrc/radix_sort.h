@@ -8,7 +8,11 @@
 namespace cav {
 
 // Sort of the first min(cap, *n_dev) pairs.
-constexpr int kCountedSortWords = 8 * 256 + 8;  // digit counts and tile counters of up to 8 passes
+// Digit counts and tile counters of up to 8 passes, and the failure word:
+// nonzero after the sort when a look-back wait exceeded its bound (what the
+// sort left is no order then).
+constexpr int kCountedSortErr = 8 * 256 + 8;
+constexpr int kCountedSortWords = kCountedSortErr + 1;
 template <typename K>
 struct CountedSort {
     K* keys[2] = {nullptr, nullptr};              // keys[0] holds the input
@@ -16,7 +20,6 @@ struct CountedSort {
     uint32_t* work = nullptr;                     // kCountedSortWords, zero before the sort
     uint64_t* status[2] = {nullptr, nullptr};     // counted_sort_status_bytes(cap) each
     const uint32_t* n_dev = nullptr;
-    uint32_t* err = nullptr;                      // nonzero: a look-back wait exceeded its bound
     int result = 0;                               // index of the buffer holding the output
 };
 

@@ -321,7 +321,7 @@ hipError_t counted_impl(CountedSort<K>& b, int64_t cap, int key_bits, LaunchSink
     for (int p = 0; p < passes; ++p) {
         ls.launch("k_onesweep", &k_onesweep<K, S, kOsSmall>, dim3((unsigned)sort_tiles(cap)), dim3(kOsSmall),
                   b.keys[cur], b.vals[cur], b.keys[cur ^ 1], b.vals[cur ^ 1], cap, b.n_dev, 8 * p,
-                  b.work + p * kRadix, b.status[p & 1], b.status[(p & 1) ^ 1], b.work + kRadix * 8 + p, b.err);
+                  b.work + p * kRadix, b.status[p & 1], b.status[(p & 1) ^ 1], b.work + kRadix * 8 + p, b.work + kCountedSortErr);
         cur ^= 1;
     }
     b.result = cur;

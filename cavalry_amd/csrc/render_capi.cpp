@@ -601,7 +601,7 @@ int cav_render(cav_ctx* ctx, cav_scene* sc, const cav_camera* cam, const cav_ren
     a.film_f64 = (prm->flags & CAV_RENDER_FILM_F64) != 0;
     hipStream_t s = ctx->stream;
     RCHK(ctx, hipMemsetAsync(a.rays, 0, 16, s));
-    RCHK(ctx, hipMemsetAsync(a.trace_counters, 0, 32, s));
+    RCHK(ctx, hipMemsetAsync(a.trace_counters, 0, kTraceCounterBytes, s));
     RCHK(ctx, hipEventRecord(rs->ev[0], s));
     RlArgs r = rs->rl;
     if (!det) {
@@ -626,11 +626,12 @@ int cav_render(cav_ctx* ctx, cav_scene* sc, const cav_camera* cam, const cav_ren
     RCHK(ctx, hipGetLastError());
     RCHK(ctx, hipEventRecord(rs->ev[1], s));
     unsigned long long tally[2] = {0, 0};
-    uint32_t tc[2] = {0, 0};
+    uint32_t tc[2] = {0, 0}, sort_err = 0;
     RCHK(ctx, hipMemcpyAsync(film_rgb, a.film_rgb, 12 * (size_t)npix, hipMemcpyDeviceToHost, s));
     RCHK(ctx, hipMemcpyAsync(film_weight, a.film_w, 4 * (size_t)npix, hipMemcpyDeviceToHost, s));
     RCHK(ctx, hipMemcpyAsync(tally, a.rays, 16, hipMemcpyDeviceToHost, s));
     RCHK(ctx, hipMemcpyAsync(tc, a.trace_counters, 8, hipMemcpyDeviceToHost, s));
+    RCHK(ctx, hipMemcpyAsync(&sort_err, a.trace_counters + kSortErrWord, 4, hipMemcpyDeviceToHost, s));
     RCHK(ctx, hipStreamSynchronize(s));
     float ms = 0.f;
     RCHK(ctx, hipEventElapsedTime(&ms, rs->ev[0], rs->ev[1]));
@@ -641,6 +642,7 @@ int cav_render(cav_ctx* ctx, cav_scene* sc, const cav_camera* cam, const cav_ren
         stats->mrays_per_s = ms > 0 ? (double)(tally[0] + tally[1]) / (ms * 1e3) : 0.0;
         stats->rounds = rounds;
     }
+    if (sort_err) return fail(ctx, CAV_ERR_HIP, "radix sort: a look-back wait exceeded its bound while rendering");
     if (tc[0] || tc[1]) return fail(ctx, CAV_ERR_OVERFLOW, "traversal stack overflow while rendering");
     return CAV_OK;
 }

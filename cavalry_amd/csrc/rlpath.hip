@@ -1227,6 +1227,14 @@ __global__ __launch_bounds__(kBlock) void k_entry_keys(SceneDev sc, Grid gr, Que
     vals[i] = (uint32_t)i;
 }
 
+// Whether a sort gave up on a look-back: what it left is not used then, and
+// the render (the served request) ends with an error.
+__device__ __forceinline__ bool sort_failed(const uint32_t* err, uint32_t* failures) {
+    if (*err == 0u) return false;
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(failures, 1u);
+    return true;
+}
+
 // The bounce's tasks and hits copied into shading order, so that the three
 // kernels that follow read and write them in line. Reading them through the
 // order each time took the kernels 64-byte fetches for 4-byte words. The
@@ -1242,10 +1250,12 @@ struct RlHits {
 __global__ __launch_bounds__(kBlock) void k_gather(const uint32_t* __restrict__ count, const uint32_t* perm, Queue qi,
                                                    RlQueue ri, const int32_t* __restrict__ hit_prim,
                                                    const float* __restrict__ hit_t, const float* __restrict__ hit_u,
-                                                   const float* __restrict__ hit_v, Queue qo, RlQueue ro, RlHits ho) {
+                                                   const float* __restrict__ hit_v, Queue qo, RlQueue ro, RlHits ho,
+                                                   const uint32_t* err, uint32_t* failures) {
     const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (j >= (int64_t)*count) return;
-    const int64_t i = (int64_t)perm[j];
+    const bool failed = sort_failed(err, failures);
+    const int64_t i = failed ? j : (int64_t)perm[j];
     const float2* r = reinterpret_cast<const float2*>(qi.ray + i * 6);
     const float2 r0 = r[0], r1 = r[1], r2 = r[2];
     const float m0 = qi.mult[i * 3], m1 = qi.mult[i * 3 + 1], m2 = qi.mult[i * 3 + 2];
@@ -1275,9 +1285,6 @@ __global__ __launch_bounds__(kBlock) void k_gather(const uint32_t* __restrict__ 
 // Zeroes for a counted sort. Deterministic mode, before k_qdist: no records
 // yet either (count; k_qdist appends them, the sort takes only the appended
 // ones).
-// A look-back that waits past its bound counts as a traversal failure: the
-// render (the served request) ends with an error.
-inline uint32_t* sort_err(uint32_t* trace_counters) { return trace_counters + 1; }
 constexpr int kResetBlock = 1024;
 __global__ __launch_bounds__(kResetBlock) void k_sort_reset(uint32_t* work, uint32_t* count) {
     for (int i = threadIdx.x; i < kCountedSortWords; i += kResetBlock) work[i] = 0u;
@@ -1303,7 +1310,9 @@ template <class Tab>
 __global__ __launch_bounds__(kBlock) void k_rec_sum(const uint64_t* __restrict__ keys,
                                                     const uint32_t* __restrict__ idx,
                                                     const float* __restrict__ val, const uint32_t* count,
-                                                    int64_t cap, Tab tab, int nlights) {
+                                                    int64_t cap, Tab tab, int nlights, const uint32_t* err,
+                                                    uint32_t* failures) {
+    if (sort_failed(err, failures)) return;
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const int64_t n = (int64_t)*count < cap ? (int64_t)*count : cap;
     if (i >= n) return;
@@ -1332,18 +1341,18 @@ __global__ __launch_bounds__(kBlock) void k_rec_sum(const uint64_t* __restrict__
 // Sorts a bounce's records by key (only the appended ones) and sums them.
 template <class Tab>
 hipError_t rec_sort_sum(uint64_t* const keys[2], uint32_t* const idx[2], float* val, uint32_t* count,
-                        uint32_t* work, uint64_t* status0, uint64_t* status1, uint32_t* err, int64_t cap, Tab tab,
+                        uint32_t* work, uint64_t* status0, uint64_t* status1, uint32_t* failures, int64_t cap, Tab tab,
                         int nlights, LaunchSink& ls) {
     CountedSort<uint64_t> sb;
     sb.keys[0] = keys[0]; sb.keys[1] = keys[1];
     sb.vals[0] = idx[0]; sb.vals[1] = idx[1];
     sb.work = work; sb.status[0] = status0; sb.status[1] = status1;
     sb.n_dev = count;
-    sb.err = err;
     hipError_t e = sort_pairs_counted(sb, cap, 64, ls);
     if (e != hipSuccess) return e;
     ls.launch("k_rec_sum", &k_rec_sum<Tab>, dim3((unsigned)((cap + kBlock - 1) / kBlock)), dim3(kBlock),
-              sb.keys[sb.result], sb.vals[sb.result], val, count, cap, tab, nlights);
+              sb.keys[sb.result], sb.vals[sb.result], val, count, cap, tab, nlights,
+              (const uint32_t*)(work + kCountedSortErr), failures);
     return ls.err;
 }
 
@@ -1398,7 +1407,6 @@ hipError_t render_rlpath(const RenderArgs& a, const RlArgs& rl, bool init_tables
             sb.vals[0] = rl.svals[0]; sb.vals[1] = rl.svals[1];
             sb.work = rl.swork; sb.status[0] = rl.sstatus[0]; sb.status[1] = rl.sstatus[1];
             sb.n_dev = a.counts + qin;
-            sb.err = sort_err(a.trace_counters);
             int bits = 1;
             while (((int64_t)1 << bits) < 8 * nent) ++bits;
             if ((e = sort_pairs_counted(sb, nsamp, bits, ls)) != hipSuccess) return e;
@@ -1407,7 +1415,8 @@ hipError_t render_rlpath(const RenderArgs& a, const RlArgs& rl, bool init_tables
                          hu ? (float*)rl.skeys[1] : nullptr};
             ls.launch("k_gather", &k_gather, dim3(nb), dim3(kBlock), (const uint32_t*)(a.counts + qin),
                       (const uint32_t*)sb.vals[sb.result], a.q[from], rl.q[from], (const int32_t*)a.hit_prim,
-                      (const float*)a.hit_t, (const float*)hu, (const float*)hv, a.q[at], rl.q[at], hit);
+                      (const float*)a.hit_t, (const float*)hu, (const float*)hv, a.q[at], rl.q[at], hit,
+                      (const uint32_t*)(rl.swork + kCountedSortErr), a.trace_counters + kSortErrWord);
         }
         const int to = at ^ 1;
         ls.launch("k_lighting", &k_lighting<RenderSrc>, dim3(nb), dim3(kBlock), src, a.scene, a.halton, a.q[at],
@@ -1422,7 +1431,7 @@ hipError_t render_rlpath(const RenderArgs& a, const RlArgs& rl, bool init_tables
                                 rl.q[at], rl.slots, a.vis, hit.prim, hit.t, hit.u, hit.v, a.counts, qin, rec);
         if (rec.keys &&
             (e = rec_sort_sum(rl.rec_keys, rl.rec_idx, rl.rec_val, rl.rec_count, rl.rec_work, rl.rec_status[0],
-                              rl.rec_status[1], sort_err(a.trace_counters), rl.rec_cap, RenderTables{t}, L, ls)) !=
+                              rl.rec_status[1], a.trace_counters + kSortErrWord, rl.rec_cap, RenderTables{t}, L, ls)) !=
                 hipSuccess)
             return e;
         hipLaunchKernelGGL(k_finish_q, dim3((unsigned)((nent + kEntryWaves - 1) / kEntryWaves)),
@@ -1477,7 +1486,7 @@ void pool_rl_learn(const PoolDev& p, int qin, bool det, LaunchSink& ls) {
                           p.rl.q[qin], p.rl.sl, p.vis, p.hit_prim, p.hit_t, hu, hv, p.counts, qin, rec);
     if (det)
         (void)rec_sort_sum(p.rl.rec_keys, p.rl.rec_idx, p.rl.rec_val, p.rl.rec_count, p.rl.rec_work, p.rl.rec_status[0],
-                           p.rl.rec_status[1], sort_err(p.trace_counters), p.rl.rec_cap, PoolTables{p.rl.req},
+                           p.rl.rec_status[1], p.trace_counters + kSortErrWord, p.rl.rec_cap, PoolTables{p.rl.req},
                            p.scene.nlights, ls);
     // the updates of every request with hits
     ls.launch("k_pool_finish_q", &k_pool_finish_q, dim3(kPoolFinishBlocks), dim3(64 * kEntryWaves),

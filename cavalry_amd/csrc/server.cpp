@@ -131,7 +131,7 @@ struct Request {
     float *res = nullptr, *sxy = nullptr, *rgb = nullptr, *w = nullptr;
     float4* partial = nullptr;
     float *h_rgb = nullptr, *h_w = nullptr;
-    uint32_t* h_ovf = nullptr;  // pool overflow counters at admission [0..1] and at the end [2..3]
+    uint32_t* h_ovf = nullptr;  // pool overflow counters at admission [0..1] and at the end [2..3], sort failures [4], [5]
     hipEvent_t ready = nullptr;
     bool finishing = false;
     bool cancel = false;
@@ -403,7 +403,7 @@ bool activate(cav_server* sv, Pool* p, Request* r) {
     char* h = sv->host_arena.at(hoff);
     r->h_rgb = reinterpret_cast<float*>(carve(h, 12 * P));
     r->h_w = reinterpret_cast<float*>(carve(h, 4 * P));
-    r->h_ovf = reinterpret_cast<uint32_t*>(carve(h, 16));
+    r->h_ovf = reinterpret_cast<uint32_t*>(carve(h, 24));
     r->dev_off = doff; r->dev_len = dlen; r->host_off = hoff; r->host_len = hlen;
     r->slot = slot;
     p->slots[slot] = r;
@@ -426,6 +426,8 @@ bool activate(cav_server* sv, Pool* p, Request* r) {
     // the pool's overflow counters before the request's first bounce
     if (he == hipSuccess)
         he = hipMemcpyAsync(r->h_ovf, p->dev.trace_counters, 8, hipMemcpyDeviceToHost, p->stream);
+    if (he == hipSuccess)
+        he = hipMemcpyAsync(r->h_ovf + 4, p->dev.trace_counters + kSortErrWord, 4, hipMemcpyDeviceToHost, p->stream);
     if (he != hipSuccess) sv->error = hip_msg("request admission", he);
     r->active = true;
     return true;
@@ -583,6 +585,8 @@ int pool_step(cav_server* sv, Pool* p) {
             }
             if (e == hipSuccess) e = hipMemcpyAsync(r->h_w, r->w, 4 * (size_t)r->npix, hipMemcpyDeviceToHost, p->stream);
             if (e == hipSuccess) e = hipMemcpyAsync(r->h_ovf + 2, p->dev.trace_counters, 8, hipMemcpyDeviceToHost, p->stream);
+            if (e == hipSuccess)
+                e = hipMemcpyAsync(r->h_ovf + 5, p->dev.trace_counters + kSortErrWord, 4, hipMemcpyDeviceToHost, p->stream);
             if (e == hipSuccess) {
                 what = "request event";
                 e = hipEventCreateWithFlags(&r->ready, hipEventDisableTiming);
@@ -620,6 +624,10 @@ void finish_ready(cav_server* sv) {
             msg = hip_msg("request completion event", q);
         } else if (r->cancel) {
             st = CAV_SERVE_CANCELLED;
+        } else if (r->h_ovf[5] != r->h_ovf[4]) {
+            st = CAV_SERVE_FAILED;
+            err = CAV_ERR_HIP;
+            msg = "radix sort: a look-back wait exceeded its bound in the request's ray pool";
         } else if (ovf) {
             st = CAV_SERVE_FAILED;
             err = CAV_ERR_OVERFLOW;

@@ -88,6 +88,7 @@ struct WideBuild {
     const float* tris;
     const int32_t* mesh;
     const uint32_t* bounds;  // the triangles' box (order-preserving ints)
+    const uint32_t* err;     // set: the sort failed, nothing is built
     uint4* nodes;
     float4* wtris;
     uint32_t* ctr;
@@ -298,6 +299,7 @@ __device__ __forceinline__ uint32_t ctr_load(const uint32_t* p) {
 __global__ __launch_bounds__(1024) void k_wide_levels(WideBuild w, int skip, uint32_t limit) {
     __shared__ uint4 stage[16][40];
     const int wave = threadIdx.x >> 6, g = (threadIdx.x & 63) >> 3;
+    if (*w.err) return;
     const uint32_t min_unit = min_unit_of(w.bounds);
     int lvl = (int)ctr_load(w.ctr + kCtrTop) + skip;
     uint32_t start = 0;
@@ -321,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void k_wide_level(WideBuild w, int j) {
     __shared__ uint4 stage[kBlock / 64][40];
     const int wave = threadIdx.x >> 6, g = (threadIdx.x & 63) >> 3;
     const int lvl = (int)w.ctr[kCtrTop] + j;
-    if (lvl >= kMaxWideLevels) return;
+    if (lvl >= kMaxWideLevels || *w.err) return;
     uint32_t start = 0;
     for (int k = 0; k < lvl; ++k) start += w.ctr[k];
     const uint32_t cnt = w.ctr[lvl], min_unit = min_unit_of(w.bounds);
@@ -389,11 +391,11 @@ hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, const float* tris, const i
     mark(mk, "wide_sort");
     const uint32_t* order = ob.vals[ob.result];
     // (the heights go to the level list, which only the treelet rounds use)
-    const BottomUpOut out{order, w.nbox, w.topo, b.lvl_list, w.gate};
+    const BottomUpOut out{order, w.nbox, w.topo, b.lvl_list, w.gate, ob.err};
     e = bottom_up_tree(ob.keys[ob.result], kCodeBits, tris, n, out, s, nullptr);
     if (e != hipSuccess) return e;
     mark(mk, "wide_tree");
-    const WideBuild wb{w.nbox, w.topo, order, tris, mesh, bounds, w.nodes, w.tris, w.ctr, n};
+    const WideBuild wb{w.nbox, w.topo, order, tris, mesh, bounds, ob.err, w.nodes, w.tris, w.ctr, n};
     // up to 512 nodes per level in one workgroup; then a launch per level
     // until all but a skewed tree's last few nodes are done; then those
     const bool small = n <= 4096;
