@@ -103,7 +103,6 @@ static int bvh_alloc(cav_ctx* ctx, cav_bvh* h, int n) {
     void* wide = nullptr;
     if (hipMalloc(&wide, wide_bytes(n)) == hipSuccess) {
         wide_carve(h->wide, wide, n);
-        HIPCHK(ctx, hipMemsetAsync(h->wide.gate, 0, sizeof(uint64_t) * bottom_up_gate_words(n), ctx->stream));
     } else {
         (void)hipGetLastError();
     }
@@ -161,15 +160,20 @@ static int bvh_run(cav_ctx* ctx, cav_bvh* h, const float* tris_dev, const float*
     mark(mk, "readback");
     for (int r = 0; r < opt_rounds; ++r) HIPCHK(ctx, treelet_round_impl(h->b, n, s, mk));
     if (opt_rounds > 0) HIPCHK(ctx, lbvh_refs(h->b, n, s, mk, "flatten_refs"));
-    HIPCHK(ctx, lbvh_flatten(h->b, tris_dev, h->mesh, n, opt_rounds == 0, h->rec, h->root, h->wide.leaf_of, s, mk));
+    const auto flatten = [&] {
+        return lbvh_flatten(h->b, tris_dev, h->mesh, n, opt_rounds == 0, h->rec, h->root, h->wide.leaf_of, s, mk);
+    };
+    const bool flat_first = !h->wide.base || h->wide.scratch;
+    if (flat_first) HIPCHK(ctx, flatten());
     const uint32_t* bounds = h->b.scene_ord;
     if (h->wide.base) {
         if (scene_bounds) {
             bounds = h->wide.bounds;
             HIPCHK(ctx, lbvh_scene_bounds(tris_dev, n, h->wide.bounds, h->b.bounds_part, s, nullptr));
         }
-        HIPCHK(ctx, wide_build(h->wide, h->b, tris_dev, h->mesh, n, bounds, s, mk));
+        HIPCHK(ctx, wide_build(h->wide, h->b, flat_first ? h->wide.scratch : h->rec, tris_dev, h->mesh, n, bounds, s, mk));
     }
+    if (!flat_first) HIPCHK(ctx, flatten());
     float root_final[8];
     uint32_t box[6], height = 0, wide_err = 0;
     HIPCHK(ctx, hipMemcpyAsync(box, bounds, sizeof box, hipMemcpyDeviceToHost, s));

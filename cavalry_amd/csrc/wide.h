@@ -54,16 +54,20 @@ __host__ __device__ inline WideScale wide_scale(const float* box6) {
     return WideScale{pow2(k + 20), pow2(104 - k), pow2(k - 16), (uint32_t)(e < 40 ? 40 : e)};
 }
 
-// Scratch and results of one build (library-owned, sized for n triangles).
+// Where a build keeps its codes and its binary tree (112 bytes a triangle).
+// Up to this many triangles in memory of their own: the traversal records are
+// then written before the wide tree, which the first traces find in the
+// caches (1M triangles, 131K rays: 1.36 ms a frame, 1.39 the other way
+// round). Above, where neither stays cached, in the place of those records,
+// which are written last.
+constexpr int kWideApart = 1 << 21;
+
+// The tree (library-owned, sized for n triangles): 89 bytes a triangle.
 struct WideBuffers {
-    void* base = nullptr;  // the one allocation that holds the rest
-    uint32_t* keys[2] = {nullptr, nullptr};
-    uint32_t* vals[2] = {nullptr, nullptr};
-    NodeBox* nbox = nullptr;             // the binary tree over the wide tree's codes
-    int4* topo = nullptr;
-    unsigned long long* gate = nullptr;  // bottom_up_gate_words(n), zero between builds
-    uint32_t* ctr = nullptr;             // kWideCtrWords
-    uint32_t* bounds = nullptr;          // 6 order-preserving ints: the triangles' box
+    void* base = nullptr;        // the one allocation that holds the rest
+    void* scratch = nullptr;     // wide_scratch_bytes(n), part of it (null above kWideApart)
+    uint32_t* ctr = nullptr;     // kWideCtrWords
+    uint32_t* bounds = nullptr;  // 6 order-preserving ints: the triangles' box
     uint4* nodes = nullptr;
     float4* tris = nullptr;
     int32_t* leaf_of = nullptr;
@@ -72,9 +76,11 @@ constexpr int kWideCtrWords = 96;
 size_t wide_bytes(int n);
 void wide_carve(WideBuffers& w, void* base, int n);
 // Builds the tree. bounds: the triangles' box (b.scene_ord when the caller
-// gave none, else w.bounds). Uses b's sort work space and level list as
-// scratch, on the same stream as b's own build and after it.
-hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, const float* tris, const int32_t* mesh, int n,
+// gave none, else w.bounds). Uses b's sort work space, gates and level list
+// and wide_scratch_bytes(n) at `scratch` on the same stream as b's own build
+// and after it.
+size_t wide_scratch_bytes(int n);
+hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, void* scratch, const float* tris, const int32_t* mesh, int n,
                       const uint32_t* bounds, hipStream_t s, Marker* mk);
 
 }  // namespace cav

@@ -75,6 +75,8 @@ __global__ __launch_bounds__(kBlock) void k_wide_codes(const float* __restrict__
 }
 
 // Sort histograms, tile counters and level counts to zero; the root's item.
+// (The failure word stays: where b's own sort failed, its gates may hold
+// arrivals and nothing is built.)
 __global__ void k_wide_init(uint32_t* hist, int nhist, uint32_t* ctr, uint4* nodes, int n) {
     for (int i = threadIdx.x; i < nhist; i += blockDim.x) hist[i] = 0u;
     for (int i = threadIdx.x; i < kWideCtrWords; i += blockDim.x) ctr[i] = i == 0 ? 1u : 0u;
@@ -339,51 +341,60 @@ size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 }  // namespace
 
 size_t wide_bytes(int n) {
-    const size_t N = (size_t)n, M = 2 * N - 1;
-    return 4 * up256(4 * N) + up256(sizeof(NodeBox) * M) + up256(sizeof(int4) * M) +
-           up256(8 * (size_t)bottom_up_gate_words(n)) + up256(4 * kWideCtrWords) + 256 +
-           up256(16 * kWideWords * (size_t)wide_node_capacity(n)) + up256(48 * N) + up256(4 * N);
+    const size_t N = (size_t)n;
+    return up256(4 * kWideCtrWords) + 256 + up256(16 * kWideWords * (size_t)wide_node_capacity(n)) + up256(48 * N) +
+           up256(4 * N) + (n <= kWideApart ? wide_scratch_bytes(n) : 0);
 }
+size_t wide_scratch_bytes(int n) {
+    const size_t N = (size_t)n, M = 2 * N - 1;
+    return 4 * up256(4 * N) + up256(sizeof(NodeBox) * M) + up256(sizeof(int4) * M);
+}
+
+namespace {
+struct Carver {
+    unsigned char* p;
+    template <typename T>
+    void take(T*& out, size_t bytes) {
+        out = reinterpret_cast<T*>(p);
+        p += up256(bytes);
+    }
+};
+}  // namespace
 
 void wide_carve(WideBuffers& w, void* base, int n) {
-    const size_t N = (size_t)n, M = 2 * N - 1;
-    unsigned char* p = static_cast<unsigned char*>(base);
-    const auto take = [&p](size_t bytes) {
-        void* q = p;
-        p += up256(bytes);
-        return q;
-    };
+    const size_t N = (size_t)n;
+    Carver c{static_cast<unsigned char*>(base)};
     w.base = base;
-    for (int k = 0; k < 2; ++k) {
-        w.keys[k] = static_cast<uint32_t*>(take(4 * N));
-        w.vals[k] = static_cast<uint32_t*>(take(4 * N));
-    }
-    w.nbox = static_cast<NodeBox*>(take(sizeof(NodeBox) * M));
-    w.topo = static_cast<int4*>(take(sizeof(int4) * M));
-    w.gate = static_cast<unsigned long long*>(take(8 * (size_t)bottom_up_gate_words(n)));
-    w.ctr = static_cast<uint32_t*>(take(4 * kWideCtrWords));
-    w.bounds = static_cast<uint32_t*>(take(64));
-    w.nodes = static_cast<uint4*>(take(16 * kWideWords * (size_t)wide_node_capacity(n)));
-    w.tris = static_cast<float4*>(take(48 * N));
-    w.leaf_of = static_cast<int32_t*>(take(4 * N));
+    c.take(w.ctr, 4 * kWideCtrWords);
+    c.take(w.bounds, 64);
+    c.take(w.nodes, 16 * kWideWords * (size_t)wide_node_capacity(n));
+    c.take(w.tris, 48 * N);
+    c.take(w.leaf_of, 4 * N);
+    w.scratch = n <= kWideApart ? c.p : nullptr;
 }
 
-hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, const float* tris, const int32_t* mesh, int n,
+hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, void* scratch, const float* tris, const int32_t* mesh, int n,
                       const uint32_t* bounds, hipStream_t s, Marker* mk) {
+    const size_t N = (size_t)n, M = 2 * N - 1;
     const int64_t tiles = onesweep_tiles(n);
     OnesweepBuffers<uint32_t> ob;
+    Carver c{static_cast<unsigned char*>(scratch)};
     for (int k = 0; k < 2; ++k) {
-        ob.keys[k] = w.keys[k];
-        ob.vals[k] = w.vals[k];
+        c.take(ob.keys[k], 4 * N);
+        c.take(ob.vals[k], 4 * N);
     }
+    NodeBox* nbox;
+    int4* topo;
+    c.take(nbox, sizeof(NodeBox) * M);
+    c.take(topo, sizeof(int4) * M);
     ob.hist = b.hist;
     ob.status = b.counts;
     ob.tile_ctr = b.hist + kSortHistWords;
     ob.err = b.hist + kSortHistWords + 8;
     int nb = (n + kBlock - 1) / kBlock;
     if (nb > kCodeBlocks) nb = kCodeBlocks;
-    hipLaunchKernelGGL(k_wide_init, dim3(1), dim3(1024), 0, s, b.hist, kSortHistWords + 16, w.ctr, w.nodes, n);
-    hipLaunchKernelGGL(k_wide_codes, dim3(nb), dim3(kBlock), 0, s, tris, (int64_t)n, bounds, ob.keys[0], w.vals[0],
+    hipLaunchKernelGGL(k_wide_init, dim3(1), dim3(1024), 0, s, b.hist, kSortHistWords + 8, w.ctr, w.nodes, n);
+    hipLaunchKernelGGL(k_wide_codes, dim3(nb), dim3(kBlock), 0, s, tris, (int64_t)n, bounds, ob.keys[0], ob.vals[0],
                        b.hist, b.counts, 4 * 256 * tiles);
     mark(mk, "wide_codes");
     hipError_t e = onesweep_sort_pairs(ob, n, kCodeBits, s, nullptr);
@@ -391,11 +402,11 @@ hipError_t wide_build(WideBuffers& w, LbvhBuffers& b, const float* tris, const i
     mark(mk, "wide_sort");
     const uint32_t* order = ob.vals[ob.result];
     // (the heights go to the level list, which only the treelet rounds use)
-    const BottomUpOut out{order, w.nbox, w.topo, b.lvl_list, w.gate, ob.err};
+    const BottomUpOut out{order, nbox, topo, b.lvl_list, b.gate64, ob.err};
     e = bottom_up_tree(ob.keys[ob.result], kCodeBits, tris, n, out, s, nullptr);
     if (e != hipSuccess) return e;
     mark(mk, "wide_tree");
-    const WideBuild wb{w.nbox, w.topo, order, tris, mesh, bounds, ob.err, w.nodes, w.tris, w.ctr, n};
+    const WideBuild wb{nbox, topo, order, tris, mesh, bounds, ob.err, w.nodes, w.tris, w.ctr, n};
     // up to 512 nodes per level in one workgroup; then a launch per level
     // until all but a skewed tree's last few nodes are done; then those
     const bool small = n <= 4096;

@@ -300,3 +300,35 @@ def test_which_tree_is_walked_and_what_it_cost(ctx):
     other = sum(ms for name, ms in bvh.kernel_times() if name in ("readback", "levels"))
     print(f"[wide] stages {stages:.4f} + {other:.4f} of {st['ms_total']:.4f} ms, wide {st['ms_wide']:.4f}", flush=True)
     assert st["ms_wide"] > 0 and abs(stages + other - st["ms_total"]) < 0.02 * st["ms_total"]
+
+
+@pytest.mark.parametrize("n", [(1 << 21) - 3, 1 << 21, (1 << 21) + 1])
+def test_build_in_the_place_of_the_records(ctx, n):
+    """Above 2^21 triangles the wide tree is built where the traversal records
+    go afterwards: its traces and the reference's (through those records) agree,
+    also after a rebuild, and a build holds less memory per triangle."""
+    import torch
+    tris = scenes.gmm_triangles(n, seed=n & 255, edge=2e-3)
+    dev = torch.from_numpy(tris).cuda()
+    rays = scenes.random_rays(50000, seed=20, lo=0.0, hi=1.0)
+    lim = scenes.shadow_limits(len(rays), seed=21)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    bvh = BVH.build(ctx, dev, device=True)
+    held = (free - torch.cuda.mem_get_info()[0]) / n
+    assert held < (500 if n <= 1 << 21 else 400)  # (371 and the allocations' rounding)
+    saved = tune.get_launch(ctx, tune.STANDALONE)
+    for again in (False, True):
+        if again:
+            bvh.rebuild(dev, optimization_rounds=1)
+        got, vis = bvh.intersect(rays), bvh.test_visibility(rays, lim)
+        try:
+            tune.set_launch(ctx, tune.STANDALONE, dict(saved, handoff_steps=1 << 30))
+            ref, rvis = bvh.intersect(rays), bvh.test_visibility(rays, lim)
+        finally:
+            tune.set_launch(ctx, tune.STANDALONE, saved)
+        print(f"[wide] n={n}: {held:.0f} bytes a triangle, {(ref['prim'] >= 0).sum()} hits", flush=True)
+        np.testing.assert_array_equal(got["prim"], ref["prim"])
+        np.testing.assert_array_equal(bits(got["t"]), bits(ref["t"]))
+        np.testing.assert_array_equal(vis, rvis)
+    bvh.close()
