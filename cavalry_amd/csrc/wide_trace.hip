@@ -327,7 +327,11 @@ struct WideList {           // rays left to the finishing pass
     uint32_t* n = nullptr;  // rays listed (past cap: the rest are marked in the hit ids)
     uint32_t cap = 0;
     int after = 0;          // steps before a ray still in flight at the batch's end is listed (0: never)
+    uint32_t mark = 0;      // whole_mark
 };
+// The bit of a closest-hit ray's id that says it has to be taken over its
+// whole line, where ids leave one for it (0: the pass finds out by itself).
+inline uint32_t whole_mark(int64_t nrays) { return nrays <= (int64_t(1) << 31) ? 1u << 31 : 0u; }
 
 // kAny: any-hit (limit, src, dst, ovis) instead of closest-hit (oprim ...).
 template <bool kAny, int B>
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
         const uint64_t idle = __ballot(ri == -1 || over);
         if (idle && (__popcll(idle) >= kRefill || !__ballot(ri >= 0 && !over))) {
             if (over) {
-                bool ask = odd;  // the finishing pass has to decide
+                bool ask = odd, whole = false;  // the finishing pass has to decide; over the whole line
                 int prim = -1;
                 if (bt >= 0) {
                     const float4* tp = tris + (int64_t)bt * 3;
@@ -378,8 +382,9 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                     ask = ask || touch || !(e >= 0.f);
                     if (!kAny) {
                         const float near = slack * unscale(r);
-                        ask = ask || rival <= fmx(best, e) || e > best * kOwnBox + 0.5f * near || !(best < FLT_MAX) ||
-                              thin || thin_hit(a, b, c, r.o, d, best, best * (kReach - 1.f) + near);
+                        whole = thin || thin_hit(a, b, c, r.o, d, best, best * (kReach - 1.f) + near);
+                        ask = ask || whole || rival <= fmx(best, e) || e > best * kOwnBox + 0.5f * near ||
+                              !(best < FLT_MAX);
                     }
                 }
                 if (kAny) {
@@ -392,7 +397,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                 }
                 if (ask) {
                     const uint32_t slot = atomicAdd(wl.n, 1u);
-                    if (slot < wl.cap) wl.ids[slot] = (uint32_t)ri;
+                    if (slot < wl.cap) wl.ids[slot] = (uint32_t)ri | (whole ? wl.mark : 0u);
                     else if (kAny) ovis[ri] = 255;
                     else oprim[ri] = kUndecided;
                 }
@@ -536,7 +541,8 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
 // Few rays go over their whole line (5 of 2M camera rays, 86 of 1M random
 // ones), but one holds up the launch: by one wave it took 130 us in an
 // interior and 190 in a soup of 0.5M triangles, a microsecond for each eight
-// nodes.
+// nodes. By a workgroup's eight waves, and without the wave's own attempt
+// where the trace already knows (WideList::mark), 39 and 36.
 constexpr int kPend = 1024;
 constexpr int kCands = 64;
 constexpr int kFinishWaves = 8;       // closest-hit: waves of a workgroup
@@ -729,6 +735,7 @@ struct FinishArgs {
     uint32_t* overflow;
     unsigned long long* fetched;
     int ntris;
+    uint32_t mark;
 };
 
 // Which of the hits of a wave's lanes (rival, two or more) the reference's
@@ -1115,8 +1122,11 @@ __global__ __launch_bounds__(64 * kFinishWaves) void k_wide_finish_closest(Finis
     if (blockIdx.x >= total) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     Fetches nfetch;
+    const auto leave = [&](uint32_t ri) {
+        if (lane == 0) queue[atomicAdd(&queued, 1u)] = ri;
+    };
     const auto take = [&](int64_t ri) {
-        if (!finish_closest(A, ri, lds.wave[wave], out, nfetch) && lane == 0) queue[atomicAdd(&queued, 1u)] = (uint32_t)ri;
+        if (!finish_closest(A, ri, lds.wave[wave], out, nfetch)) leave((uint32_t)ri);
     };
     const auto wholes = [&]() {  // all threads
         __syncthreads();
@@ -1133,7 +1143,10 @@ __global__ __launch_bounds__(64 * kFinishWaves) void k_wide_finish_closest(Finis
     for (int64_t base = 0; base < (int64_t)total; base += lanes * kFinishTurn) {
         for (int j = 0; j < kFinishTurn; ++j) {
             const int64_t i = base + j * lanes + (int64_t)wave * gridDim.x + blockIdx.x;
-            if (i < (int64_t)total) take(A.ids[i]);
+            if (i >= (int64_t)total) break;
+            const uint32_t id = A.ids[i];
+            if (id & A.mark) leave(id & ~A.mark);
+            else take(id);
         }
         wholes();
     }
@@ -1201,13 +1214,13 @@ void launch_wide_block(const TraceLaunch& L, int64_t nrays, LaunchSink& ls, A...
 void wide_closest(const TraceBvh& bvh, const float* rays, int64_t nrays, const uint32_t* nrays_dev, int32_t* prim,
                   float* t, float* u, float* v, uint32_t* counters, const TraceLaunch& L, const TraceCoop& coop,
                   LaunchSink& ls) {
-    const WideList wl{coop.longs, counters + 26, coop.long_cap, L.handoff};
+    const WideList wl{coop.longs, counters + 26, coop.long_cap, L.handoff, whole_mark(nrays)};
     launch_wide_block<false>(L, nrays, ls, bvh.wide.nodes, bvh.wide.tris, rays, nrays, nrays_dev, prim, t, u, v,
                              (const float*)nullptr, (const int32_t*)nullptr, (const int32_t*)nullptr,
                              (uint8_t*)nullptr, counters, reinterpret_cast<unsigned long long*>(counters + 2),
                              fetch_word(counters, true), wl, bvh.wide.far_origin, bvh.wide.rcp_max, bvh.wide.near_slack);
     const FinishArgs A{bvh.wide, bvh.rec, bvh.root, rays, nrays, nrays_dev, coop.longs, counters + 26,
-                       coop.long_cap, counters + 30, counters, fetch_word(counters, true), bvh.ntris};
+                       coop.long_cap, counters + 30, counters, fetch_word(counters, true), bvh.ntris, wl.mark};
     const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks / kFinishWaves, nrays);
     ls.launch("k_wide_finish_closest", &k_wide_finish_closest, dim3(blocks), dim3(64 * kFinishWaves), A,
               ClosestOut{prim, t, u, v});
@@ -1218,13 +1231,13 @@ void wide_occluded(const TraceBvh& bvh, const float* rays, int64_t nrays, const 
                    const float* limit, const int32_t* src, const int32_t* dst, uint8_t* visible, uint32_t* counters,
                    const TraceLaunch& L, const TraceCoop& coop, LaunchSink& ls) {
     uint32_t* ids = reinterpret_cast<uint32_t*>(coop.spill + coop.spill_cap);
-    const WideList wl{ids, counters + 20, coop.spill_cap, L.handoff};
+    const WideList wl{ids, counters + 20, coop.spill_cap, L.handoff, 0u};
     launch_wide_block<true>(L, nrays, ls, bvh.wide.nodes, bvh.wide.tris, rays, nrays, nrays_dev, (int32_t*)nullptr,
                             (float*)nullptr, (float*)nullptr, (float*)nullptr, limit, src, dst, visible,
                             counters + 1, reinterpret_cast<unsigned long long*>(counters + 4),
                             fetch_word(counters, false), wl, bvh.wide.far_origin, bvh.wide.rcp_max, bvh.wide.near_slack);
     const FinishArgs A{bvh.wide, bvh.rec, bvh.root, rays, nrays, nrays_dev, ids, counters + 20,
-                       coop.spill_cap, counters + 22, counters + 1, fetch_word(counters, false), bvh.ntris};
+                       coop.spill_cap, counters + 22, counters + 1, fetch_word(counters, false), bvh.ntris, 0u};
     const unsigned blocks = (unsigned)std::min<int64_t>(kFinishBlocks, nrays);
     ls.launch("k_wide_finish_any", &k_wide_finish_any, dim3(blocks), dim3(64), A, limit, src, dst, visible);
 }
