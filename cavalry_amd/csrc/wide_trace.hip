@@ -309,17 +309,23 @@ struct WideStackLds {
     uint16_t bits[kWideStack][B];
 };
 
-// A wave's nodes and triangles fetched into the launch's words (fetch_word).
-__device__ __forceinline__ void add_fetches(unsigned long long* fetched, uint64_t nodes, uint64_t tris) {
+// A lane of the trace counts in one register (a second one cost camera rays
+// 1%): records, and triangles from bit kTriShift. Counts that come near their
+// fields' ends are added between rays.
+constexpr int kTriShift = 17;
+constexpr uint32_t kFetchesFull = 1u << 31 | 1u << (kTriShift - 1);
+__device__ __forceinline__ uint64_t packed_fetches(uint32_t n) {  // triangles << 32 | records
+    return (uint64_t)(n >> kTriShift) << 32 | (n & ((1u << kTriShift) - 1u));
+}
+__device__ __forceinline__ void add_fetches_lane(unsigned long long* fetched, uint64_t n) {
+    atomicAdd(fetched, (unsigned long long)(uint32_t)n);
+    atomicAdd(fetched + kFetchTris, (unsigned long long)(n >> 32));
+}
+// A wave's counts into the launch's words (fetch_word).
+__device__ __forceinline__ void add_fetches(unsigned long long* fetched, uint64_t n) {
 #pragma unroll
-    for (int dd = 32; dd >= 1; dd >>= 1) {
-        nodes += __shfl_xor(nodes, dd, 64);
-        tris += __shfl_xor(tris, dd, 64);
-    }
-    if ((threadIdx.x & 63) == 0 && nodes + tris > 0) {
-        atomicAdd(fetched, (unsigned long long)(nodes + tris));
-        atomicAdd(fetched + kFetchTris, (unsigned long long)tris);
-    }
+    for (int dd = 32; dd >= 1; dd >>= 1) n += __shfl_xor(n, dd, 64);
+    if ((threadIdx.x & 63) == 0 && n > 0) add_fetches_lane(fetched, n);
 }
 
 struct WideList {           // rays left to the finishing pass
@@ -364,7 +370,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
     uint32_t tbase = 0, tbits = 0;  // triangles to test
     int sp = 0, maxsp = 0;
     uint32_t deep[2 * (kWideDeep - kWideStack)];
-    uint32_t nnodes = 0, ntris = 0;  // fetched
+    uint32_t nfetch = 0;  // records fetched, triangles among them << kTriShift
     Dispenser disp(nrays, most);
 
     while (true) {
@@ -400,6 +406,10 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                     if (slot < wl.cap) wl.ids[slot] = (uint32_t)ri | (whole ? wl.mark : 0u);
                     else if (kAny) ovis[ri] = 255;
                     else oprim[ri] = kUndecided;
+                }
+                if (nfetch & kFetchesFull) {
+                    add_fetches_lane(fetched, packed_fetches(nfetch));
+                    nfetch = 0;
                 }
                 over = false;
                 ri = -1;
@@ -485,7 +495,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
                 }
                 const uint4* nd = nodes + (int64_t)child * kWideWords;
                 const uint4 w0 = nd[0], w1 = nd[1], w2 = nd[2], w3 = nd[3], w4 = nd[4];
-                ++nnodes;
+                ++nfetch;
                 const uint32_t mask = test_children(w0, w1, w2, w3, w4, r, cut);
                 cbase = w1.x;
                 tbase = w1.y;
@@ -498,7 +508,7 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
             tbits &= tbits - 1u;
             const float4* tp = tris + (int64_t)(tbase + k) * 3;
             const float4 a = tp[0], b = tp[1], c = tp[2];
-            ++ntris;
+            nfetch += 1u + (1u << kTriShift);
             float t, u, v;
             if (kAny) {
                 const int mesh = __float_as_int(b.w);
@@ -523,10 +533,29 @@ __global__ __launch_bounds__(B) __attribute__((amdgpu_waves_per_eu(6))) void k_w
             else over = true;
         }
     }
+    // (an atomic per workgroup and word: they serialise, 5 ns each, and a wave's
+    // made each launch of the Cornell box 20 us longer)
+    __shared__ uint64_t wfetch[B / 64];
+    __shared__ int wdeep[B / 64];
+    uint64_t fetches = packed_fetches(nfetch);
 #pragma unroll
-    for (int dd = 32; dd >= 1; dd >>= 1) maxsp = max(maxsp, __shfl_xor(maxsp, dd, 64));
-    if (lane == 0 && maxsp > 0) atomicMax(overflow + 6, (uint32_t)maxsp);
-    add_fetches(fetched, nnodes, ntris);
+    for (int dd = 32; dd >= 1; dd >>= 1) {
+        maxsp = max(maxsp, __shfl_xor(maxsp, dd, 64));
+        fetches += __shfl_xor(fetches, dd, 64);
+    }
+    if (lane == 0) {
+        wfetch[threadIdx.x >> 6] = fetches;
+        wdeep[threadIdx.x >> 6] = maxsp;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < B / 64; ++w) {
+            fetches += wfetch[w];
+            maxsp = max(maxsp, wdeep[w]);
+        }
+        if (maxsp > 0) atomicMax(overflow + 6, (uint32_t)maxsp);
+        if (fetches > 0) add_fetches_lane(fetched, fetches);
+    }
 }
 
 // ------------------------------------------------------------- finishing pass
@@ -664,9 +693,6 @@ __device__ bool reference_blocked(const TRec* recs, v3 o, v3 d, float lim, int s
     }
 }
 
-struct Fetches {
-    uint64_t nodes = 0, tris = 0;
-};
 struct FinishLds {
     uint32_t pend[kPend];
     float t[kCands], u[kCands], v[kCands], e[kCands];
@@ -811,7 +837,7 @@ __device__ __forceinline__ bool root_hit(const FinishArgs& A, v3 o, v3 d) {
 }
 
 // A ray by a wave. false: it has to be taken over its whole line.
-__device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, const ClosestOut& out, Fetches& nfetch) {
+__device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, const ClosestOut& out, uint64_t& nfetch) {
     const int lane = threadIdx.x & 63;
     v3 o, d;
     load_ray(A.rays, ri, o, d);
@@ -837,7 +863,7 @@ __device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, co
             const uint32_t node = L.pend[count - 1 - g];
             const float cut = best == FLT_MAX ? FLT_MAX : __builtin_fmaf(best * r.scale, kReach, A.w.near_slack);
             lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, cut, inner, at, nt);
-            nfetch.nodes += (lane & 7) == 0 ? 1u : 0u;
+            nfetch += (lane & 7) == 0 ? 1u : 0u;
         }
         count -= k;
         wave_fence();
@@ -848,7 +874,7 @@ __device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, co
             if (j < nt) {
                 const float4* tp = A.w.tris + (int64_t)(at + (uint32_t)j) * 3;
                 const float4 a = tp[0], b = tp[1], c = tp[2];
-                ++nfetch.tris;
+                nfetch += (1ull << 32) + 1u;
                 thin = thin || thin_test(a, b, c, d, r.scale);
                 if (wide_tri_hit(a, b, c, o, d, t, u, v)) {
                     thin = thin || thin_hit(a, b, c, o, d, t, t * (kReach - 1.f) + near);
@@ -930,7 +956,7 @@ __device__ bool finish_closest(const FinishArgs& A, int64_t ri, FinishLds& L, co
 // A ray over its whole line by all waves of the workgroup, 64 nodes at a
 // time: no box of the line is skipped, so that the answer does not rest on
 // where the hits' distances lie.
-__device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const ClosestOut& out, Fetches& nfetch) {
+__device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const ClosestOut& out, uint64_t& nfetch) {
     const int lane = threadIdx.x & 63;
     v3 o, d;
     load_ray(A.rays, ri, o, d);
@@ -957,7 +983,7 @@ __device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const
         int nt = 0;
         if (g < k) {
             lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, FLT_MAX, inner, at, nt);
-            nfetch.nodes += (lane & 7) == 0 ? 1u : 0u;
+            nfetch += (lane & 7) == 0 ? 1u : 0u;
         }
         const uint64_t im = __ballot(inner);
         if (im != 0ull) {
@@ -967,15 +993,10 @@ __device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const
             if (inner && base < (uint32_t)kWholePend) W.pend[base] = at;
             if (inner && base >= (uint32_t)kWholePend) W.bad = 1u;
         }
-        float4 tri[kWideLeaf * 3];  // (loaded together: a latency each otherwise)
-#pragma unroll
-        for (int j = 0; j < kWideLeaf * 3; ++j)
-            if (j < 3 * nt) tri[j] = A.w.tris[(int64_t)at * 3 + j];
-#pragma unroll
-        for (int j = 0; j < kWideLeaf; ++j) {
-            if (j >= nt) continue;
-            const float4 a = tri[3 * j], b = tri[3 * j + 1], c = tri[3 * j + 2];
-            ++nfetch.tris;
+        for (int j = 0; j < nt; ++j) {
+            const float4* tp = A.w.tris + (int64_t)(at + (uint32_t)j) * 3;
+            const float4 a = tp[0], b = tp[1], c = tp[2];
+            nfetch += (1ull << 32) + 1u;
             float t, u, v;
             if (!wide_tri_hit(a, b, c, o, d, t, u, v)) continue;
             bool touch, bad = false;
@@ -1041,7 +1062,7 @@ __device__ void finish_whole(const FinishArgs& A, int64_t ri, WholeLds& W, const
 }
 
 __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const float* limit, const int32_t* src,
-                           const int32_t* dst, uint8_t* ovis, Fetches& nfetch) {
+                           const int32_t* dst, uint8_t* ovis, uint64_t& nfetch) {
     const int lane = threadIdx.x;
     v3 o, d;
     load_ray(A.rays, ri, o, d);
@@ -1065,14 +1086,14 @@ __device__ void finish_any(const FinishArgs& A, int64_t ri, FinishLds& L, const 
         if (g < k) {
             const uint32_t node = L.pend[count - 1 - g];
             lane_child(A.w.nodes + (int64_t)node * kWideWords, lane & 7, r, cut, inner, at, nt);
-            nfetch.nodes += (lane & 7) == 0 ? 1u : 0u;
+            nfetch += (lane & 7) == 0 ? 1u : 0u;
         }
         count -= k;
         wave_fence();
         for (int j = 0; j < nt && !hit; ++j) {
             const float4* tp = A.w.tris + (int64_t)(at + (uint32_t)j) * 3;
             const float4 a = tp[0], b = tp[1], c = tp[2];
-            ++nfetch.tris;
+            nfetch += (1ull << 32) + 1u;
             const int mesh = __float_as_int(b.w);
             float t, u, v;
             if (mesh != sm && mesh != dm && wide_tri_hit(a, b, c, o, d, t, u, v) && (!use || t < lim)) {
@@ -1121,7 +1142,7 @@ __global__ __launch_bounds__(64 * kFinishWaves) void k_wide_finish_closest(Finis
     const uint32_t total = min(all, A.cap);
     if (blockIdx.x >= total) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    Fetches nfetch;
+    uint64_t nfetch = 0;  // triangles << 32 | records
     const auto leave = [&](uint32_t ri) {
         if (lane == 0) queue[atomicAdd(&queued, 1u)] = ri;
     };
@@ -1159,7 +1180,7 @@ __global__ __launch_bounds__(64 * kFinishWaves) void k_wide_finish_closest(Finis
             wholes();
         }
     }
-    add_fetches(A.fetched, nfetch.nodes, nfetch.tris);
+    add_fetches(A.fetched, nfetch);
 }
 
 __global__ __launch_bounds__(64) void k_wide_finish_any(FinishArgs A, const float* limit, const int32_t* src,
@@ -1168,7 +1189,7 @@ __global__ __launch_bounds__(64) void k_wide_finish_any(FinishArgs A, const floa
     const uint32_t all = *A.n;
     const uint32_t total = min(all, A.cap);
     if (blockIdx.x >= total) return;
-    Fetches nfetch;
+    uint64_t nfetch = 0;  // triangles << 32 | records
     for (uint32_t i = blockIdx.x; i < total; i += gridDim.x) finish_any(A, A.ids[i], L, limit, src, dst, ovis, nfetch);
     if (all > A.cap) {  // the list ran over: find the marked rays
         const int64_t nrays = A.nrays_dev ? (int64_t)*A.nrays_dev : A.nrays;
@@ -1178,7 +1199,7 @@ __global__ __launch_bounds__(64) void k_wide_finish_any(FinishArgs A, const floa
                 finish_any(A, b + __ffsll((long long)m) - 1, L, limit, src, dst, ovis, nfetch);
         }
     }
-    add_fetches(A.fetched, nfetch.nodes, nfetch.tris);
+    add_fetches(A.fetched, nfetch);
 }
 
 constexpr int kFinishBlocks = 4096;
