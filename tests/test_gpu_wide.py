@@ -112,28 +112,64 @@ def test_scene_far_from_the_origin_and_given_bounds(ctx):
     _check(bvh, nd, tris, rays, lim, "far")
 
 
+def _reference_order(ctx, call):
+    saved = tune.get_launch(ctx, tune.STANDALONE)
+    try:
+        tune.set_launch(ctx, tune.STANDALONE, dict(saved, handoff_steps=1 << 30))
+        return call()
+    finally:
+        tune.set_launch(ctx, tune.STANDALONE, saved)
+
+
+LIST = 1 << 20  # rays the finishing pass's list holds
+
+
 def test_more_undecided_rays_than_the_list_holds(ctx):
-    """Every triangle twice: every hit is undecided. 2^20 + 4099 rays, one list
-    of 2^20; the rest are found by scanning. Compared with the reference's
-    order on one lane per ray."""
+    """Every triangle twice: every hit is undecided. More of them than the list
+    holds; the rest are found by scanning. Compared with the reference's order
+    on one lane per ray."""
     half = scenes.gmm_triangles(500, seed=11, edge=0.3)
     tris = np.ascontiguousarray(np.concatenate([half, half]), np.float32)
-    n = (1 << 20) + 4099
+    n = LIST + 20011
     rays = scenes.random_rays(n, seed=12, lo=0.3, hi=0.7)
     bvh = BVH.build(ctx, tris)
     got = bvh.intersect(rays)
     f = bvh.trace_fetches()
-    saved = tune.get_launch(ctx, tune.STANDALONE)
-    try:
-        tune.set_launch(ctx, tune.STANDALONE, dict(saved, handoff_steps=1 << 30))
-        ref = bvh.intersect(rays)
-    finally:
-        tune.set_launch(ctx, tune.STANDALONE, saved)
-    print(f"[wide] undecided: {f}", flush=True)
-    assert (ref["prim"] >= 0).mean() > 0.9
+    ref = _reference_order(ctx, lambda: bvh.intersect(rays))
+    print(f"[wide] undecided: {f}, {(ref['prim'] >= 0).sum()} hits", flush=True)
+    assert (ref["prim"] >= 0).sum() > LIST + 10000 and f["long_closest_rays"] == LIST  # (clamped to the list)
     np.testing.assert_array_equal(got["prim"], ref["prim"])
     for k in ("t", "u", "v"):
         np.testing.assert_array_equal(bits(got[k]), bits(ref[k]), err_msg=k)
+
+
+def test_more_undecided_any_hit_rays_than_the_list_holds(ctx):
+    """Walls standing on y = 0 and rays along that plane through their lower
+    edges: every blocker is met along a plane of its box, where the sign of the
+    direction's zero decides, so every ray is undecided."""
+    rng = np.random.default_rng(22)
+    x = np.arange(1, 41) / 41.0
+    top = rng.uniform(0.2, 1, (40, 2))
+    tris = np.stack([x, 0 * x, 0 * x, x, 0 * x, 0 * x + 1, x, top[:, 0], top[:, 1]], -1).astype(np.float32)
+    n = LIST + 20011
+    rays = np.zeros((n, 6), np.float32)
+    rays[:, 0] = rng.uniform(-1, 0.9, n)
+    rays[:, 2] = rng.uniform(0.05, 0.95, n)
+    rays[:, 3] = 1.0
+    rays[:, 4] = np.where(rng.random(n) < 0.5, 0.0, -0.0)
+    lim = np.full(n, np.inf, np.float32)
+    lim[::2] = 2.5
+    bvh = BVH.build(ctx, tris)
+    got = bvh.test_visibility(rays, lim)
+    f = bvh.trace_fetches()
+    ref = _reference_order(ctx, lambda: bvh.test_visibility(rays, lim))
+    print(f"[wide] undecided any-hit: {f}, {int((ref == 0).sum())} blocked", flush=True)
+    assert f["spilled_rays"] == LIST  # (clamped to the list)
+    assert 0.2 < ref.mean() < 0.8
+    np.testing.assert_array_equal(got, ref)
+    few = slice(0, 5000)
+    _, _, nd = oracle.lbvh_build(tris, 30)
+    np.testing.assert_array_equal(got[few], oracle.trace_occluded(nd, tris, rays[few], lim[few]))
 
 
 def test_rebuild_reuses_the_tree(ctx):
