@@ -12,7 +12,7 @@
 //   order  : u32[N] sorted position -> original triangle index
 //   nbox   : NodeBox[M]   (lo, sa | hi, cost), 32 B
 //   ntopo  : int4[M]      (left, right, parent, prim), 16 B
-//   visited: u32[M]       refit / treelet climb gates
+//   visited: u32[M]       2 << 16 | height of the inner nodes (the climb's words; treelets keep them)
 #include "dev_common.h"
 #include "lbvh.h"
 

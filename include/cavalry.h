@@ -429,10 +429,11 @@ int cav_scene_create_from_pbrt(cav_ctx* ctx, const char* path, const cav_pbrt_ov
  * the limit is skipped, since no triangle in it can block the ray unless
  * Moller-Trumbore's t is off by more than that, which takes a ray within
  * about 1e-5 or 1e-4 rad of a sliver's plane).
- * Each ray's closest-hit node order is the reference's, the any-hit answer
- * does not depend on the order the reachable leaves are tested in, and each
- * sample's shading is its own, so results do not depend on the shape. STANDALONE applies to cav_trace_*, WAVEFRONT to
- * cav_render and to servers opened on the context afterwards. No
+ * Each ray's closest hit is that of the reference's node order, the any-hit
+ * answer does not depend on the order the reachable leaves are tested in, and
+ * each sample's shading is its own, so results do not depend on the shape (but
+ * for the assumptions stated above). STANDALONE applies to cav_trace_*,
+ * WAVEFRONT to cav_render and to servers opened on the context afterwards. No
  * counterpart in the reference (its launch shapes are compile-time, 256
  * threads: Utils/GpuCommons.h:63); cavalry_amd/tune.py times the candidates
  * and keeps the fastest in a JSON cache. */
