@@ -287,6 +287,40 @@ def test_rays_in_the_plane_of_a_turned_floor(ctx, size, walls):
             np.testing.assert_array_equal(bits(got[k]), bits(ref[k]), err_msg=k)
 
 
+@pytest.mark.parametrize("seed", [1323, 1394, 1432])
+def test_determinants_that_round_to_zero(ctx, seed):
+    """Rays in the plane of a coarse turned floor whose triangles before the
+    nearest wall all have a determinant of exactly 0, the sum of terms that are
+    not: one behind the wall rounds to something, and its t to less than the
+    wall's."""
+    rng = np.random.default_rng(seed)
+    floor = _floor(int(rng.integers(3, 60)), 1.0)
+    floor[..., :2] -= 0.5
+    tris = [floor]
+    for x in rng.uniform(-0.4, 0.4, rng.integers(0, 5)):
+        all_ = np.concatenate(tris)
+        w = all_[::int(rng.integers(1, 9)), :, [2, 1, 0]].copy()
+        w[..., 0] = x
+        tris = [np.concatenate([all_, w])]
+    size = 10.0 ** rng.uniform(-3, 3)
+    tt, q = _turned(tris[0], seed, size)
+    shift = np.float32(0)
+    if rng.random() < 0.3:
+        shift = rng.uniform(-2, 2, 3).astype(np.float32)[np.tile([0, 1, 2], 3)] * np.float32(size)
+    tt = (tt + shift).astype(np.float32)
+    n = 60000
+    o = np.stack([rng.uniform(-0.8, 0.8, n), rng.uniform(-0.8, 0.8, n), np.zeros(n)], -1)
+    a = rng.uniform(0, 2 * np.pi, n)
+    d = np.stack([np.cos(a), np.sin(a), rng.normal(size=n) * 10.0 ** rng.uniform(-9, -4) * (rng.random() < 0.7)], -1)
+    at = tt.reshape(-1, 3).mean(0) - tris[0].reshape(-1, 3).mean(0) @ q.T * size
+    rays = np.ascontiguousarray(np.concatenate([o @ q.T * size + at, d @ q.T], 1), np.float32)
+    bvh, nd = _tree(ctx, tt, 30, int(rng.integers(0, 4)))
+    ref, got = oracle.trace_closest(nd, tt, rays), bvh.intersect(rays)
+    print(f"[wide] zero determinants, seed {seed}: {(ref['prim'] != got['prim']).sum()} differ", flush=True)
+    np.testing.assert_array_equal(got["prim"], ref["prim"])
+    np.testing.assert_array_equal(bits(got["t"]), bits(ref["t"]))
+
+
 @pytest.mark.parametrize("ratio", [300, 30000, 3000000])
 def test_needles(ctx, ratio):
     """Triangles `ratio` times longer than wide among ordinary ones, and rays
